@@ -50,6 +50,9 @@ struct DevVolume {
     float sx, sy, sz;     // spacing
     float rsx, rsy, rsz;  // RN(1/spacing), host-computed
     double rdx, rdy, rdz; // RN64(1/spacing), host-computed (exact-path divisions)
+    float rhx, rhy, rhz;  // RN(1/spacing) and the float of what it leaves of 1/spacing: the divisions of
+    float rlx, rly, rlz;  // birp_div_fma2, when div_fma2 says that they are exact on every axis
+    int div_fma2;
     float fnx, fny, fnz;  // (float) n per axis, as the reference's bound test compares
     int interp;           // 0 nearest, 1 trilinear
     int dtype;            // BIRP_DTYPE_*
@@ -82,8 +85,8 @@ struct ExactView {
     int vol;          // multi-view launches: index of the view's volume in the volume table
     int accumulate;   // start from out's values
     float margin;     // FP64 slab expansion (RE) that covers FP32 position error
-    int fast_guards;  // positive cube whose scaled samples stay normal floats: only the
-                      // scale's midpoint guard is needed
+    int fast_guards;  // positive cube whose scaled samples stay normal floats: 1: only the scale's
+                      // midpoint guard is needed; 2: the samples also stay in birp_scale_fma2's range
     float* out;       // device image H*W
     unsigned long long* counter;  // optional: samples added (one atomic per wave)
     unsigned* wave_counts;  // optional, instead of counter: each wave stores its samples added at
@@ -172,6 +175,9 @@ int launch_fast_batch(const DevVolume* vols_dev, int dtype, const FastPose* pose
 int launch_reset_counter(unsigned* counter, void* stream);
 int launch_zero_f32(float* p, size_t n, void* stream);
 int launch_scan_class(const float* values, size_t n, unsigned* flags_dev, void* stream);
+// Checks birp_div_fma2 for the volume's spacings over every significand: ORs bit `axis` into *bad_dev for
+// an axis with a mismatch.
+int launch_check_div(const DevVolume& v, unsigned* bad_dev, void* stream);
 int launch_build_quad(const DevVolume& v, void* quad, void* stream);
 int launch_build_oct(const DevVolume& v, void* oct, float* bscale, void* stream);
 

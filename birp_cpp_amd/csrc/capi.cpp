@@ -98,6 +98,7 @@ int exact_view(const birp_volume* vol, const birp_view* v, float* out_dev, Exact
     // midpoint guard (interpolated values stay within [vmin, vmax])
     const double kf = (1.0 * BIRP_SCALE_K_HOST / BIRP_SCALE_C_HOST) / 10000;
     ev.fast_guards = (d.vclass == VC_POSITIVE && (double)d.vmin * ev.w * kf >= 0x1p-124 && (double)d.vmax * ev.w * kf <= 0x1p126) ? 1 : 0;
+    if (ev.fast_guards && (double)d.vmin * ev.w >= 0x1p-99 && (double)d.vmax * ev.w <= 0x1p109) ev.fast_guards = 2;
     ev.out = out_dev;
     ev.vol = 0;
     ev.counter = nullptr;
@@ -406,6 +407,16 @@ static uint32_t spread3(uint32_t b) {
     return x;
 }
 
+// 1/b as rh + rl (birp_div_fma2). False when rl is so small that a * rl could leave the normal floats for
+// an ingress a >= 2^-56 (the check over significands holds at every exponent only while it does not).
+static bool split_reciprocal(float b, float& rh, float& rl) {
+    volatile float one = 1.0f;
+    rh = one / b;
+    const double left = std::fma(-(double)rh, (double)b, 1.0) / (double)b;
+    rl = (float)left;
+    return b >= 0x1p-20f && b <= 0x1p20f && (rl == 0.f || std::abs(rl) >= rh * 0x1p-44f);
+}
+
 // Per-axis byte-offset tables of a bricked record layout (see birp_internal.h): returns the
 // number of brick slots the layout spans, or 0 when the byte offsets would not fit 32 bits.
 static size_t brick_tables(int nx, int ny, int nz, unsigned brick_bytes, std::vector<unsigned>& tab, bool* morton) {
@@ -481,6 +492,7 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
         d.rdy = done / (double)d.sy;
         d.rdz = done / (double)d.sz;
     }
+    const bool splits = split_reciprocal(d.sx, d.rhx, d.rlx) && split_reciprocal(d.sy, d.rhy, d.rly) && split_reciprocal(d.sz, d.rhz, d.rlz);
     d.fnx = (float)nx;
     d.fny = (float)ny;
     d.fnz = (float)nz;
@@ -494,7 +506,7 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
 
     hipError_t e;
     int rc = BIRP_OK;
-    unsigned flags[3] = {0u, 0x7F7FFFFFu, 0u};
+    unsigned flags[4] = {0u, 0x7F7FFFFFu, 0u, 0u};
     unsigned* dflags = (unsigned*)dev->d_counter;
     size_t quad_bytes = 0, oct_bytes = 0, slots = 0;
     bool morton = false;
@@ -510,12 +522,14 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
         goto fail_out;
     }
     if ((rc = launch_scan_class(v->linear, nvox, dflags, dev->stream)) != BIRP_OK) goto fail_out;
+    if (splits && desc->dtype == BIRP_DTYPE_F32 && (rc = launch_check_div(d, dflags + 3, dev->stream)) != BIRP_OK) goto fail_out;
     if ((e = hipMemcpyAsync(flags, dflags, sizeof(flags), hipMemcpyDeviceToHost, dev->stream)) != hipSuccess ||
         (e = hipStreamSynchronize(dev->stream)) != hipSuccess) {
         rc = hip_fail(e, "class scan");
         goto fail_out;
     }
     d.vclass = (flags[0] & 2u) ? VC_NONFINITE : (flags[0] & 1u) ? VC_FINITE : VC_POSITIVE;
+    d.div_fma2 = splits && flags[3] == 0u && desc->dtype == BIRP_DTYPE_F32;
     memcpy(&d.vmin, &flags[1], 4);
     memcpy(&d.vmax, &flags[2], 4);
     if (desc->dtype == BIRP_DTYPE_F32) {

@@ -20,6 +20,24 @@
 //                           roundings agree unless the product lies within 16 double ulps of a
 //                           float rounding midpoint (or outside the normal float range); those
 //                           rare inputs take the three-operation chain.
+//  birp_div_fma2(a, rh, rl): RN(a / b) for rh = RN(1/b) and rl = RN(1/b - rh), as one multiply and
+//                           one FMA (Brisebarre, Muller and Raina, "Accelerating correctly rounded
+//                           floating-point division when the divisor is known in advance", IEEE
+//                           Trans. Computers 53(8), 2004). The sum a rh + RN(a rl) is within 2^-47
+//                           (relative) of a/b, so it rounds like a/b for nearly every divisor; which
+//                           ones is checked for all 2^23 significands of a when a cube is uploaded
+//                           (the result does not depend on a's exponent or sign while a rl is a
+//                           normal float), and the others keep birp_div_rn64.
+//  birp_scale_fma2(vw):     the chain of Camera.cpp:201 the same way: the chain's constant as a sum of
+//                           two floats, one multiply and one FMA. Equal to the chain for every
+//                           significand of vw (checked exhaustively), while vw times the low part and
+//                           the result are normal floats: |vw| in [2^-100, 2^110].
+//  birp_lerp_unit(a, b, t): std::lerp(a, b, t) for 0 <= t <= 1 - 2^-24 when a and b do not straddle
+//                           zero: a + t (b - a), whose final clamp towards b never applies. Let
+//                           X = RN(b - a) (b > a; the other case mirrors it), X = b - a + d with
+//                           |d| <= ulp(X)/2. Since t <= 1 - 2^-24, RN(t X) <= X - ulp(X)/2 (a float;
+//                           a subnormal X is exact, d = 0), so a + RN(t X) <= b + d - ulp(X)/2 <= b,
+//                           and rounding keeps <= b. v_fract_f32 never returns more than 1 - 2^-24.
 #pragma once
 
 #include <stdint.h>
@@ -63,6 +81,10 @@ BIRP_HD float birp_div_rn(float a, float b, float rb) {
 
 BIRP_HD float birp_div_rn64(float a, double rb64) { return (float)((double)a * rb64); }
 
+BIRP_HD float birp_div_fma2(float a, float rh, float rl) { return birp_fmaf(a, rh, a * rl); }
+
+BIRP_HD float birp_lerp_unit(float a, float b, float t) { return a + t * (b - a); }
+
 // The reference chain, operation by operation (Camera.cpp:201).
 BIRP_HD float birp_scale_chain(float vw) {
     return (float)(((double)vw * BIRP_SCALE_K / BIRP_SCALE_C) / 10000);
@@ -70,6 +92,12 @@ BIRP_HD float birp_scale_chain(float vw) {
 
 // The chain's constant: the chain applied to 1.0 (the first product is exact).
 #define BIRP_SCALE_FOLDED ((1.0 * BIRP_SCALE_K / BIRP_SCALE_C) / 10000)
+
+// The folded constant as a sum of two floats.
+#define BIRP_SCALE_HI ((float)BIRP_SCALE_FOLDED)
+#define BIRP_SCALE_LO ((float)(BIRP_SCALE_FOLDED - (double)BIRP_SCALE_HI))
+
+BIRP_HD float birp_scale_fma2(float vw) { return birp_fmaf(vw, BIRP_SCALE_HI, vw * BIRP_SCALE_LO); }
 
 // 1 when the folded product y cannot be trusted to round like the chain.
 BIRP_HD int birp_scale_needs_chain(double y) {

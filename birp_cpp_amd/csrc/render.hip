@@ -80,13 +80,6 @@ __device__ __forceinline__ float lerp_general(float a, float b, float t) {
     return straddle ? s1 : r;
 }
 
-// std::lerp when a, b > 0 and finite and 0 <= t < 1: a + t(b-a) clamped towards b, which is
-// the median of (x, a, b) since x never passes a.
-__device__ __forceinline__ float lerp_positive(float a, float b, float t) {
-    float x = a + t * (b - a);
-    return __builtin_amdgcn_fmed3f(x, a, b);
-}
-
 // Clamp in the float domain to [0, hi], then convert (NaN -> 0 in hardware).
 __device__ __forceinline__ int to_index(float x, float hi) { return (int)__builtin_amdgcn_fmed3f(x, 0.0f, hi); }
 
@@ -131,10 +124,13 @@ struct ExactIdx {
     float xd, yd, zd;  // index
 };
 
-// GUARD: the double-product division is exact while the quotient is a normal float, which
+// DIV_GUARD: the double-product division is exact while the quotient is a normal float, which
 // holds for |ingress| >= 2^-64 (spacing <= 2^30); below that (possible only when an origin
 // component is within 2^-30 of 0) the IEEE division is used.
-template <bool GUARD>
+// DIV_FMA2: the divisions as birp_div_fma2 (volumes whose spacings passed the upload's check; |origin|
+// >= 2^-30, so a nonzero ingress is at least 2^-56 and a rl stays normal).
+enum DivForm { DIV_GUARD = 0, DIV_RN64 = 1, DIV_FMA2 = 2 };
+template <int DIV>
 __device__ __forceinline__ ExactIdx exact_index(const DevVolume& v, float dx, float dy, float dz, float px, float py,
                                                 float pz, float t) {
     ExactIdx r;
@@ -144,7 +140,13 @@ __device__ __forceinline__ ExactIdx exact_index(const DevVolume& v, float dx, fl
     r.xi = x - v.ox;
     r.yi = y - v.oy;
     r.zi = z - v.oz;
-    if constexpr (GUARD) {
+    if constexpr (DIV == DIV_FMA2) {
+        r.xd = birp_div_fma2(r.xi, v.rhx, v.rlx);
+        r.yd = birp_div_fma2(r.yi, v.rhy, v.rly);
+        r.zd = birp_div_fma2(r.zi, v.rhz, v.rlz);
+        return r;
+    }
+    if constexpr (DIV == DIV_GUARD) {
         float m = fminf(fminf(fabsf(r.xi), fabsf(r.yi)), fabsf(r.zi));
         if (__builtin_expect(m < 0x1p-64f && m != 0.0f, 0)) {
             r.xd = r.xi / v.sx;
@@ -215,9 +217,9 @@ template <bool POS>
 __device__ __forceinline__ float quad_lerp(const QuadFetch& q) {
     const float4 a = q.a, b = q.b;
     if constexpr (POS) {
-        float ly = lerp_positive(lerp_positive(a.x, a.y, q.fx), lerp_positive(a.z, a.w, q.fx), q.fy);
-        float hy = lerp_positive(lerp_positive(b.x, b.y, q.fx), lerp_positive(b.z, b.w, q.fx), q.fy);
-        return lerp_positive(ly, hy, q.fz);
+        float ly = birp_lerp_unit(birp_lerp_unit(a.x, a.y, q.fx), birp_lerp_unit(a.z, a.w, q.fx), q.fy);
+        float hy = birp_lerp_unit(birp_lerp_unit(b.x, b.y, q.fx), birp_lerp_unit(b.z, b.w, q.fx), q.fy);
+        return birp_lerp_unit(ly, hy, q.fz);
     } else {
         float ly = lerp_general(lerp_general(a.x, a.y, q.fx), lerp_general(a.z, a.w, q.fx), q.fy);
         float hy = lerp_general(lerp_general(b.x, b.y, q.fx), lerp_general(b.z, b.w, q.fx), q.fy);
@@ -387,8 +389,8 @@ __device__ void exact_clip(const DevVolume& v, const ExactView& ev, const float*
     klo = fmin(fmax(klo, 0.0), (double)n);
     khi = fmin(fmax(khi, -1.0), (double)(n - 1));
     int a = (int)klo, b = (int)khi;
-    while (a <= b && !exact_inside(v, exact_index<true>(v, dx, dy, dz, ev.px, ev.py, ev.pz, s_t[a]))) a++;
-    while (b >= a && !exact_inside(v, exact_index<true>(v, dx, dy, dz, ev.px, ev.py, ev.pz, s_t[b]))) b--;
+    while (a <= b && !exact_inside(v, exact_index<DIV_GUARD>(v, dx, dy, dz, ev.px, ev.py, ev.pz, s_t[a]))) a++;
+    while (b >= a && !exact_inside(v, exact_index<DIV_GUARD>(v, dx, dy, dz, ev.px, ev.py, ev.pz, s_t[b]))) b--;
     kf = a;
     kl = b;
 }
@@ -420,6 +422,68 @@ __device__ __forceinline__ void exact_lane(int lane, int& ti, int& tj, int& sub)
     tj = (blk / (TW / 2)) * 2 + ((lane >> 1) & 1);
 }
 
+
+// The samples of a wave's rays over a positive cube, added in k order (exact_block's main loop).
+// P samples per lane per iteration (k, k + S, ...), staged so that the later samples' LDS and
+// buffer reads are in flight while the first ones' lerps run. The sum order is unchanged: the S
+// samples at k, then the S samples at k + S, and so on.
+// Every lane samples inside the cube, so the corner indices need no clamp: a lane past its ray's last
+// in-cube sample kl re-reads kl's t (its result is masked), and a lane whose ray has no in-cube
+// sample is at the cube's origin (zero direction), which is inside. The in-cube samples kf..kl are
+// contiguous (the FP32 index is monotone in t). t is read at LDS byte address min(t_lo + 4k, t_hi),
+// both bounds including the LDS base.
+// Trips that every lane of the wave fills (kb + P S <= full, the wave's shortest range) need neither
+// the clamp of t's address nor the mask, and read their P t values at constant offsets from one
+// address; the arithmetic and the sum order are those of the masked trips.
+// FMA2: divisions and scale as one multiply and one FMA each (birp_div_fma2, birp_scale_fma2), where the
+// volume's spacings and values allow it: 51 VALU instructions per sample and no branch, against 57
+// and one rarely taken branch per sample. Issue-bound batches gain what the instructions save (64 orbit
+// views of a 256^3 cube: 1.189 ms with FP64 divisions and scale and clamped lerps, 1.058 ms now); a
+// single 576x336 x 800 view, whose waves also wait on the vector L1, goes from 87.4 to 84.7 us.
+typedef __attribute__((address_space(3))) const float* lds_float_ptr;
+template <int S, int P, bool FMA2>
+__device__ __forceinline__ float march_positive(const DevVolume& v, const QuadCtx& qc, float rx, float ry, float rz, float qx, float qy,
+                                                float qz, unsigned t_lo, unsigned t_hi, int full, int trips, int lim, float w, float acc) {
+    constexpr int DIV = FMA2 ? DIV_FMA2 : DIV_RN64;
+    auto scaled = [&](const QuadFetch& q) {  // Camera.cpp:201
+        const float vw = quad_lerp<true>(q) * w;
+        return FMA2 ? birp_scale_fma2(vw) : scale_pos(vw);
+    };
+    int kb = 0;
+    for (; kb + P * S <= full; kb += P * S) {
+        QuadFetch q[P];
+        const unsigned tb = t_lo + (unsigned)kb * 4u;
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const float t = *(lds_float_ptr)(uintptr_t)(tb + (unsigned)(u * S) * 4u);
+            const ExactIdx r = exact_index<DIV>(v, rx, ry, rz, qx, qy, qz, t);
+            q[u] = quad_fetch_inside(qc, r.xd, r.yd, r.zd);
+        }
+        float sc[P];
+#pragma unroll
+        for (int u = 0; u < P; ++u) sc[u] = scaled(q[u]);
+#pragma unroll
+        for (int u = 0; u < P; ++u) acc = add_in_order<S>(acc, sc[u]);
+    }
+    for (; kb < trips; kb += P * S) {
+        QuadFetch q[P];
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const float t = *(lds_float_ptr)(uintptr_t)min(t_lo + (unsigned)(kb + u * S) * 4u, t_hi);
+            const ExactIdx r = exact_index<DIV>(v, rx, ry, rz, qx, qy, qz, t);
+            q[u] = quad_fetch_inside(qc, r.xd, r.yd, r.zd);
+        }
+        float sc[P];
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            sc[u] = scaled(q[u]);
+            sc[u] = (kb + u * S < lim) ? sc[u] : -0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < P; ++u) acc = add_in_order<S>(acc, sc[u]);
+    }
+    return acc;
+}
 
 // ------------------------------------------------------------------------------------------
 // the exact render: one block renders one 2x2-wave tile `lb` of a view (wg_x tiles per row of
@@ -484,59 +548,18 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
     const float px = ev.px, py = ev.py, pz = ev.pz;
 
     if constexpr (POS) {
-        // P samples per lane per iteration (k, k + S, ...), staged so that the later samples' LDS
-        // and buffer reads are in flight while the first ones' lerps run. The sum order is
-        // unchanged: the S samples at k, then the S samples at k + S, and so on.
-        // Every lane samples inside the cube, so the corner indices need no clamp: a lane past
-        // its ray's last in-cube sample kl re-reads kl's t (its result is masked), and a lane
-        // whose ray has no in-cube sample is sent to the cube's origin (zero direction), which is
-        // inside. The in-cube samples kf..kl are contiguous (the FP32 index is monotone in t).
         const bool has = len > 0;
         const float rx = has ? dx : 0.f, ry = has ? dy : 0.f, rz = has ? dz : 0.f;
         const float qx = has ? px : v.ox, qy = has ? py : v.oy, qz = has ? pz : v.oz;
-        // t is read at LDS byte address min(t_lo + 4k, t_hi), both bounds including the LDS base
-        typedef __attribute__((address_space(3))) const float* lds_float_ptr;
         const unsigned t_base = (unsigned)(uintptr_t)(lds_float_ptr)s_t;
         unsigned t_lo = t_base + (has ? t_first : 0u), t_hi = t_base + (has ? (unsigned)kl * 4u : 0u);
         // keep the selects above out of the loop (the compiler would otherwise redo them per sample)
         asm volatile("" : "+v"(t_lo), "+v"(t_hi));
-        // Trips that every lane of the wave fills (kb + P S <= the wave's shortest range) need
-        // neither the clamp of t's address nor the mask, and read their P t values at constant
-        // offsets from one address. The arithmetic and the sum order are those of the loop below.
         const int full = wave_min_i(len);
-        int kb = 0;
-        for (; kb + P * S <= full; kb += P * S) {
-            QuadFetch q[P];
-            const unsigned tb = t_lo + (unsigned)kb * 4u;
-#pragma unroll
-            for (int u = 0; u < P; ++u) {
-                const float t = *(lds_float_ptr)(uintptr_t)(tb + (unsigned)(u * S) * 4u);
-                const ExactIdx r = exact_index<false>(v, rx, ry, rz, qx, qy, qz, t);
-                q[u] = quad_fetch_inside(qc, r.xd, r.yd, r.zd);
-            }
-            float sc[P];
-#pragma unroll
-            for (int u = 0; u < P; ++u) sc[u] = scale_pos(quad_lerp<true>(q[u]) * w);  // Camera.cpp:201
-#pragma unroll
-            for (int u = 0; u < P; ++u) acc = add_in_order<S>(acc, sc[u]);
-        }
-        for (; kb < trips; kb += P * S) {
-            QuadFetch q[P];
-#pragma unroll
-            for (int u = 0; u < P; ++u) {
-                const float t = *(lds_float_ptr)(uintptr_t)min(t_lo + (unsigned)(kb + u * S) * 4u, t_hi);
-                const ExactIdx r = exact_index<false>(v, rx, ry, rz, qx, qy, qz, t);
-                q[u] = quad_fetch_inside(qc, r.xd, r.yd, r.zd);
-            }
-            float sc[P];
-#pragma unroll
-            for (int u = 0; u < P; ++u) {
-                sc[u] = scale_pos(quad_lerp<true>(q[u]) * w);  // Camera.cpp:201
-                sc[u] = (kb + u * S < lim) ? sc[u] : -0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < P; ++u) acc = add_in_order<S>(acc, sc[u]);
-        }
+        if (ev.fast_guards == 2 && v.div_fma2)
+            acc = march_positive<S, P, true>(v, qc, rx, ry, rz, qx, qy, qz, t_lo, t_hi, full, trips, lim, w, acc);
+        else
+            acc = march_positive<S, P, false>(v, qc, rx, ry, rz, qx, qy, qz, t_lo, t_hi, full, trips, lim, w, acc);
     }
     for (int kb = 0; !POS && kb < trips; kb += S) {
         const float t = *(const float*)((const char*)s_t + min(t_first + (unsigned)kb * 4u, t_last));
@@ -545,7 +568,7 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
         if constexpr (MODE == SM_CMEM) {
             val = cmem_sample(v.cmem, dx * t + px, dy * t + py, dz * t + pz);
         } else {
-            ExactIdx r = exact_index<true>(v, dx, dy, dz, px, py, pz, t);
+            ExactIdx r = exact_index<DIV_GUARD>(v, dx, dy, dz, px, py, pz, t);
             if constexpr (MODE == SM_QUAD_GEN) val = sample_quad<false>(qc, r.xd, r.yd, r.zd);
             else if constexpr (MODE == SM_LIN_TRI) val = sample_linear_tri(v, r);
             else val = sample_linear_nearest(v, r);
@@ -619,7 +642,7 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
 // even and backward when odd, so that every CU draws one tile from each round and the heavy
 // rounds are spread evenly (the longest-processing-time-first rule). The grid is then nblocks.
 template <int S, int MODE, int P = 1>
-__global__ __launch_bounds__(BIRP_BLOCK) void k_render_exact(DevVolume v, ExactView ev, int wg_x, int nblocks,
+__global__ __launch_bounds__(BIRP_BLOCK, MODE == SM_QUAD_POS && S < 16 ? 7 : 1) void k_render_exact(DevVolume v, ExactView ev, int wg_x, int nblocks,
                                                              const int* __restrict__ order, int ncu) {
     if ((int)blockIdx.x >= nblocks) return;
     int lb = blockIdx.x;
@@ -780,7 +803,7 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_exact_plan(DevVolume v, ExactVie
 // more tiles in flight than one view has, the SIMDs stay fed while the longest rays of a view finish.
 // `order` (may be null): block b renders item order[b] instead of item b (a batch's tile plan).
 template <int S, int MODE, int P = 1>
-__global__ __launch_bounds__(BIRP_BLOCK) void k_render_exact_multi(const DevVolume* __restrict__ vols,
+__global__ __launch_bounds__(BIRP_BLOCK, MODE == SM_QUAD_POS && S < 16 ? 7 : 1) void k_render_exact_multi(const DevVolume* __restrict__ vols,
                                                                    const ExactView* __restrict__ views,
                                                                    const int* __restrict__ prefix, int nview, int total,
                                                                    const int* __restrict__ order) {
@@ -1011,6 +1034,19 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_scan_class(const float* vals, si
         atomicMin(flags + 1, mn);
         atomicMax(flags + 2, mx);
     }
+}
+
+// birp_div_fma2 against the correctly rounded birp_div_rn64 for every significand of the dividend and
+// the three spacings; a mismatch sets bit `axis` of *bad.
+__global__ __launch_bounds__(BIRP_BLOCK) void k_check_div(DevVolume v, unsigned* bad) {
+    const unsigned m = blockIdx.x * BIRP_BLOCK + threadIdx.x;
+    if (m >= (1u << 23)) return;
+    const float a = __uint_as_float(0x3F800000u | m);
+    unsigned f = 0;
+    f |= birp_div_fma2(a, v.rhx, v.rlx) != birp_div_rn64(a, v.rdx) ? 1u : 0u;
+    f |= birp_div_fma2(a, v.rhy, v.rly) != birp_div_rn64(a, v.rdy) ? 2u : 0u;
+    f |= birp_div_fma2(a, v.rhz, v.rlz) != birp_div_rn64(a, v.rdz) ? 4u : 0u;
+    if (f) atomicOr(bad, f);
 }
 
 // Quad records: one thread per (x, y, brick z, layer 0..8) slot; tz[bz*8] is the brick's base.
@@ -1778,6 +1814,11 @@ int launch_scan_class(const float* values, size_t n, unsigned* flags_dev, void* 
     if (blocks > 4096) blocks = 4096;
     if (blocks == 0) blocks = 1;
     hipLaunchKernelGGL(k_scan_class, dim3((unsigned)blocks), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, values, n, flags_dev);
+    return hip_status(hipGetLastError());
+}
+
+int launch_check_div(const DevVolume& v, unsigned* bad_dev, void* stream) {
+    hipLaunchKernelGGL(k_check_div, dim3((1u << 23) / BIRP_BLOCK), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, v, bad_dev);
     return hip_status(hipGetLastError());
 }
 
