@@ -417,10 +417,12 @@ static bool split_reciprocal(float b, float& rh, float& rl) {
     return b >= 0x1p-20f && b <= 0x1p20f && (rl == 0.f || std::abs(rl) >= rh * 0x1p-44f);
 }
 
-// Per-axis byte-offset tables of a bricked record layout (see birp_internal.h): returns the
-// number of brick slots the layout spans, or 0 when the byte offsets would not fit 32 bits.
-static size_t brick_tables(int nx, int ny, int nz, unsigned brick_bytes, std::vector<unsigned>& tab, bool* morton) {
-    const int nbx = (nx - 1 + 7) / 8, nby = (ny - 1 + 7) / 8, nbz = (nz - 1 + 7) / 8;
+// Per-axis byte-offset tables of a bricked record layout with nz_rec records along z (see
+// birp_internal.h): returns the number of brick slots the layout spans, or 0 when the byte offsets
+// would not fit 32 bits.
+static size_t brick_tables(int nx, int ny, int nz, int nz_rec, std::vector<unsigned>& tab, bool* morton) {
+    const unsigned brick_bytes = 512u * 16u;
+    const int nbx = (nx - 1 + 7) / 8, nby = (ny - 1 + 7) / 8, nbz = (nz_rec + 7) / 8;
     int bits = 0;
     while ((1 << bits) < std::max(nbx, std::max(nby, nbz))) bits++;
     const double dense = (double)nbx * nby * nbz;
@@ -429,7 +431,6 @@ static size_t brick_tables(int nx, int ny, int nz, unsigned brick_bytes, std::ve
     const double slots = *morton ? mspace : dense;
     if (slots * brick_bytes >= 4294967296.0) return 0;
     tab.assign((size_t)nx + ny + nz, 0u);
-    const unsigned sub[3] = {16u, 128u, 1024u};
     const int dims[3] = {nx, ny, nz};
     size_t base = 0;
     for (int a = 0; a < 3; a++) {
@@ -437,7 +438,7 @@ static size_t brick_tables(int nx, int ny, int nz, unsigned brick_bytes, std::ve
             uint32_t b = (uint32_t)(i >> 3), code;
             if (*morton) code = spread3(b) << a;
             else code = a == 0 ? b : (a == 1 ? b * (uint32_t)nbx : b * (uint32_t)nbx * (uint32_t)nby);
-            tab[base + i] = code * brick_bytes + (uint32_t)(i & 7) * sub[a];
+            tab[base + i] = code * brick_bytes + (spread3((uint32_t)i & 7u) << a) * 16u;
         }
         base += dims[a];
     }
@@ -534,8 +535,8 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
     memcpy(&d.vmax, &flags[2], 4);
     if (desc->dtype == BIRP_DTYPE_F32) {
         if (desc->interp == BIRP_INTERP_TRILINEAR && d.vclass != VC_NONFINITE &&
-            (slots = brick_tables(nx, ny, nz, 576u * 16u, tab, &morton)) != 0 && (size_t)nx + ny + nz <= 8192) {
-            quad_bytes = slots * 576u * 16u;
+            (slots = brick_tables(nx, ny, nz, nz, tab, &morton)) != 0 && (size_t)nx + ny + nz <= 8192) {
+            quad_bytes = slots * 512u * 16u;
             if ((e = hipMalloc(&v->qtab, tab.size() * 4)) != hipSuccess) { rc = hip_fail(e, "hipMalloc(tables)"); goto fail_out; }
             if ((e = hipMemcpy(v->qtab, tab.data(), tab.size() * 4, hipMemcpyHostToDevice)) != hipSuccess) { rc = hip_fail(e, "tables"); goto fail_out; }
             if ((e = hipMalloc(&v->quad, quad_bytes)) != hipSuccess) { rc = hip_fail(e, "hipMalloc(quad)"); goto fail_out; }
@@ -547,7 +548,7 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
         }
     } else {
         if (d.vclass == VC_NONFINITE) { rc = fail(BIRP_ERR_UNSUPPORTED, "16-bit storage needs finite values"); goto fail_out; }
-        if ((slots = brick_tables(nx, ny, nz, 512u * 16u, tab, &morton)) == 0 || (size_t)nx + ny + nz > 2048) {
+        if ((slots = brick_tables(nx, ny, nz, nz - 1, tab, &morton)) == 0 || (size_t)nx + ny + nz > 2048) {
             rc = fail(BIRP_ERR_UNSUPPORTED, "16-bit storage supports cubes with nx+ny+nz <= 2048");
             goto fail_out;
         }

@@ -83,6 +83,13 @@ __device__ __forceinline__ float lerp_general(float a, float b, float t) {
 // Clamp in the float domain to [0, hi], then convert (NaN -> 0 in hardware).
 __device__ __forceinline__ int to_index(float x, float hi) { return (int)__builtin_amdgcn_fmed3f(x, 0.0f, hi); }
 
+// a + b + c in one instruction (two sums that share a + b would otherwise take three)
+__device__ __forceinline__ unsigned add3(unsigned a, unsigned b, unsigned c) {
+    unsigned r;
+    asm("v_add3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, unsigned bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, BIRP_RSRC_WORD3);
 }
@@ -193,9 +200,10 @@ __device__ __forceinline__ QuadFetch quad_fetch(const QuadCtx& c, float xd, floa
     q.fx = __builtin_amdgcn_fractf(xd);
     q.fy = __builtin_amdgcn_fractf(yd);
     q.fz = __builtin_amdgcn_fractf(zd);
-    unsigned off = c.tx[to_index(xd, c.hx)] + c.ty[to_index(yd, c.hy)] + c.tz[to_index(zd, c.hz)];
-    q.a = load16(c.rs, off);
-    q.b = load16(c.rs, off + 1024u);
+    const unsigned xo = c.tx[to_index(xd, c.hx)], yo = c.ty[to_index(yd, c.hy)];
+    const unsigned* zo = c.tz + to_index(zd, c.hz);
+    q.a = load16(c.rs, add3(xo, yo, zo[0]));
+    q.b = load16(c.rs, add3(xo, yo, zo[1]));
     return q;
 }
 
@@ -206,9 +214,10 @@ __device__ __forceinline__ QuadFetch quad_fetch_inside(const QuadCtx& c, float x
     q.fx = __builtin_amdgcn_fractf(xd);
     q.fy = __builtin_amdgcn_fractf(yd);
     q.fz = __builtin_amdgcn_fractf(zd);
-    unsigned off = c.tx[(int)xd] + c.ty[(int)yd] + c.tz[(int)zd];
-    q.a = load16(c.rs, off);
-    q.b = load16(c.rs, off + 1024u);
+    const unsigned xo = c.tx[(int)xd], yo = c.ty[(int)yd];
+    const unsigned* zo = c.tz + (int)zd;
+    q.a = load16(c.rs, add3(xo, yo, zo[0]));
+    q.b = load16(c.rs, add3(xo, yo, zo[1]));
     return q;
 }
 
@@ -1049,24 +1058,21 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_check_div(DevVolume v, unsigned*
     if (f) atomicOr(bad, f);
 }
 
-// Quad records: one thread per (x, y, brick z, layer 0..8) slot; tz[bz*8] is the brick's base.
+// Quad records: one thread per (x, y, z).
 __global__ __launch_bounds__(BIRP_BLOCK) void k_build_quad(DevVolume v, unsigned char* quad) {
     const unsigned* tx = v.qtab;
     const unsigned* ty = v.qtab + v.nx;
     const unsigned* tz = v.qtab + v.nx + v.ny;
     size_t cx = v.nx - 1, cy = v.ny - 1;
-    size_t total = cx * cy * (size_t)v.nbz * 9u;
+    size_t total = cx * cy * (size_t)v.nz;
     for (size_t r = (size_t)blockIdx.x * BIRP_BLOCK + threadIdx.x; r < total; r += (size_t)gridDim.x * BIRP_BLOCK) {
         int x = (int)(r % cx);
         int y = (int)((r / cx) % cy);
-        int zr = (int)(r / (cx * cy));
-        int bz = zr / 9, lz = zr % 9;
-        int z = bz * 8 + lz;
-        if (z >= v.nz) continue;
+        int z = (int)(r / (cx * cy));
         const float* L = v.linear;
         size_t base = ((size_t)z * v.ny + y) * v.nx + x;
         float4 q = make_float4(L[base], L[base + 1], L[base + v.nx], L[base + v.nx + 1]);
-        unsigned off = tx[x] + ty[y] + tz[bz * 8] + (unsigned)lz * 1024u;
+        unsigned off = tx[x] + ty[y] + tz[z];
         *(float4*)(quad + off) = q;
     }
 }
@@ -1177,9 +1183,10 @@ __device__ __forceinline__ float fast_sample(const DevVolume& v, __amdgpu_buffer
                                              float yd, float zd) {
     float fx = __builtin_amdgcn_fractf(xd), fy = __builtin_amdgcn_fractf(yd), fz = __builtin_amdgcn_fractf(zd);
     int ix = (int)xd, iy = (int)yd, iz = (int)zd;
-    unsigned off = tab[ix] + tab[v.nx + iy] + tab[v.nx + v.ny + iz];
+    const unsigned* zo = tab + v.nx + v.ny + iz;
+    const unsigned xo = tab[ix], yo = tab[v.nx + iy], off = xo + yo + zo[0];
     if constexpr (DT == BIRP_DTYPE_F32) {
-        float4 a = load16(rs, off), b = load16(rs, off + 1024u);
+        float4 a = load16(rs, off), b = load16(rs, add3(xo, yo, zo[1]));
         float ly = flerp(flerp(a.x, a.y, fx), flerp(a.z, a.w, fx), fy);
         float hy = flerp(flerp(b.x, b.y, fx), flerp(b.z, b.w, fx), fy);
         return flerp(ly, hy, fz);
@@ -1823,7 +1830,7 @@ int launch_check_div(const DevVolume& v, unsigned* bad_dev, void* stream) {
 }
 
 int launch_build_quad(const DevVolume& v, void* quad, void* stream) {
-    size_t total = (size_t)(v.nx - 1) * (v.ny - 1) * v.nbz * 9u;
+    size_t total = (size_t)(v.nx - 1) * (v.ny - 1) * v.nz;
     size_t blocks = (total + BIRP_BLOCK - 1) / BIRP_BLOCK;
     if (blocks > 65536) blocks = 65536;
     hipLaunchKernelGGL(k_build_quad, dim3((unsigned)blocks), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, v, (unsigned char*)quad);
