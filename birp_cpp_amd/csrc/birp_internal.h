@@ -32,7 +32,8 @@ namespace birp {
 enum VolumeClass : int {
     VC_POSITIVE = 0,  // every value finite and > 0: the lerps never straddle zero
     VC_FINITE = 1,    // finite, any sign
-    VC_NONFINITE = 2  // some inf/nan: only the linear layout with ceil-corner semantics is exact
+    VC_NONFINITE = 2, // some inf/nan: only the linear layout with ceil-corner semantics is exact
+    VC_NONNEG = 3     // every value finite and >= +0 (no sign bit), some zero: no sample is negative
 };
 
 enum SpaceKind : int { SK_CUBE = 0, SK_CMEM = 1 };
@@ -90,7 +91,7 @@ struct ExactView {
     int vol;          // multi-view launches: index of the view's volume in the volume table
     int accumulate;   // start from out's values
     float margin;     // FP64 slab expansion (RE) that covers FP32 position error
-    int fast_guards;  // positive cube whose scaled samples stay normal floats: 1: only the scale's
+    int fast_guards;  // cube without negative values whose scaled samples stay normal floats: 1: only the scale's
                       // midpoint guard is needed; 2: the samples also stay in birp_scale_fma2's range
     float* out;       // device image H*W
     unsigned long long* counter;  // optional: samples added (one atomic per wave)
@@ -147,10 +148,13 @@ int launch_exact_plan(const DevVolume& v, const ExactView& ev, int lanes_per_ray
 // Slots of ExactView::wave_counts for a W x H image at `lanes_per_ray` (4 waves per block).
 int exact_wave_slots(int W, int H, int lanes_per_ray);
 // Sample modes of the exact kernels. SM_QUAD_POS: positive finite cube, |origin| >= 2^-30 on every
-// axis and scaled samples that stay normal floats, so the only guard left is the scale's midpoint
-// test; SM_QUAD_GEN: any finite cube (std::lerp's branches); SM_LIN_TRI / SM_LIN_NEAREST: the
-// [z][y][x] copy (any data, nearest sampling); SM_CMEM: the analytic model.
-enum SampleMode { SM_QUAD_POS = 0, SM_QUAD_GEN = 1, SM_LIN_TRI = 2, SM_LIN_NEAREST = 3, SM_CMEM = 4 };
+// axis and scaled samples that stay normal floats, so the only guard left is the scale's; SM_QUAD_NN: the
+// same with zeros among the values; SM_NEAR_NN: nearest sampling of such a cube with or without zeros;
+// SM_QUAD_GEN: any finite cube (std::lerp's branches); SM_LIN_TRI / SM_LIN_NEAREST: the
+// [z][y][x] copy (any data, nearest sampling); SM_CMEM: the analytic model. In the first three no
+// sample is negative, so no ray stops early and the samples need no clamp of their cell.
+enum SampleMode { SM_QUAD_POS = 0, SM_QUAD_NN, SM_NEAR_NN, SM_QUAD_GEN, SM_LIN_TRI, SM_LIN_NEAREST, SM_CMEM };
+constexpr bool mode_nonneg(int mode) { return mode == SM_QUAD_POS || mode == SM_QUAD_NN || mode == SM_NEAR_NN; }
 int exact_mode_of(const DevVolume& v, const ExactView& ev);
 // Lanes per ray of multi-view exact launches of many tiles: 4 for CMEM, 2 for cubes (the measured
 // best of each). Exact batches of few small images take 4 for cubes too (exact_batch_setup).
@@ -161,7 +165,7 @@ size_t exact_lds_bytes(const DevVolume& v, int n, int mode);
 int exact_tiles(int W, int H, int lanes_per_ray);
 // Views [0, nview) of one sample mode, tiles view-major from prefix (nview + 1 entries, device),
 // at `lanes` per ray (2 or 4; SM_CMEM always takes 4) with `pipe` samples in flight per lane in the
-// positive-cube mode (2 or 4); block b renders item order_dev[b] when order_dev is given.
+// modes without negative samples (2 or 4); block b renders item order_dev[b] when order_dev is given.
 int launch_exact_multi(const DevVolume* vols_dev, const ExactView* views_dev, const int* prefix_dev, int nview, int total,
                        int mode, size_t lds, void* stream, const int* order_dev = nullptr, int lanes = 2, int pipe = 2);
 // Per-item work estimates of such a list (not for SM_CMEM) at `lanes` per ray: cost_dev[g] for g < total.

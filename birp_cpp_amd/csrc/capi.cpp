@@ -94,10 +94,10 @@ int exact_view(const birp_volume* vol, const birp_view* v, float* out_dev, Exact
                    v->ray_length + std::abs((double)d.ox) + std::abs((double)d.oy) + std::abs((double)d.oz) +
                    (double)d.nx * d.sx + (double)d.ny * d.sy + (double)d.nz * d.sz + 1.0;
     ev.margin = (float)(scale * 0x1p-16);
-    // positive cube whose scaled samples v*w*K stay normal floats: the scale needs only its
-    // midpoint guard (interpolated values stay within [vmin, vmax])
+    // cube without negative values whose nonzero values' scaled samples v*w*K stay normal floats: the
+    // scale needs only its midpoint guard (values lerped between positive ones stay within [vmin, vmax])
     const double kf = (1.0 * BIRP_SCALE_K_HOST / BIRP_SCALE_C_HOST) / 10000;
-    ev.fast_guards = (d.vclass == VC_POSITIVE && (double)d.vmin * ev.w * kf >= 0x1p-124 && (double)d.vmax * ev.w * kf <= 0x1p126) ? 1 : 0;
+    ev.fast_guards = ((d.vclass == VC_POSITIVE || d.vclass == VC_NONNEG) && (double)d.vmin * ev.w * kf >= 0x1p-124 && (double)d.vmax * ev.w * kf <= 0x1p126) ? 1 : 0;
     if (ev.fast_guards && (double)d.vmin * ev.w >= 0x1p-99 && (double)d.vmax * ev.w <= 0x1p109) ev.fast_guards = 2;
     ev.out = out_dev;
     ev.vol = 0;
@@ -529,7 +529,7 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
         rc = hip_fail(e, "class scan");
         goto fail_out;
     }
-    d.vclass = (flags[0] & 2u) ? VC_NONFINITE : (flags[0] & 1u) ? VC_FINITE : VC_POSITIVE;
+    d.vclass = (flags[0] & 2u) ? VC_NONFINITE : !(flags[0] & 1u) ? VC_POSITIVE : (flags[0] & 4u) ? VC_FINITE : VC_NONNEG;
     d.div_fma2 = splits && flags[3] == 0u && desc->dtype == BIRP_DTYPE_F32;
     memcpy(&d.vmin, &flags[1], 4);
     memcpy(&d.vmax, &flags[2], 4);
@@ -1267,7 +1267,7 @@ int exact_batch_setup(birp_batch* b) {
             if (tiny && t8 <= cap) G.lanes = 8;
             else if (small && t4 <= cap) G.lanes = 4;
             G.resident = (G.lanes == 8 ? t8 : G.lanes == 4 ? t4 : t2) <= cap;
-            if (G.resident && m == SM_QUAD_POS) G.pipe = 4;
+            if (G.resident && mode_nonneg(m)) G.pipe = 4;
         }
         prefix.push_back(0);
         for (int k = 0; k < n; k++) {

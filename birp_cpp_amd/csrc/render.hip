@@ -80,6 +80,19 @@ __device__ __forceinline__ float lerp_general(float a, float b, float t) {
     return straddle ? s1 : r;
 }
 
+// std::lerp for finite a, b and 0 <= t <= 1 - 2^-24 (no clamp: birp_lerp_unit); a and b straddle
+// zero, or one of them is zero, exactly when the median of a, b and 0 is 0.
+__device__ __forceinline__ float lerp_finite(float a, float b, float t) {
+    const float s = t * b + (1 - t) * a;
+    return __builtin_amdgcn_fmed3f(a, b, 0.0f) == 0.0f ? s : birp_lerp_unit(a, b, t);
+}
+
+// The same for a, b >= +0: a straddling pair holds a zero, t b + (1 - t) a is then exact in its zero
+// term, and for a = 0 it is what birp_lerp_unit gives.
+__device__ __forceinline__ float lerp_nonneg(float a, float b, float t) {
+    return b == 0.0f ? (1 - t) * a : birp_lerp_unit(a, b, t);
+}
+
 // Clamp in the float domain to [0, hi], then convert (NaN -> 0 in hardware).
 __device__ __forceinline__ int to_index(float x, float hi) { return (int)__builtin_amdgcn_fmed3f(x, 0.0f, hi); }
 
@@ -184,6 +197,7 @@ struct QuadCtx {
     const unsigned* ty;
     const unsigned* tz;
     float hx, hy, hz;  // n - 2 per axis
+    unsigned row, slice;  // nearest: nx and nx ny, rs the [z][y][x] copy
 };
 
 // For an in-cube sample the index is >= 0, so the lower corner floor(x) is the truncating
@@ -207,6 +221,13 @@ __device__ __forceinline__ QuadFetch quad_fetch(const QuadCtx& c, float xd, floa
     return q;
 }
 
+// Nearest (DataCube.cpp:273) of a sample that passed the reference's bounds test: the value at the
+// truncated index, from the [z][y][x] copy (nx ny < 2^24 and under 2^30 values: exact_mode_of).
+__device__ __forceinline__ float near_fetch(const QuadCtx& c, float xd, float yd, float zd) {
+    const unsigned at = __umul24((unsigned)(int)zd, c.slice) + (__umul24((unsigned)(int)yd, c.row) + (unsigned)(int)xd);
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(c.rs, (int)(at * 4u), 0, 0));
+}
+
 // For a sample that passed the reference's bounds test (0 <= ingress, index + 1 < n): the index
 // is in [0, n-1), so its truncation is the lower corner and needs no clamp.
 __device__ __forceinline__ QuadFetch quad_fetch_inside(const QuadCtx& c, float xd, float yd, float zd) {
@@ -222,23 +243,27 @@ __device__ __forceinline__ QuadFetch quad_fetch_inside(const QuadCtx& c, float x
 }
 
 // x first, then y, then z (DataCube.cpp:260-270).
-template <bool POS>
+enum LerpForm { LERP_POS, LERP_NONNEG, LERP_FINITE };
+template <int LERP>
 __device__ __forceinline__ float quad_lerp(const QuadFetch& q) {
+    auto lerp = [](float a, float b, float t) {
+        return LERP == LERP_POS ? birp_lerp_unit(a, b, t) : LERP == LERP_NONNEG ? lerp_nonneg(a, b, t) : lerp_finite(a, b, t);
+    };
     const float4 a = q.a, b = q.b;
-    if constexpr (POS) {
-        float ly = birp_lerp_unit(birp_lerp_unit(a.x, a.y, q.fx), birp_lerp_unit(a.z, a.w, q.fx), q.fy);
-        float hy = birp_lerp_unit(birp_lerp_unit(b.x, b.y, q.fx), birp_lerp_unit(b.z, b.w, q.fx), q.fy);
-        return birp_lerp_unit(ly, hy, q.fz);
-    } else {
-        float ly = lerp_general(lerp_general(a.x, a.y, q.fx), lerp_general(a.z, a.w, q.fx), q.fy);
-        float hy = lerp_general(lerp_general(b.x, b.y, q.fx), lerp_general(b.z, b.w, q.fx), q.fy);
-        return lerp_general(ly, hy, q.fz);
-    }
+    const float ly = lerp(lerp(a.x, a.y, q.fx), lerp(a.z, a.w, q.fx), q.fy);
+    const float hy = lerp(lerp(b.x, b.y, q.fx), lerp(b.z, b.w, q.fx), q.fy);
+    return lerp(ly, hy, q.fz);
 }
 
-template <bool POS>
-__device__ __forceinline__ float sample_quad(const QuadCtx& c, float xd, float yd, float zd) {
-    return quad_lerp<POS>(quad_fetch(c, xd, yd, zd));
+// The least (or, MAX, the greatest) corner of a cell without negative values, as its bits.
+template <bool MAX>
+__device__ __forceinline__ unsigned fold_corners(const QuadFetch& q) {
+    auto f = [](float x, float y, float z) {
+        const unsigned a = __float_as_uint(x), b = __float_as_uint(y), c = __float_as_uint(z);
+        return __uint_as_float(MAX ? max(max(a, b), c) : min(min(a, b), c));
+    };
+    const float m = f(q.a.x, q.a.y, q.a.z), n = f(q.a.w, q.b.x, q.b.y);
+    return __float_as_uint(f(f(m, n, q.b.z), q.b.w, q.b.w));
 }
 
 // The scale chain of Camera.cpp:201 for a positive cube whose scaled samples stay normal floats:
@@ -275,6 +300,18 @@ __device__ __forceinline__ float add_in_order(float acc, float s) {
         acc = acc + row_next_f<12>(sr);
     }
     return acc;
+}
+
+// Sub-lane m's value of this ray, on sub-lane 0.
+template <int S>
+__device__ __forceinline__ float sub_lane_f(float s, int m) {
+    if (m >= 4) s = __shfl_down(s, 16 * (m >> 2), 64);
+    switch (m & 3) {
+        case 1: return row_next_f<4>(s);
+        case 2: return row_next_f<8>(s);
+        case 3: return row_next_f<12>(s);
+        default: return s;
+    }
 }
 
 // Trilinear sample from the [z][y][x] layout with floor/ceil corners (DataCube.cpp:224-270):
@@ -432,9 +469,9 @@ __device__ __forceinline__ void exact_lane(int lane, int& ti, int& tj, int& sub)
 }
 
 
-// The samples of a wave's rays over a positive cube, added in k order (exact_block's main loop).
-// P samples per lane per iteration (k, k + S, ...), staged so that the later samples' LDS and
-// buffer reads are in flight while the first ones' lerps run. The sum order is unchanged: the S
+// The samples of a wave's rays over a cube without negative values, added in k order (exact_block's
+// main loop). P samples per lane per iteration (k, k + S, ...), staged so that the later samples' LDS
+// and buffer reads are in flight while the first ones' lerps run. The sum order is unchanged: the S
 // samples at k, then the S samples at k + S, and so on.
 // Every lane samples inside the cube, so the corner indices need no clamp: a lane past its ray's last
 // in-cube sample kl re-reads kl's t (its result is masked), and a lane whose ray has no in-cube
@@ -445,52 +482,65 @@ __device__ __forceinline__ void exact_lane(int lane, int& ti, int& tj, int& sub)
 // the clamp of t's address nor the mask, and read their P t values at constant offsets from one
 // address; the arithmetic and the sum order are those of the masked trips.
 // FMA2: divisions and scale as one multiply and one FMA each (birp_div_fma2, birp_scale_fma2), where the
-// volume's spacings and values allow it: 51 VALU instructions per sample and no branch, against 57
+// volume's spacings and values allow it: 52 VALU instructions per sample and no branch, against 58
 // and one rarely taken branch per sample. Issue-bound batches gain what the instructions save (64 orbit
 // views of a 256^3 cube: 1.189 ms with FP64 divisions and scale and clamped lerps, 1.058 ms now); a
 // single 576x336 x 800 view, whose waves also wait on the vector L1, goes from 87.4 to 84.7 us.
+// SM_QUAD_NN: a cell of positive corners lerps as in SM_QUAD_POS, an empty one gives 0 either way, and
+// only a cell with both takes std::lerp's zero branches and the scale's full test (its values can be
+// arbitrarily small): the least corner finds the samples where some lane has such a cell, on the
+// surfaces of a cavity, and inside it. 3 samples in flight instead of 4 (the branch keeps corners alive:
+// 4 spill). A 256^3 cube with an empty cavity, 576x336 x 800: 270 us with the general lerps, their stop
+// test and one sample in flight, 75 us now (72 without zeros); 64 orbit views 3.35 -> 0.97 ms.
+// SM_NEAR_NN: one value per sample from the [z][y][x] copy, its index in two 24-bit multiply-adds:
+// 576x336 x 800 124 -> 56 us, a camera inside a 144^3 cube at 265x155 x 200 29.4 -> 11.5 us.
 typedef __attribute__((address_space(3))) const float* lds_float_ptr;
-template <int S, int P, bool FMA2>
-__device__ __forceinline__ float march_positive(const DevVolume& v, const QuadCtx& qc, float rx, float ry, float rz, float qx, float qy,
-                                                float qz, unsigned t_lo, unsigned t_hi, int full, int trips, int lim, float w, float acc) {
+template <int S, int P, int MODE, bool FMA2, bool MASK>
+__device__ __forceinline__ float march_trip(const DevVolume& v, const QuadCtx& qc, float rx, float ry, float rz, float qx, float qy,
+                                            float qz, unsigned t_lo, unsigned t_hi, int kb, int lim, float w, float acc) {
+    constexpr bool NEAR = MODE == SM_NEAR_NN;
     constexpr int DIV = FMA2 ? DIV_FMA2 : DIV_RN64;
-    auto scaled = [&](const QuadFetch& q) {  // Camera.cpp:201
-        const float vw = quad_lerp<true>(q) * w;
-        return FMA2 ? birp_scale_fma2(vw) : scale_pos(vw);
-    };
+    QuadFetch q[NEAR ? 1 : P];
+    float near[NEAR ? P : 1];
+    const unsigned tb = t_lo + (unsigned)kb * 4u;
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+        const unsigned ta = tb + (unsigned)(u * S) * 4u;
+        const float t = *(lds_float_ptr)(uintptr_t)(MASK ? min(ta, t_hi) : ta);
+        const ExactIdx r = exact_index<DIV>(v, rx, ry, rz, qx, qy, qz, t);
+        if constexpr (NEAR) near[u] = near_fetch(qc, r.xd, r.yd, r.zd);
+        else q[u] = quad_fetch_inside(qc, r.xd, r.yd, r.zd);
+    }
+    float sc[P];
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+        float val;
+        if constexpr (NEAR) val = near[u];
+        else val = quad_lerp<LERP_POS>(q[u]);
+        const float vw = val * w;  // Camera.cpp:201
+        sc[u] = FMA2 ? birp_scale_fma2(vw) : scale_pos(vw);
+        if constexpr (MODE == SM_QUAD_NN) {
+            if (__builtin_expect(fold_corners<false>(q[u]) == 0u, 0) && fold_corners<true>(q[u]) != 0u)
+                sc[u] = birp_scale_sample(quad_lerp<LERP_NONNEG>(q[u]) * w);
+        }
+    }
+    if constexpr (MASK) {
+#pragma unroll
+        for (int u = 0; u < P; ++u) sc[u] = (kb + u * S < lim) ? sc[u] : -0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < P; ++u) acc = add_in_order<S>(acc, sc[u]);
+    return acc;
+}
+
+template <int S, int P, int MODE, bool FMA2>
+__device__ __forceinline__ float march_nonneg(const DevVolume& v, const QuadCtx& qc, float rx, float ry, float rz, float qx, float qy,
+                                              float qz, unsigned t_lo, unsigned t_hi, int full, int trips, int lim, float w, float acc) {
     int kb = 0;
-    for (; kb + P * S <= full; kb += P * S) {
-        QuadFetch q[P];
-        const unsigned tb = t_lo + (unsigned)kb * 4u;
-#pragma unroll
-        for (int u = 0; u < P; ++u) {
-            const float t = *(lds_float_ptr)(uintptr_t)(tb + (unsigned)(u * S) * 4u);
-            const ExactIdx r = exact_index<DIV>(v, rx, ry, rz, qx, qy, qz, t);
-            q[u] = quad_fetch_inside(qc, r.xd, r.yd, r.zd);
-        }
-        float sc[P];
-#pragma unroll
-        for (int u = 0; u < P; ++u) sc[u] = scaled(q[u]);
-#pragma unroll
-        for (int u = 0; u < P; ++u) acc = add_in_order<S>(acc, sc[u]);
-    }
-    for (; kb < trips; kb += P * S) {
-        QuadFetch q[P];
-#pragma unroll
-        for (int u = 0; u < P; ++u) {
-            const float t = *(lds_float_ptr)(uintptr_t)min(t_lo + (unsigned)(kb + u * S) * 4u, t_hi);
-            const ExactIdx r = exact_index<DIV>(v, rx, ry, rz, qx, qy, qz, t);
-            q[u] = quad_fetch_inside(qc, r.xd, r.yd, r.zd);
-        }
-        float sc[P];
-#pragma unroll
-        for (int u = 0; u < P; ++u) {
-            sc[u] = scaled(q[u]);
-            sc[u] = (kb + u * S < lim) ? sc[u] : -0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < P; ++u) acc = add_in_order<S>(acc, sc[u]);
-    }
+    for (; kb + P * S <= full; kb += P * S)
+        acc = march_trip<S, P, MODE, FMA2, false>(v, qc, rx, ry, rz, qx, qy, qz, t_lo, t_hi, kb, lim, w, acc);
+    for (; kb < trips; kb += P * S)
+        acc = march_trip<S, P, MODE, FMA2, true>(v, qc, rx, ry, rz, qx, qy, qz, t_lo, t_hi, kb, lim, w, acc);
     return acc;
 }
 
@@ -500,8 +550,8 @@ __device__ __forceinline__ float march_positive(const DevVolume& v, const QuadCt
 // ------------------------------------------------------------------------------------------
 template <int S, int MODE, int P>
 __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView& ev, int lb, int wg_x) {
-    constexpr bool QUAD = (MODE == SM_QUAD_POS || MODE == SM_QUAD_GEN);
-    constexpr bool POS = (MODE == SM_QUAD_POS);
+    constexpr bool QUAD = (MODE == SM_QUAD_POS || MODE == SM_QUAD_NN || MODE == SM_QUAD_GEN);
+    constexpr bool NN = mode_nonneg(MODE);
     extern __shared__ unsigned s_mem[];
     float* s_t = (float*)s_mem;
     const int n = ev.n;
@@ -519,6 +569,10 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
         qc.hx = v.fnx - 2.0f;
         qc.hy = v.fny - 2.0f;
         qc.hz = v.fnz - 2.0f;
+    } else if constexpr (MODE == SM_NEAR_NN) {
+        qc.row = (unsigned)v.nx;
+        qc.slice = (unsigned)v.nx * (unsigned)v.ny;
+        qc.rs = make_rsrc(v.linear, qc.slice * (unsigned)v.nz * 4u);
     }
     __syncthreads();
 
@@ -551,12 +605,11 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
 
     float acc = 0.f;
     if (valid && ev.accumulate) acc = ev.out[(size_t)j * ev.W + i];
-    bool alive = true;
-    unsigned added = 0;
+    unsigned added = (unsigned)len;
     const float w = ev.w;
     const float px = ev.px, py = ev.py, pz = ev.pz;
 
-    if constexpr (POS) {
+    if constexpr (NN) {
         const bool has = len > 0;
         const float rx = has ? dx : 0.f, ry = has ? dy : 0.f, rz = has ? dz : 0.f;
         const float qx = has ? px : v.ox, qy = has ? py : v.oy, qz = has ? pz : v.oz;
@@ -566,11 +619,16 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
         asm volatile("" : "+v"(t_lo), "+v"(t_hi));
         const int full = wave_min_i(len);
         if (ev.fast_guards == 2 && v.div_fma2)
-            acc = march_positive<S, P, true>(v, qc, rx, ry, rz, qx, qy, qz, t_lo, t_hi, full, trips, lim, w, acc);
+            acc = march_nonneg<S, P, MODE, true>(v, qc, rx, ry, rz, qx, qy, qz, t_lo, t_hi, full, trips, lim, w, acc);
         else
-            acc = march_positive<S, P, false>(v, qc, rx, ry, rz, qx, qy, qz, t_lo, t_hi, full, trips, lim, w, acc);
+            acc = march_nonneg<S, P, MODE, false>(v, qc, rx, ry, rz, qx, qy, qz, t_lo, t_hi, full, trips, lim, w, acc);
     }
-    for (int kb = 0; !POS && kb < trips; kb += S) {
+    // Any data: a ray stops at its first negative sample (Camera.cpp:207-210). While no sample of the wave
+    // is negative and no ray of it has stopped, the samples are added as above; after that each ray
+    // gathers its S samples and tests them in k order on sub-lane 0 (the other sub-lanes' sums and stops
+    // are not used).
+    bool alive = true, quiet = true;
+    for (int kb = 0; !NN && kb < trips; kb += S) {
         const float t = *(const float*)((const char*)s_t + min(t_first + (unsigned)kb * 4u, t_last));
         const bool act = kb < lim;
         float val;
@@ -578,60 +636,26 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
             val = cmem_sample(v.cmem, dx * t + px, dy * t + py, dz * t + pz);
         } else {
             ExactIdx r = exact_index<DIV_GUARD>(v, dx, dy, dz, px, py, pz, t);
-            if constexpr (MODE == SM_QUAD_GEN) val = sample_quad<false>(qc, r.xd, r.yd, r.zd);
+            if constexpr (MODE == SM_QUAD_GEN) val = quad_lerp<LERP_FINITE>(quad_fetch(qc, r.xd, r.yd, r.zd));
             else if constexpr (MODE == SM_LIN_TRI) val = sample_linear_tri(v, r);
             else val = sample_linear_nearest(v, r);
         }
-        const float vw = val * w;  // Camera.cpp:201
-        {
-            const float s = birp_scale_sample(vw);
-            if constexpr (S == 1) {
-                bool add = act && alive;
-                bool stop = add && (s < 0);  // Camera.cpp:207-210
-                acc = (add && !stop) ? acc + s : acc;
-                added += (add && !stop) ? 1u : 0u;
+        const float s = birp_scale_sample(val * w);  // Camera.cpp:201
+        quiet = quiet && __ballot(act && s < 0) == 0ull;
+        if (quiet) {
+            acc = add_in_order<S>(acc, act ? s : -0.0f);
+        } else {
+#pragma unroll
+            for (int mm = 0; mm < S; ++mm) {
+                const float sm = sub_lane_f<S>(s, mm);
+                const bool add = alive && kb + mm < len;
+                const bool stop = add && sm < 0;
+                acc = (add && !stop) ? acc + sm : acc;
+                if (stop) added = (unsigned)(kb + mm);
                 alive = alive && !stop;
-            } else {
-                // sub-lane 0 gathers the ray's S samples in k order (the other sub-lanes'
-                // sums and stops are not used)
-                float sv[S];
-                int av[S];
-                const int ai = act ? 1 : 0;
-                sv[0] = s;
-                av[0] = ai;
-                sv[1] = row_next_f<4>(s);
-                av[1] = row_next<4>(ai);
-                if constexpr (S >= 4) {
-                    sv[2] = row_next_f<8>(s);
-                    av[2] = row_next<8>(ai);
-                    sv[3] = row_next_f<12>(s);
-                    av[3] = row_next<12>(ai);
-                }
-#pragma unroll
-                for (int rr = 1; rr < S / 4; ++rr) {  // sub-lanes 4rr..4rr+3: row rr
-                    const float sr = __shfl_down(s, 16 * rr, 64);
-                    const int ar = __shfl_down(ai, 16 * rr, 64);
-                    sv[4 * rr] = sr;
-                    av[4 * rr] = ar;
-                    sv[4 * rr + 1] = row_next_f<4>(sr);
-                    av[4 * rr + 1] = row_next<4>(ar);
-                    sv[4 * rr + 2] = row_next_f<8>(sr);
-                    av[4 * rr + 2] = row_next<8>(ar);
-                    sv[4 * rr + 3] = row_next_f<12>(sr);
-                    av[4 * rr + 3] = row_next<12>(ar);
-                }
-#pragma unroll
-                for (int mm = 0; mm < S; ++mm) {
-                    bool add = av[mm] && alive;
-                    bool stop = add && (sv[mm] < 0);
-                    acc = (add && !stop) ? acc + sv[mm] : acc;
-                    added += (add && !stop) ? 1u : 0u;
-                    alive = alive && !stop;
-                }
             }
         }
     }
-    if constexpr (POS) added = (unsigned)len;
     if (valid && sub == 0) ev.out[(size_t)j * ev.W + i] = acc;
     if (ev.counter || ev.wave_counts) {
         unsigned tot = wave_sum_u((valid && sub == 0) ? added : 0u);
@@ -640,6 +664,12 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
             else if (tot) atomicAdd(ev.counter, (unsigned long long)tot);
         }
     }
+}
+
+// Waves per SIMD the exact kernels' registers leave room for: 7 where no spill follows (72 VGPRs); the rare
+// branch of SM_QUAD_NN and the shuffles of 8 and 16 lanes per ray take more.
+constexpr int exact_waves(int S, int mode) {
+    return !mode_nonneg(mode) || S == 16 ? 1 : (mode == SM_QUAD_NN && S == 8 ? 6 : 7);
 }
 
 // One view: block b renders tile lb(b).
@@ -651,7 +681,7 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
 // even and backward when odd, so that every CU draws one tile from each round and the heavy
 // rounds are spread evenly (the longest-processing-time-first rule). The grid is then nblocks.
 template <int S, int MODE, int P = 1>
-__global__ __launch_bounds__(BIRP_BLOCK, MODE == SM_QUAD_POS && S < 16 ? 7 : 1) void k_render_exact(DevVolume v, ExactView ev, int wg_x, int nblocks,
+__global__ __launch_bounds__(BIRP_BLOCK, exact_waves(S, MODE)) void k_render_exact(DevVolume v, ExactView ev, int wg_x, int nblocks,
                                                              const int* __restrict__ order, int ncu) {
     if ((int)blockIdx.x >= nblocks) return;
     int lb = blockIdx.x;
@@ -812,7 +842,7 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_exact_plan(DevVolume v, ExactVie
 // more tiles in flight than one view has, the SIMDs stay fed while the longest rays of a view finish.
 // `order` (may be null): block b renders item order[b] instead of item b (a batch's tile plan).
 template <int S, int MODE, int P = 1>
-__global__ __launch_bounds__(BIRP_BLOCK, MODE == SM_QUAD_POS && S < 16 ? 7 : 1) void k_render_exact_multi(const DevVolume* __restrict__ vols,
+__global__ __launch_bounds__(BIRP_BLOCK, exact_waves(S, MODE)) void k_render_exact_multi(const DevVolume* __restrict__ vols,
                                                                    const ExactView* __restrict__ views,
                                                                    const int* __restrict__ prefix, int nview, int total,
                                                                    const int* __restrict__ order) {
@@ -1018,7 +1048,7 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_sample_points(DevVolume v, const
 // ------------------------------------------------------------------------------------------
 // layout builders and scans
 // ------------------------------------------------------------------------------------------
-// flags[0]: bit 0 = some value <= 0, bit 1 = some value non-finite; flags[1], flags[2]: min and
+// flags[0]: bit 0 = some value <= 0, bit 1 = some value non-finite, bit 2 = some sign bit set; flags[1], flags[2]: min and
 // max of |v| over the nonzero finite values as float bits (ordered as unsigned for positive floats).
 __global__ __launch_bounds__(BIRP_BLOCK) void k_scan_class(const float* vals, size_t n, unsigned* flags) {
     unsigned f = 0, mn = 0x7F7FFFFFu, mx = 0u;
@@ -1026,6 +1056,7 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_scan_class(const float* vals, si
         float x = vals[idx];
         if (!(x > 0.f)) f |= 1u;
         if (!isfinite(x)) f |= 2u;
+        if (__float_as_uint(x) >> 31) f |= 4u;
         float a = fabsf(x);
         if (a > 0.f && isfinite(a)) {
             unsigned u = __float_as_uint(a);
@@ -1183,15 +1214,16 @@ __device__ __forceinline__ float fast_sample(const DevVolume& v, __amdgpu_buffer
                                              float yd, float zd) {
     float fx = __builtin_amdgcn_fractf(xd), fy = __builtin_amdgcn_fractf(yd), fz = __builtin_amdgcn_fractf(zd);
     int ix = (int)xd, iy = (int)yd, iz = (int)zd;
-    const unsigned* zo = tab + v.nx + v.ny + iz;
-    const unsigned xo = tab[ix], yo = tab[v.nx + iy], off = xo + yo + zo[0];
     if constexpr (DT == BIRP_DTYPE_F32) {
-        float4 a = load16(rs, off), b = load16(rs, add3(xo, yo, zo[1]));
+        const unsigned xo = tab[ix], yo = tab[v.nx + iy];
+        const unsigned* zo = tab + v.nx + v.ny + iz;
+        float4 a = load16(rs, add3(xo, yo, zo[0])), b = load16(rs, add3(xo, yo, zo[1]));
         float ly = flerp(flerp(a.x, a.y, fx), flerp(a.z, a.w, fx), fy);
         float hy = flerp(flerp(b.x, b.y, fx), flerp(b.z, b.w, fx), fy);
         return flerp(ly, hy, fz);
     } else {  // BF16, F16 with per-brick scale, F16 with one scale (BIRP_KDT_F16_UNIFORM)
         // each dword of the record holds the x-pair (x0, x1) of one (y, z) corner row
+        const unsigned off = tab[ix] + tab[v.nx + iy] + tab[v.nx + v.ny + iz];
         uint4 o = load16u(rs, off);
         float c00, c10, c01, c11;  // the four x-lerps, at (y0,z0), (y1,z0), (y0,z1), (y1,z1)
         if constexpr (DT == BIRP_DTYPE_BF16) {
@@ -1649,15 +1681,19 @@ static int hip_status(hipError_t e) { return e == hipSuccess ? BIRP_OK : BIRP_ER
 
 int exact_mode_of(const DevVolume& v, const ExactView& ev) {
     if (v.kind == SK_CMEM) return SM_CMEM;
-    if (v.interp == BIRP_INTERP_NEAREST) return SM_LIN_NEAREST;
+    const bool nonneg = (v.vclass == VC_POSITIVE || v.vclass == VC_NONNEG) && v.origin_far && ev.fast_guards;
+    if (v.interp == BIRP_INTERP_NEAREST) {
+        const size_t slice = (size_t)v.nx * v.ny;  // near_fetch: 24-bit products, 32-bit byte offsets
+        return nonneg && slice < (1u << 24) && slice * v.nz < (1u << 30) ? SM_NEAR_NN : SM_LIN_NEAREST;
+    }
     if (v.vclass == VC_NONFINITE || !v.quad || !v.qtab) return SM_LIN_TRI;
-    if (v.vclass == VC_POSITIVE && v.origin_far && ev.fast_guards) return SM_QUAD_POS;
+    if (nonneg) return v.vclass == VC_POSITIVE ? SM_QUAD_POS : SM_QUAD_NN;
     return SM_QUAD_GEN;
 }
 
 size_t exact_lds_bytes(const DevVolume& v, int n, int mode) {
     size_t lds = (size_t)((n + 3) & ~3) * sizeof(float);
-    if (mode == SM_QUAD_POS || mode == SM_QUAD_GEN) lds += (size_t)(v.nx + v.ny + v.nz) * sizeof(unsigned);
+    if (mode == SM_QUAD_POS || mode == SM_QUAD_NN || mode == SM_QUAD_GEN) lds += (size_t)(v.nx + v.ny + v.nz) * sizeof(unsigned);
     return lds;
 }
 
@@ -1685,12 +1721,22 @@ static int launch_exact_s(const DevVolume& v, const ExactView& ev, int pipe, hip
         ncu = ord->ncu;
     }
     switch (mode) {
+#define BIRP_LRE(MODE, P) hipLaunchKernelGGL((k_render_exact<S, MODE, P>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, ev, wg_x, nblocks, order, ncu)
         case SM_QUAD_POS:
-            if (pipe >= 4) hipLaunchKernelGGL((k_render_exact<S, SM_QUAD_POS, 4>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, ev, wg_x, nblocks, order, ncu);
-            else if (pipe == 3) hipLaunchKernelGGL((k_render_exact<S, SM_QUAD_POS, 3>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, ev, wg_x, nblocks, order, ncu);
-            else if (pipe == 1) hipLaunchKernelGGL((k_render_exact<S, SM_QUAD_POS, 1>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, ev, wg_x, nblocks, order, ncu);
-            else hipLaunchKernelGGL((k_render_exact<S, SM_QUAD_POS, 2>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, ev, wg_x, nblocks, order, ncu);
+            if (pipe >= 4) BIRP_LRE(SM_QUAD_POS, 4);
+            else if (pipe == 3) BIRP_LRE(SM_QUAD_POS, 3);
+            else if (pipe == 1) BIRP_LRE(SM_QUAD_POS, 1);
+            else BIRP_LRE(SM_QUAD_POS, 2);
             break;
+        case SM_QUAD_NN:
+            if (pipe >= 3) BIRP_LRE(SM_QUAD_NN, 3);
+            else BIRP_LRE(SM_QUAD_NN, 2);
+            break;
+        case SM_NEAR_NN:
+            if (pipe >= 3) BIRP_LRE(SM_NEAR_NN, 4);
+            else BIRP_LRE(SM_NEAR_NN, 2);
+            break;
+#undef BIRP_LRE
         case SM_QUAD_GEN: hipLaunchKernelGGL((k_render_exact<S, SM_QUAD_GEN>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, ev, wg_x, nblocks, order, ncu); break;
         case SM_LIN_TRI: hipLaunchKernelGGL((k_render_exact<S, SM_LIN_TRI>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, ev, wg_x, nblocks, order, ncu); break;
         case SM_LIN_NEAREST: hipLaunchKernelGGL((k_render_exact<S, SM_LIN_NEAREST>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, ev, wg_x, nblocks, order, ncu); break;
@@ -1718,10 +1764,20 @@ static int launch_exact_multi_s(const DevVolume* vols, const ExactView* views, c
                                 size_t lds, hipStream_t st, const int* order, int pipe) {
     const int grid = total;
     switch (mode) {
+#define BIRP_LRM(MODE, P) hipLaunchKernelGGL((k_render_exact_multi<S, MODE, P>), dim3(grid), dim3(BIRP_BLOCK), lds, st, vols, views, prefix, nview, total, order)
         case SM_QUAD_POS:
-            if (pipe >= 4) hipLaunchKernelGGL((k_render_exact_multi<S, SM_QUAD_POS, 4>), dim3(grid), dim3(BIRP_BLOCK), lds, st, vols, views, prefix, nview, total, order);
-            else hipLaunchKernelGGL((k_render_exact_multi<S, SM_QUAD_POS, 2>), dim3(grid), dim3(BIRP_BLOCK), lds, st, vols, views, prefix, nview, total, order);
+            if (pipe >= 4) BIRP_LRM(SM_QUAD_POS, 4);
+            else BIRP_LRM(SM_QUAD_POS, 2);
             break;
+        case SM_QUAD_NN:
+            if (pipe >= 4) BIRP_LRM(SM_QUAD_NN, 3);
+            else BIRP_LRM(SM_QUAD_NN, 2);
+            break;
+        case SM_NEAR_NN:
+            if (pipe >= 4) BIRP_LRM(SM_NEAR_NN, 4);
+            else BIRP_LRM(SM_NEAR_NN, 2);
+            break;
+#undef BIRP_LRM
         case SM_QUAD_GEN: hipLaunchKernelGGL((k_render_exact_multi<S, SM_QUAD_GEN>), dim3(grid), dim3(BIRP_BLOCK), lds, st, vols, views, prefix, nview, total, order); break;
         case SM_LIN_TRI: hipLaunchKernelGGL((k_render_exact_multi<S, SM_LIN_TRI>), dim3(grid), dim3(BIRP_BLOCK), lds, st, vols, views, prefix, nview, total, order); break;
         case SM_LIN_NEAREST: hipLaunchKernelGGL((k_render_exact_multi<S, SM_LIN_NEAREST>), dim3(grid), dim3(BIRP_BLOCK), lds, st, vols, views, prefix, nview, total, order); break;

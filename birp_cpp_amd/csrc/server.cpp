@@ -360,7 +360,7 @@ int launch_slot(birp_server* S, Slot& s) {
         const long long cap = 7LL * S->dev->ncu;
         if (etiny[m] && et8[m] <= cap) elanes[m] = 8;
         else if (esmall[m] && et4[m] <= cap) elanes[m] = 4;
-        if (m == SM_QUAD_POS && (elanes[m] == 8 ? et8[m] : elanes[m] == 4 ? et4[m] : et2[m]) <= cap) epipe[m] = 4;
+        if (mode_nonneg(m) && (elanes[m] == 8 ? et8[m] : elanes[m] == 4 ? et4[m] : et2[m]) <= cap) epipe[m] = 4;
     }
     int nexact = 0;
     for (int m = 0; m < kModes; m++) nexact += ecount[m];
