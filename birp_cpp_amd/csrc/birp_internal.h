@@ -183,6 +183,12 @@ int launch_fast_batch(const DevVolume* vols_dev, int dtype, const FastPose* pose
                       int lanes_per_ray, int unroll, int grid, void* stream, int tab_entries);
 int launch_reset_counter(unsigned* counter, void* stream);
 int launch_zero_f32(float* p, size_t n, void* stream);
+// Words of the class scan's flags (one cache line each), in a buffer of BIRP_SCAN_WORDS.
+#define BIRP_SCAN_CLASS 0
+#define BIRP_SCAN_MIN 64
+#define BIRP_SCAN_MAX 128
+#define BIRP_SCAN_DIV 192 /* launch_check_div */
+#define BIRP_SCAN_WORDS 193
 int launch_scan_class(const float* values, size_t n, unsigned* flags_dev, void* stream);
 // Checks birp_div_fma2 for the volume's spacings over every significand: ORs bit `axis` into *bad_dev for
 // an axis with a mismatch.

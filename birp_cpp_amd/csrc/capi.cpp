@@ -285,7 +285,7 @@ extern "C" int birp_device_open(int ordinal, birp_device** out) {
     else if ((e = hipEventCreate(&d->ev0)) != hipSuccess || (e = hipEventCreate(&d->ev1)) != hipSuccess ||
              (e = hipEventCreate(&d->ev_a)) != hipSuccess || (e = hipEventCreate(&d->ev_b)) != hipSuccess)
         what = "hipEventCreate";
-    else if ((e = hipMalloc(&d->d_counter, 64)) != hipSuccess) what = "hipMalloc(counter)";
+    else if ((e = hipMalloc(&d->d_counter, BIRP_SCAN_WORDS * sizeof(unsigned))) != hipSuccess) what = "hipMalloc(counter)";
     else if ((e = hipMalloc(&d->plan_order, birp_device::kPlanSlots * BIRP_PLAN_INTS * sizeof(int))) != hipSuccess)
         what = "hipMalloc(tile plans)";
     else if ((e = hipMemsetAsync(d->plan_order, 0, birp_device::kPlanSlots * BIRP_PLAN_INTS * sizeof(int), d->stream)) != hipSuccess)
@@ -507,7 +507,8 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
 
     hipError_t e;
     int rc = BIRP_OK;
-    unsigned flags[4] = {0u, 0x7F7FFFFFu, 0u, 0u};
+    unsigned flags[BIRP_SCAN_WORDS] = {}, cls = 0;
+    flags[BIRP_SCAN_MIN] = 0x7F7FFFFFu;
     unsigned* dflags = (unsigned*)dev->d_counter;
     size_t quad_bytes = 0, oct_bytes = 0, slots = 0;
     bool morton = false;
@@ -523,16 +524,17 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
         goto fail_out;
     }
     if ((rc = launch_scan_class(v->linear, nvox, dflags, dev->stream)) != BIRP_OK) goto fail_out;
-    if (splits && desc->dtype == BIRP_DTYPE_F32 && (rc = launch_check_div(d, dflags + 3, dev->stream)) != BIRP_OK) goto fail_out;
+    if (splits && desc->dtype == BIRP_DTYPE_F32 && (rc = launch_check_div(d, dflags + BIRP_SCAN_DIV, dev->stream)) != BIRP_OK) goto fail_out;
     if ((e = hipMemcpyAsync(flags, dflags, sizeof(flags), hipMemcpyDeviceToHost, dev->stream)) != hipSuccess ||
         (e = hipStreamSynchronize(dev->stream)) != hipSuccess) {
         rc = hip_fail(e, "class scan");
         goto fail_out;
     }
-    d.vclass = (flags[0] & 2u) ? VC_NONFINITE : !(flags[0] & 1u) ? VC_POSITIVE : (flags[0] & 4u) ? VC_FINITE : VC_NONNEG;
-    d.div_fma2 = splits && flags[3] == 0u && desc->dtype == BIRP_DTYPE_F32;
-    memcpy(&d.vmin, &flags[1], 4);
-    memcpy(&d.vmax, &flags[2], 4);
+    cls = flags[BIRP_SCAN_CLASS];
+    d.vclass = (cls & 2u) ? VC_NONFINITE : !(cls & 1u) ? VC_POSITIVE : (cls & 4u) ? VC_FINITE : VC_NONNEG;
+    d.div_fma2 = splits && flags[BIRP_SCAN_DIV] == 0u && desc->dtype == BIRP_DTYPE_F32;
+    memcpy(&d.vmin, &flags[BIRP_SCAN_MIN], 4);
+    memcpy(&d.vmax, &flags[BIRP_SCAN_MAX], 4);
     if (desc->dtype == BIRP_DTYPE_F32) {
         if (desc->interp == BIRP_INTERP_TRILINEAR && d.vclass != VC_NONFINITE &&
             (slots = brick_tables(nx, ny, nz, nz, tab, &morton)) != 0 && (size_t)nx + ny + nz <= 8192) {
@@ -540,7 +542,6 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
             if ((e = hipMalloc(&v->qtab, tab.size() * 4)) != hipSuccess) { rc = hip_fail(e, "hipMalloc(tables)"); goto fail_out; }
             if ((e = hipMemcpy(v->qtab, tab.data(), tab.size() * 4, hipMemcpyHostToDevice)) != hipSuccess) { rc = hip_fail(e, "tables"); goto fail_out; }
             if ((e = hipMalloc(&v->quad, quad_bytes)) != hipSuccess) { rc = hip_fail(e, "hipMalloc(quad)"); goto fail_out; }
-            if ((e = hipMemsetAsync(v->quad, 0, quad_bytes, dev->stream)) != hipSuccess) { rc = hip_fail(e, "memset(quad)"); goto fail_out; }
             d.quad = v->quad;
             d.qtab = v->qtab;
             d.quad_bytes = (unsigned)quad_bytes;
@@ -557,7 +558,6 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
         if ((e = hipMemcpy(v->otab, tab.data(), tab.size() * 4, hipMemcpyHostToDevice)) != hipSuccess) { rc = hip_fail(e, "tables"); goto fail_out; }
         if ((e = hipMalloc(&v->oct, oct_bytes)) != hipSuccess) { rc = hip_fail(e, "hipMalloc(oct)"); goto fail_out; }
         if ((e = hipMalloc(&v->bscale, slots * sizeof(float))) != hipSuccess) { rc = hip_fail(e, "hipMalloc(scale)"); goto fail_out; }
-        if ((e = hipMemsetAsync(v->oct, 0, oct_bytes, dev->stream)) != hipSuccess) { rc = hip_fail(e, "memset(oct)"); goto fail_out; }
         d.oct = v->oct;
         d.otab = v->otab;
         d.oct_bytes = (unsigned)oct_bytes;

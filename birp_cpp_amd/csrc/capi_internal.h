@@ -26,7 +26,7 @@ struct birp_device {
     hipStream_t stream = nullptr;      // render stream (default priority)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;   // per-render timing
     hipEvent_t ev_a = nullptr, ev_b = nullptr; // birp_timer_begin/end
-    void* d_counter = nullptr;         // 64 B: the upload's class-scan flags
+    void* d_counter = nullptr;         // BIRP_SCAN_WORDS: the upload's class-scan flags
     void* scratch = nullptr;           // image / point staging, grown on demand
     size_t scratch_bytes = 0;
     void* pinned = nullptr;            // pinned host staging for birp_render's image copy

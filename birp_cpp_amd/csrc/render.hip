@@ -1048,31 +1048,55 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_sample_points(DevVolume v, const
 // ------------------------------------------------------------------------------------------
 // layout builders and scans
 // ------------------------------------------------------------------------------------------
-// flags[0]: bit 0 = some value <= 0, bit 1 = some value non-finite, bit 2 = some sign bit set; flags[1], flags[2]: min and
-// max of |v| over the nonzero finite values as float bits (ordered as unsigned for positive floats).
+// The class of a cube's values, in the BIRP_SCAN_* words of flags: bit 0 = some value <= 0, bit 1 =
+// some value non-finite, bit 2 = some sign bit set; min and max of |v| over the nonzero finite values as
+// float bits (ordered as unsigned for positive floats). Bound by the read: 4 values per load, at most
+// two blocks per CU, each with one atomic per word, and the words in cache lines of their own (an
+// atomic on a contended line takes about 8 ns: three per wave on one line took 376 us for 256^3
+// values, whose read takes 13 us at 5.2 TB/s; 27 us now).
 __global__ __launch_bounds__(BIRP_BLOCK) void k_scan_class(const float* vals, size_t n, unsigned* flags) {
     unsigned f = 0, mn = 0x7F7FFFFFu, mx = 0u;
-    for (size_t idx = (size_t)blockIdx.x * BIRP_BLOCK + threadIdx.x; idx < n; idx += (size_t)gridDim.x * BIRP_BLOCK) {
-        float x = vals[idx];
+    auto look = [&](float x) {
+        const unsigned u = __float_as_uint(x) & 0x7FFFFFFFu;
         if (!(x > 0.f)) f |= 1u;
-        if (!isfinite(x)) f |= 2u;
+        if (u >= 0x7F800000u) f |= 2u;
         if (__float_as_uint(x) >> 31) f |= 4u;
-        float a = fabsf(x);
-        if (a > 0.f && isfinite(a)) {
-            unsigned u = __float_as_uint(a);
+        if (u != 0u && u < 0x7F800000u) {
             mn = min(mn, u);
             mx = max(mx, u);
         }
+    };
+    const size_t n4 = n / 4, step = (size_t)gridDim.x * BIRP_BLOCK, first = (size_t)blockIdx.x * BIRP_BLOCK + threadIdx.x;
+    for (size_t k = first; k < n4; k += step) {
+        const float4 x = reinterpret_cast<const float4*>(vals)[k];  // hipMalloc'ed: aligned
+        look(x.x);
+        look(x.y);
+        look(x.z);
+        look(x.w);
     }
+    for (size_t k = 4 * n4 + first; k < n; k += step) look(vals[k]);
+    __shared__ unsigned s_f, s_mn, s_mx;
+    if (threadIdx.x == 0) {
+        s_f = 0u;
+        s_mn = 0x7F7FFFFFu;
+        s_mx = 0u;
+    }
+    __syncthreads();
     for (int o = 32; o > 0; o >>= 1) {
         f |= (unsigned)__shfl_xor((int)f, o, 64);
         mn = min(mn, (unsigned)__shfl_xor((int)mn, o, 64));
         mx = max(mx, (unsigned)__shfl_xor((int)mx, o, 64));
     }
     if (lane_id() == 0) {
-        if (f) atomicOr(flags, f);
-        atomicMin(flags + 1, mn);
-        atomicMax(flags + 2, mx);
+        atomicOr(&s_f, f);
+        atomicMin(&s_mn, mn);
+        atomicMax(&s_mx, mx);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (s_f) atomicOr(flags + BIRP_SCAN_CLASS, s_f);
+        atomicMin(flags + BIRP_SCAN_MIN, s_mn);
+        atomicMax(flags + BIRP_SCAN_MAX, s_mx);
     }
 }
 
@@ -1089,22 +1113,53 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_check_div(DevVolume v, unsigned*
     if (f) atomicOr(bad, f);
 }
 
-// Quad records: one thread per (x, y, z).
+// The layout builders: a block makes the records of 4 bricks in a row along x. It reads their corners
+// (33 x 9 values per layer) into LDS once, coalesced, and writes each brick's 512 records in the order of
+// their addresses, 1 KB per wave and store (a thread per cell in x order wrote each 128-byte line
+// in pieces). Corners past the cube's last layer repeat it; no sample reads those records. Consecutive
+// blocks run on successive XCDs, so the blocks are numbered XCD by XCD: the cube's rows are then read
+// into one L2. Bound by the record writes: 256^3 quad records (64 MB read, 268 MB written) 149 -> 67 us,
+// the time of such a copy at 5.2 TB/s; 512^3 BF16 records 1.05 -> 0.68 ms (0.52 at that rate), the
+// brick scales within, and no clearing before.
+constexpr int kBrickRow = 4, kTileX = 8 * kBrickRow + 1;
+
+// Brick row of this block: its first brick along x, its y and z; false past the last one.
+__device__ __forceinline__ bool brick_row(const DevVolume& v, int nbz, int& bx, int& by, int& bz) {
+    const int rows = (v.nbx + kBrickRow - 1) / kBrickRow;
+    const long long b = (long long)(blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (b >= (long long)rows * v.nby * nbz) return false;
+    bx = (int)(b % rows) * kBrickRow;
+    by = (int)(b / rows) % v.nby;
+    bz = (int)(b / rows / v.nby);
+    return true;
+}
+
+template <int LAYERS>
+__device__ __forceinline__ void load_brick_row(const DevVolume& v, int bx, int by, int bz, float* s) {
+    for (int t = threadIdx.x; t < kTileX * 9 * LAYERS; t += BIRP_BLOCK) {
+        const int x = min(bx * 8 + t % kTileX, v.nx - 1), y = min(by * 8 + t / kTileX % 9, v.ny - 1), z = min(bz * 8 + t / (kTileX * 9), v.nz - 1);
+        s[t] = v.linear[((size_t)z * v.ny + y) * v.nx + x];
+    }
+    __syncthreads();
+}
+
+// Cell r (0..511, Morton order) of brick w of the row: its lowest corner in the LDS tile.
+__device__ __forceinline__ int brick_cell(int w, int r) {
+    const int lx = (r & 1) | (r >> 2 & 2) | (r >> 4 & 4), ly = (r >> 1 & 1) | (r >> 3 & 2) | (r >> 5 & 4), lz = (r >> 2 & 1) | (r >> 4 & 2) | (r >> 6 & 4);
+    return (lz * 9 + ly) * kTileX + w * 8 + lx;
+}
+
 __global__ __launch_bounds__(BIRP_BLOCK) void k_build_quad(DevVolume v, unsigned char* quad) {
-    const unsigned* tx = v.qtab;
-    const unsigned* ty = v.qtab + v.nx;
-    const unsigned* tz = v.qtab + v.nx + v.ny;
-    size_t cx = v.nx - 1, cy = v.ny - 1;
-    size_t total = cx * cy * (size_t)v.nz;
-    for (size_t r = (size_t)blockIdx.x * BIRP_BLOCK + threadIdx.x; r < total; r += (size_t)gridDim.x * BIRP_BLOCK) {
-        int x = (int)(r % cx);
-        int y = (int)((r / cx) % cy);
-        int z = (int)(r / (cx * cy));
-        const float* L = v.linear;
-        size_t base = ((size_t)z * v.ny + y) * v.nx + x;
-        float4 q = make_float4(L[base], L[base + 1], L[base + v.nx], L[base + v.nx + 1]);
-        unsigned off = tx[x] + ty[y] + tz[z];
-        *(float4*)(quad + off) = q;
+    __shared__ float s[kTileX * 9 * 8];
+    int bx, by, bz;
+    if (!brick_row(v, (v.nz + 7) / 8, bx, by, bz)) return;
+    load_brick_row<8>(v, bx, by, bz, s);
+    const int w = threadIdx.x >> 6;  // one wave per brick
+    if (bx + w >= v.nbx) return;
+    const unsigned base = v.qtab[(bx + w) * 8] + v.qtab[v.nx + by * 8] + v.qtab[v.nx + v.ny + bz * 8];
+    for (int r = lane_id(); r < 512; r += 64) {
+        const float* c = s + brick_cell(w, r);
+        *(float4*)(quad + base + r * 16u) = make_float4(c[0], c[1], c[kTileX], c[kTileX + 1]);
     }
 }
 
@@ -1117,58 +1172,38 @@ __device__ __forceinline__ unsigned short f32_to_f16_bits(float x) {
     return *reinterpret_cast<unsigned short*>(&h);
 }
 
-// Per-brick power-of-two scale for F16: max|v| over the brick's corners maps to < 2^15. With
+// F16 records hold v / scale, a power of two per brick: max|v| over the brick's corners maps to < 2^15. With
 // v.f16_uniform every brick gets the volume's scale v.f16_scale instead.
-__global__ __launch_bounds__(BIRP_BLOCK) void k_brick_scale(DevVolume v, float* bscale) {
-    int brick = blockIdx.x;
-    if (v.f16_uniform) {
-        if (threadIdx.x == 0) {
-            int bx = brick % v.nbx, by = (brick / v.nbx) % v.nby, bz = brick / (v.nbx * v.nby);
-            const unsigned* t = v.otab;
-            bscale[(t[bx * 8] + t[v.nx + by * 8] + t[v.nx + v.ny + bz * 8]) >> 13] = v.f16_scale;
-        }
-        return;
-    }
-    int bx = brick % v.nbx, by = (brick / v.nbx) % v.nby, bz = brick / (v.nbx * v.nby);
-    float mx = 0.f;
-    for (int t = threadIdx.x; t < 729; t += BIRP_BLOCK) {
-        int lx = t % 9, ly = (t / 9) % 9, lz = t / 81;
-        int x = bx * 8 + lx, y = by * 8 + ly, z = bz * 8 + lz;
-        if (x < v.nx && y < v.ny && z < v.nz) mx = fmaxf(mx, fabsf(v.linear[((size_t)z * v.ny + y) * v.nx + x]));
-    }
-    __shared__ float red[BIRP_BLOCK / 64];
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    if (lane_id() == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-        float s = 1.f;
-        if (m > 0.f && isfinite(m)) {
-            int e;
-            frexpf(m, &e);           // m = f * 2^e, f in [0.5, 1)
-            s = ldexpf(1.f, e - 15); // m / s < 2^15
-        }
-        const unsigned* t = v.otab;
-        unsigned code = (t[bx * 8] + t[v.nx + by * 8] + t[v.nx + v.ny + bz * 8]) >> 13;
-        bscale[code] = s;
-    }
-}
-
 template <bool F16>
-__global__ __launch_bounds__(BIRP_BLOCK) void k_build_oct(DevVolume v, unsigned char* oct, const float* bscale) {
-    const unsigned* tx = v.otab;
-    const unsigned* ty = v.otab + v.nx;
-    const unsigned* tz = v.otab + v.nx + v.ny;
-    size_t cx = v.nx - 1, cy = v.ny - 1, cz = v.nz - 1;
-    size_t total = cx * cy * cz;
-    for (size_t r = (size_t)blockIdx.x * BIRP_BLOCK + threadIdx.x; r < total; r += (size_t)gridDim.x * BIRP_BLOCK) {
-        int x = (int)(r % cx), y = (int)((r / cx) % cy), z = (int)(r / (cx * cy));
-        const float* L = v.linear;
-        size_t sy = v.nx, sz = (size_t)v.nx * v.ny;
-        size_t b0 = (size_t)z * sz + (size_t)y * sy + x;
-        float c[8] = {L[b0], L[b0 + 1], L[b0 + sy], L[b0 + sy + 1], L[b0 + sz], L[b0 + sz + 1], L[b0 + sz + sy], L[b0 + sz + sy + 1]};
-        unsigned off = tx[x] + ty[y] + tz[z];
-        float inv = F16 ? 1.f / bscale[off >> 13] : 1.f;  // power of two: exact
+__global__ __launch_bounds__(BIRP_BLOCK) void k_build_oct(DevVolume v, unsigned char* oct, float* bscale) {
+    __shared__ float s[kTileX * 9 * 9];
+    int bx, by, bz;
+    if (!brick_row(v, v.nbz, bx, by, bz)) return;
+    load_brick_row<9>(v, bx, by, bz, s);
+    const int w = threadIdx.x >> 6;  // one wave per brick
+    if (bx + w >= v.nbx) return;
+    const unsigned base = v.otab[(bx + w) * 8] + v.otab[v.nx + by * 8] + v.otab[v.nx + v.ny + bz * 8];
+    float inv = 1.f;
+    if constexpr (F16) {
+        float scale = v.f16_scale;
+        if (!v.f16_uniform) {
+            float m = 0.f;
+            for (int t = lane_id(); t < 729; t += 64) m = fmaxf(m, fabsf(s[t / 9 * kTileX + w * 8 + t % 9]));
+            for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+            scale = 1.f;
+            if (m > 0.f && isfinite(m)) {
+                int e;
+                frexpf(m, &e);               // m = f * 2^e, f in [0.5, 1)
+                scale = ldexpf(1.f, e - 15); // m / scale < 2^15
+            }
+        }
+        if (lane_id() == 0) bscale[base >> 13] = scale;
+        inv = 1.f / scale;  // power of two: exact
+    }
+    for (int r = lane_id(); r < 512; r += 64) {
+        const float* c0 = s + brick_cell(w, r);
+        const float* c1 = c0 + 9 * kTileX;
+        const float c[8] = {c0[0], c0[1], c0[kTileX], c0[kTileX + 1], c1[0], c1[1], c1[kTileX], c1[kTileX + 1]};
         unsigned short h[8];
 #pragma unroll
         for (int q = 0; q < 8; q++) h[q] = F16 ? f32_to_f16_bits(c[q] * inv) : f32_to_bf16_bits(c[q]);
@@ -1177,7 +1212,7 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_build_oct(DevVolume v, unsigned 
         o.y = (unsigned)h[2] | ((unsigned)h[3] << 16);
         o.z = (unsigned)h[4] | ((unsigned)h[5] << 16);
         o.w = (unsigned)h[6] | ((unsigned)h[7] << 16);
-        *(uint4*)(oct + off) = o;
+        *(uint4*)(oct + base + r * 16u) = o;
     }
 }
 
@@ -1873,9 +1908,7 @@ int launch_sample_points(const DevVolume& v, const float* xyz, long long n, floa
 }
 
 int launch_scan_class(const float* values, size_t n, unsigned* flags_dev, void* stream) {
-    size_t blocks = (n + BIRP_BLOCK - 1) / BIRP_BLOCK;
-    if (blocks > 4096) blocks = 4096;
-    if (blocks == 0) blocks = 1;
+    const size_t blocks = std::min<size_t>((n / 4 + BIRP_BLOCK) / BIRP_BLOCK, 512);
     hipLaunchKernelGGL(k_scan_class, dim3((unsigned)blocks), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, values, n, flags_dev);
     return hip_status(hipGetLastError());
 }
@@ -1885,28 +1918,23 @@ int launch_check_div(const DevVolume& v, unsigned* bad_dev, void* stream) {
     return hip_status(hipGetLastError());
 }
 
+// blocks of a layout build: one per 4 bricks along x, a multiple of 8
+static int brick_row_grid(const DevVolume& v, int nbz) {
+    const long long rows = (long long)((v.nbx + kBrickRow - 1) / kBrickRow) * v.nby * nbz;
+    return (int)((rows + 7) / 8 * 8);
+}
+
 int launch_build_quad(const DevVolume& v, void* quad, void* stream) {
-    size_t total = (size_t)(v.nx - 1) * (v.ny - 1) * v.nz;
-    size_t blocks = (total + BIRP_BLOCK - 1) / BIRP_BLOCK;
-    if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(k_build_quad, dim3((unsigned)blocks), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, v, (unsigned char*)quad);
+    hipLaunchKernelGGL(k_build_quad, dim3(brick_row_grid(v, (v.nz + 7) / 8)), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, v, (unsigned char*)quad);
     return hip_status(hipGetLastError());
 }
 
 int launch_build_oct(const DevVolume& v, void* oct, float* bscale, void* stream) {
-    hipStream_t st = (hipStream_t)stream;
-    int nb = v.nbx * v.nby * v.nbz;
-    if (v.dtype == BIRP_DTYPE_F16) {
-        hipLaunchKernelGGL(k_brick_scale, dim3(nb), dim3(BIRP_BLOCK), 0, st, v, bscale);
-        if (hipGetLastError() != hipSuccess) return BIRP_ERR_DEVICE;
-    }
-    size_t total = (size_t)(v.nx - 1) * (v.ny - 1) * (v.nz - 1);
-    size_t blocks = (total + BIRP_BLOCK - 1) / BIRP_BLOCK;
-    if (blocks > 65536) blocks = 65536;
+    const dim3 grid(brick_row_grid(v, v.nbz));
     if (v.dtype == BIRP_DTYPE_F16)
-        hipLaunchKernelGGL((k_build_oct<true>), dim3((unsigned)blocks), dim3(BIRP_BLOCK), 0, st, v, (unsigned char*)oct, bscale);
+        hipLaunchKernelGGL((k_build_oct<true>), grid, dim3(BIRP_BLOCK), 0, (hipStream_t)stream, v, (unsigned char*)oct, bscale);
     else
-        hipLaunchKernelGGL((k_build_oct<false>), dim3((unsigned)blocks), dim3(BIRP_BLOCK), 0, st, v, (unsigned char*)oct, bscale);
+        hipLaunchKernelGGL((k_build_oct<false>), grid, dim3(BIRP_BLOCK), 0, (hipStream_t)stream, v, (unsigned char*)oct, bscale);
     return hip_status(hipGetLastError());
 }
 
