@@ -49,6 +49,16 @@ struct CmemParams {
     float cos_theta_n, sin_theta_n, cos_theta_s, sin_theta_s;
 };
 
+// Zone bounds of a CMEM model (k_cmem_zones): its surfaces depend on a point's direction only, through
+// ct = x / r and cp = y / |(y, z)|. The table has a cell per 1/128 of ct and 1/64 of cp, [ct][cp],
+// each four radii {inside, past_mp, sheath, past_bs}: every point of the cell's directions with
+// r < inside is inside the magnetopause zone (value 0), with r > past_mp outside it, and beyond that with
+// r < sheath in the sheath, with r > past_bs outside the bow shock zone. A point for which none holds
+// needs the surfaces themselves.
+#define BIRP_ZONE_CT 256
+#define BIRP_ZONE_CP 128
+#define BIRP_ZONE_BYTES (BIRP_ZONE_CT * BIRP_ZONE_CP * 16)
+
 struct DevVolume {
     int kind;    // SpaceKind
     int nx, ny, nz;
@@ -77,6 +87,7 @@ struct DevVolume {
     int f16_uniform;      // F16 records all share one power-of-two scale (f16_scale)
     float f16_scale;      // that scale: records hold v / f16_scale
     CmemParams cmem;
+    const void* zones;  // the model's zone bounds, BIRP_ZONE_BYTES
 };
 
 // Per-render constants of the exact path, computed on the host in the reference's float order.
@@ -193,6 +204,7 @@ int launch_scan_class(const float* values, size_t n, unsigned* flags_dev, void* 
 // Checks birp_div_fma2 for the volume's spacings over every significand: ORs bit `axis` into *bad_dev for
 // an axis with a mismatch.
 int launch_check_div(const DevVolume& v, unsigned* bad_dev, void* stream);
+int launch_cmem_zones(const CmemParams& m, void* zones, void* stream);
 int launch_build_quad(const DevVolume& v, void* quad, void* stream);
 int launch_build_oct(const DevVolume& v, void* oct, float* bscale, void* stream);
 

@@ -189,7 +189,7 @@ bool take_injected_failure(birp_device* dev) {
 // BIRP_EXACT_PIPE (samples in flight per lane in the positive-cube loop: 1..4) and
 // BIRP_EXACT_LAYOUT ("linear" reads the [z][y][x] copy instead of the quad bricks).
 // By default a single exact render takes 16 lanes per ray for images of at most 8,000 rays, 8 for
-// at most 20,000, 4 for CMEM and for images of at most 60,000 rays, and 2 above: a small image's
+// at most 20,000, 4 for images of at most 60,000 rays, and 2 above (CMEM: 16, 8 and 4, below): a small image's
 // few waves are bound by the chain of each ray's samples, which more lanes cut (ms per render over
 // 6 orbit poses at n = 800 with 4 samples in flight, 2 / 4 / 8 lanes: 144x84 0.032 / 0.020 / 0.016,
 // 288x168 0.038 / 0.027 / 0.030, 576x336 0.071 / 0.075 / 0.089; 8 / 16 lanes at n = 800: 72x42
@@ -202,8 +202,10 @@ int default_exact_lanes(bool cmem, int W, int H) {
         return (v == 1 || v == 2 || v == 4 || v == 8 || v == 16) ? v : 0;
     }();
     if (lanes) return lanes;
-    if (cmem) return 4;
     const long long rays = (long long)W * H;
+    // us with 4 / 8 / 16 lanes: 72x42 n = 200 168 / 41 / 27, 144x84 n = 800 196 / 123 / 84, 200x120 n = 500
+    // 142 / 99 / 100, 288x168 n = 800 247 / 218 / 224, 400x240 n = 400 192 / 210 / 258
+    if (cmem) return rays <= 20000 ? 16 : (rays <= 60000 ? 8 : 4);
     return rays <= 8000 ? 16 : (rays <= 20000 ? 8 : (rays <= 60000 ? 4 : 2));
 }
 // Single positive-cube renders keep 4 samples in flight per lane: their waves are few and wait
@@ -388,12 +390,14 @@ static void free_volume_buffers(birp_volume* v) {
     if (v->bscale) (void)hipFree(v->bscale);
     if (v->qtab) (void)hipFree(v->qtab);
     if (v->otab) (void)hipFree(v->otab);
+    if (v->zones) (void)hipFree(v->zones);
     v->linear = nullptr;
     v->quad = nullptr;
     v->oct = nullptr;
     v->bscale = nullptr;
     v->qtab = nullptr;
     v->otab = nullptr;
+    v->zones = nullptr;
 }
 
 namespace birp {
@@ -614,7 +618,17 @@ extern "C" int birp_cmem_create(birp_device* dev, const birp_cmem_state* s, birp
     c.sin_theta_s = std::sin(c.theta_s);
     v->dv.dtype = BIRP_DTYPE_F32;
     v->dv.interp = BIRP_INTERP_TRILINEAR;
-    v->bytes = 0;
+    (void)hipSetDevice(dev->ordinal);
+    hipError_t e = hipMalloc(&v->zones, BIRP_ZONE_BYTES);
+    int rc = e == hipSuccess ? launch_cmem_zones(c, v->zones, dev->stream) : hip_fail(e, "hipMalloc(zone bounds)");
+    if (rc == BIRP_OK && (e = hipStreamSynchronize(dev->stream)) != hipSuccess) rc = hip_fail(e, "zone bounds");
+    if (rc) {
+        free_volume_buffers(v);
+        delete v;
+        return rc;
+    }
+    v->dv.zones = v->zones;
+    v->bytes = BIRP_ZONE_BYTES;
     *out = v;
     return BIRP_OK;
 }

@@ -62,6 +62,7 @@ struct birp_volume {
     float* bscale = nullptr;
     unsigned* qtab = nullptr;
     unsigned* otab = nullptr;
+    void* zones = nullptr;  // CMEM: the zone bounds
     bool morton = false;
     size_t bytes = 0;
 };

@@ -280,6 +280,14 @@ __device__ __forceinline__ float scale_pos(float vw) {
     return s;
 }
 
+// The scale chain for any value: the FMA form in its range and for +0, else the tested or literal chain.
+__device__ __forceinline__ float scale_any(float vw) {
+    float s = birp_scale_fma2(vw);
+    const float a = fabsf(vw);
+    if (__builtin_expect(!(a >= 0x1p-100f && a <= 0x1p110f) && __float_as_uint(vw) != 0u, 0)) s = birp_scale_sample(vw);
+    return s;
+}
+
 // acc += the S sub-lane samples of this ray, in sub-lane (= k) order. Exact on sub-lane 0 of
 // the ray (the lane that stores the pixel); the other sub-lanes' sums are not used. With 8 lanes
 // per ray the ray spans two 16-lane rows: sub-lanes 4..7 are read from the next row's copy.
@@ -352,6 +360,16 @@ __device__ __forceinline__ float acos_to_float(double c) {
     return 3.14159265358979323846f - 2.0f * asinf(sqrtf((float)((1.0 + c) * 0.5)));
 }
 
+// Emissivity outside the bow shock (Cmem.cpp:172-175) and in the sheath (:148-152).
+__device__ __forceinline__ float cmem_outer(const CmemParams& m, float r) {
+    double sd = r / 10;
+    return (float)(m.A2 * (1 / (sd * sd * sd)));
+}
+__device__ __forceinline__ float cmem_inner(const CmemParams& m, float r, float theta, float st) {
+    float half_t = theta / 2;
+    return m.A1 * (expf(-m.B * (half_t * half_t * half_t * half_t))) * powf(r / 10, (-m.alpha - (m.beta * (st * st))));
+}
+
 __device__ __forceinline__ float cmem_sample(const CmemParams& m, float x, float y, float z) {
     float r = sqrtf(x * x + y * y + z * z);
     const float ryz = sqrtf(y * y + z * z);
@@ -386,18 +404,131 @@ __device__ __forceinline__ float cmem_sample(const CmemParams& m, float x, float
     const bool z_mp = r >= radius_mp - h && r <= radius_mp + h;
     const bool z_sheath = !z_mp && r > radius_mp + h && r < radius_bs - h;
     const bool z_bs = !z_mp && !z_sheath && r >= radius_bs - h && r <= radius_bs + h;
-    double sd = r / 10;
-    if (!(z_mp || z_sheath || z_bs)) return (float)(m.A2 * (1 / (sd * sd * sd)));
-    float half_t = theta / 2;
-    float inner = m.A1 * (expf(-m.B * (half_t * half_t * half_t * half_t))) * powf(r / 10, (-m.alpha - (m.beta * (st * st))));
+    if (!(z_mp || z_sheath || z_bs)) return cmem_outer(m, r);
+    float inner = cmem_inner(m, r, theta, st);
     if (z_mp) {
         float norm = (r - (radius_mp - h)) / (radius_mp + h);
         return lerp_general(0.f, inner, norm);
     }
     if (z_sheath) return inner;
     float norm = (r - (radius_bs - h)) / (radius_bs + h);
-    float b2 = (float)(m.A2 * (1 / (sd * sd * sd)));
-    return lerp_general(inner, b2, norm);
+    return lerp_general(inner, cmem_outer(m, r), norm);
+}
+
+// ------------------------------------------------------------------------------------------
+// CMEM zone bounds (birp_internal.h): interval arithmetic in double over each cell's directions
+// ------------------------------------------------------------------------------------------
+struct Range {
+    double lo, hi;
+};
+__device__ __forceinline__ Range operator+(Range a, Range b) { return {a.lo + b.lo, a.hi + b.hi}; }
+__device__ __forceinline__ Range operator*(Range a, Range b) {
+    const double p = a.lo * b.lo, q = a.lo * b.hi, r = a.hi * b.lo, s = a.hi * b.hi;
+    return {fmin(fmin(p, q), fmin(r, s)), fmax(fmax(p, q), fmax(r, s))};
+}
+__device__ __forceinline__ Range operator*(double k, Range a) { return Range{k, k} * a; }
+__device__ __forceinline__ Range range_exp(Range a) { return {exp(a.lo), exp(a.hi)}; }
+// x^e for x >= 0: monotone in x (lo = 0 with e < 0 gives inf)
+__device__ __forceinline__ Range range_pow(Range x, double e) {
+    const double a = pow(x.lo, e), b = pow(x.hi, e);
+    return {fmin(a, b), fmax(a, b)};
+}
+
+// Both arithmetics (cmem_sample's and cmem_fast's) must find the zone that the bounds name, so the bounds are
+// wider than the ranges by more than their rounding: the cell's directions by 1e-5 (a direction's ct
+// and cp are within 1e-6), the arc cosines' arguments by 2e-6, the radii by 1e-4 RE + 3e-5 of their terms
+// (FP32 powers and exponentials are within 1e-5). Where the model leaves the reals or is too steep for that
+// the cell bounds nothing: at the cusps, whose arc cosine's argument rounds past 1 in the reference
+// (NaN), and in the last cells of the tail, where 2 / (1 + ct) diverges and a power's base may be negative.
+__global__ __launch_bounds__(BIRP_BLOCK) void k_cmem_zones(CmemParams m, float4* zones) {
+    const int cell = blockIdx.x * BIRP_BLOCK + threadIdx.x;
+    if (cell >= BIRP_ZONE_CT * BIRP_ZONE_CP) return;
+    const int iu = cell / BIRP_ZONE_CP, iv = cell % BIRP_ZONE_CP;
+    const double wide = 1e-5;
+    const Range ct{fmax(-1.0, iu * (2.0 / BIRP_ZONE_CT) - 1 - wide), fmin(1.0, (iu + 1) * (2.0 / BIRP_ZONE_CT) - 1 + wide)};
+    const Range cp{fmax(-1.0, iv * (2.0 / BIRP_ZONE_CP) - 1 - wide), fmin(1.0, (iv + 1) * (2.0 / BIRP_ZONE_CP) - 1 + wide)};
+    auto sine = [](Range c) {  // sqrt(1 - c^2)
+        const double a = sqrt(fmax(0.0, 1 - c.lo * c.lo)), b = sqrt(fmax(0.0, 1 - c.hi * c.hi));
+        return Range{fmin(a, b), c.lo <= 0 && c.hi >= 0 ? 1.0 : fmax(a, b)};
+    };
+    const Range theta{acos(ct.hi), acos(ct.lo)}, st = sine(ct), sp = sine(cp);
+    bool known = ct.lo > -1 + 1e-3;
+    // an angle to a cusp, in [0, pi]
+    auto cusp_angle = [&](double c, double s) {
+        const Range a = c * ct + s * (st * sp);
+        const double near = 2e-3;  // of the cusp or the point opposite
+        if (cp.lo <= near && cp.hi >= -near && ((ct.lo <= c + near && ct.hi >= c - near) || (ct.lo <= -c + near && ct.hi >= -c - near)))
+            known = false;
+        return Range{acos(fmin(1.0, a.hi + 2e-6)), acos(fmax(-1.0, a.lo - 2e-6))};
+    };
+    const Range north = cusp_angle(m.cos_theta_n, m.sin_theta_n), south = cusp_angle(m.cos_theta_s, -m.sin_theta_s);
+    const Range grow{1 - exp(-theta.lo), 1 - exp(-theta.hi)}, half{cos(theta.hi / 2), cos(theta.lo / 2)};
+    const Range base = half + (2.0 * m.a5) * (st * ct * grow);
+    known = known && base.lo > 1e-4;
+    const Range power = (double)m.p1 * (Range{m.beta_c[0], m.beta_c[0]} + (double)m.beta_c[1] * cp + (double)m.beta_c[3] * (sp * sp));
+    const Range f = range_exp(power * Range{log(fmax(base.lo, 1e-300)), log(fmax(base.hi, 1e-300))});
+    const Range dip_n = range_exp(((double)m.p3 * m.dn) * range_pow(north, m.a21)), dip_s = range_exp(((double)m.p3 * m.ds) * range_pow(south, m.a21));
+    const Range far = ((double)m.p0 * m.r0_lin) * f, q = ((double)m.p2 * m.charlie) * (dip_n + dip_s);
+    const Range mp = far + q;
+    const double mp_wide = 1e-4 + 3e-5 * (fmax(fabs(far.lo), fabs(far.hi)) + fmax(fabs(q.lo), fabs(q.hi)));
+    const Range flare{2 / (1 + ct.hi), 2 / (1 + ct.lo)};
+    const Range ry = (double)m.bs * range_pow(flare, m.ay_bs), rz = (double)m.bs * range_pow(flare, m.az_bs);
+    known = known && m.bs > 0;
+    Range bs = ry;  // with one exponent: ry / sqrt(cos^2 + sin^2)
+    if (m.az_bs != m.ay_bs) {
+        const Range u = rz * cp, w = ry * sp, n = ry * rz;
+        const double lo = (cp.lo <= 0 && cp.hi >= 0 ? 0.0 : fmin(u.lo * u.lo, u.hi * u.hi)) + w.lo * w.lo;
+        bs = Range{n.lo / sqrt(fmax(u.lo * u.lo, u.hi * u.hi) + w.hi * w.hi), n.hi / sqrt(lo)};
+    }
+    const double bs_wide = 1e-4 + 3e-5 * fmax(fabs(bs.lo), fabs(bs.hi)), h = 0.025;
+    float4 t = make_float4((float)(mp.lo - h - mp_wide), (float)(mp.hi + h + mp_wide), (float)(bs.lo - h - bs_wide), (float)(bs.hi + h + bs_wide));
+    known = known && isfinite(t.x) && isfinite(t.y) && isfinite(t.z) && isfinite(t.w);
+    if (!known) t = make_float4(-INFINITY, INFINITY, -INFINITY, INFINITY);
+    zones[cell] = t;
+}
+
+// What the bounds say of a point. ZONE_EDGE: nothing; also for points on x = 0 or y = 0, where the
+// reference takes an angle of 0 (Cmem.cpp:224-246).
+enum Zone { ZONE_INSIDE, ZONE_SHEATH, ZONE_OUTER, ZONE_EDGE };
+struct ZoneQuery {
+    float4 t;
+    float r;
+    bool axis;
+};
+__device__ __forceinline__ ZoneQuery zone_fetch(__amdgpu_buffer_rsrc_t rs, float x, float y, float z) {
+    ZoneQuery q;
+    const float yz2 = __builtin_fmaf(y, y, z * z), r2 = __builtin_fmaf(x, x, yz2), ir = __builtin_amdgcn_rsqf(r2);
+    const float u = __builtin_fmaf(x * ir, 0.5f * BIRP_ZONE_CT, 0.5f * BIRP_ZONE_CT);
+    const float v = __builtin_fmaf(y * __builtin_amdgcn_rsqf(yz2), 0.5f * BIRP_ZONE_CP, 0.5f * BIRP_ZONE_CP);
+    const unsigned iu = (unsigned)__builtin_amdgcn_fmed3f(u, 0.0f, BIRP_ZONE_CT - 1.0f), iv = (unsigned)__builtin_amdgcn_fmed3f(v, 0.0f, BIRP_ZONE_CP - 1.0f);
+    q.t = load16(rs, (iu * BIRP_ZONE_CP + iv) * 16u);
+    q.r = r2 * ir;
+    q.axis = !(fabsf(x * y) > 0.0f);
+    return q;
+}
+__device__ __forceinline__ Zone zone_of(const ZoneQuery& q) {
+    if (q.axis) return ZONE_EDGE;
+    if (q.r < q.t.x) return ZONE_INSIDE;
+    if (!(q.r > q.t.y)) return ZONE_EDGE;
+    return q.r < q.t.z ? ZONE_SHEATH : q.r > q.t.w ? ZONE_OUTER : ZONE_EDGE;
+}
+
+// cmem_sample with its surfaces left out where the bounds name the point's zone: the same value, bit for bit.
+// The surfaces are the model's cost (about 900 of 1,100 VALU instructions per sample in libm calls) and a
+// zone is all that most samples need of them: a query is 35 instructions and one 16-byte load. 576x336 x
+// 800: 3.45 -> 0.65 ms; fast form 0.662 -> 0.264 ms. A table of half the cells per axis gives 0.70 and
+// 0.270 ms, of twice 0.64 and 0.262 (2 MB): what is left is the sheath's powf and the outer zone's
+// FP64 cube, not the cells on a surface.
+__device__ __forceinline__ float cmem_sample_zoned(const CmemParams& m, const ZoneQuery& q, float x, float y, float z) {
+    const Zone zone = zone_of(q);
+    float val = 0.f;
+    if (zone == ZONE_EDGE) val = cmem_sample(m, x, y, z);
+    if (zone == ZONE_SHEATH || zone == ZONE_OUTER) {
+        const float r = sqrtf(x * x + y * y + z * z);
+        if (zone == ZONE_OUTER) val = cmem_outer(m, r);
+        else val = cmem_inner(m, r, acosf(x / r), sqrtf(y * y + z * z) / r);
+    }
+    return val;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -628,19 +759,8 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
     // gathers its S samples and tests them in k order on sub-lane 0 (the other sub-lanes' sums and stops
     // are not used).
     bool alive = true, quiet = true;
-    for (int kb = 0; !NN && kb < trips; kb += S) {
-        const float t = *(const float*)((const char*)s_t + min(t_first + (unsigned)kb * 4u, t_last));
+    auto add_trip = [&](float s, int kb) {
         const bool act = kb < lim;
-        float val;
-        if constexpr (MODE == SM_CMEM) {
-            val = cmem_sample(v.cmem, dx * t + px, dy * t + py, dz * t + pz);
-        } else {
-            ExactIdx r = exact_index<DIV_GUARD>(v, dx, dy, dz, px, py, pz, t);
-            if constexpr (MODE == SM_QUAD_GEN) val = quad_lerp<LERP_FINITE>(quad_fetch(qc, r.xd, r.yd, r.zd));
-            else if constexpr (MODE == SM_LIN_TRI) val = sample_linear_tri(v, r);
-            else val = sample_linear_nearest(v, r);
-        }
-        const float s = birp_scale_sample(val * w);  // Camera.cpp:201
         quiet = quiet && __ballot(act && s < 0) == 0ull;
         if (quiet) {
             acc = add_in_order<S>(acc, act ? s : -0.0f);
@@ -655,6 +775,23 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
                 alive = alive && !stop;
             }
         }
+    };
+    if constexpr (MODE == SM_CMEM) {
+        const __amdgpu_buffer_rsrc_t zones = make_rsrc(v.zones, BIRP_ZONE_BYTES);
+        for (int kb = 0; kb < trips; kb += S) {
+            const float t = *(const float*)((const char*)s_t + min(t_first + (unsigned)kb * 4u, t_last));
+            const float x = dx * t + px, y = dy * t + py, z = dz * t + pz;
+            add_trip(scale_any(cmem_sample_zoned(v.cmem, zone_fetch(zones, x, y, z), x, y, z) * w), kb);  // Camera.cpp:201
+        }
+    }
+    for (int kb = 0; !NN && MODE != SM_CMEM && kb < trips; kb += S) {
+        const float t = *(const float*)((const char*)s_t + min(t_first + (unsigned)kb * 4u, t_last));
+        const ExactIdx r = exact_index<DIV_GUARD>(v, dx, dy, dz, px, py, pz, t);
+        float val;
+        if constexpr (MODE == SM_QUAD_GEN) val = quad_lerp<LERP_FINITE>(quad_fetch(qc, r.xd, r.yd, r.zd));
+        else if constexpr (MODE == SM_LIN_TRI) val = sample_linear_tri(v, r);
+        else val = sample_linear_nearest(v, r);
+        add_trip(scale_any(val * w), kb);  // Camera.cpp:201
     }
     if (valid && sub == 0) ev.out[(size_t)j * ev.W + i] = acc;
     if (ev.counter || ev.wave_counts) {
@@ -1300,6 +1437,12 @@ __device__ __forceinline__ float acos_fast(float x) {
 __device__ __forceinline__ float pow_fast(float b, float e) { return __builtin_amdgcn_exp2f(e * __builtin_amdgcn_logf(b)); }
 __device__ __forceinline__ float exp_fast(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896f); }
 
+__device__ __forceinline__ float cmem_fast_inner(const CmemParams& m, float sd, float theta, float st) {
+    const float ht = 0.5f * theta, ht2 = ht * ht;
+    return m.A1 * exp_fast(-m.B * (ht2 * ht2)) * pow_fast(sd, -m.alpha - m.beta * (st * st));
+}
+__device__ __forceinline__ float cmem_fast_outer(const CmemParams& m, float sd) { return m.A2 * __builtin_amdgcn_rcpf(sd * sd * sd); }
+
 __device__ __forceinline__ float cmem_fast(const CmemParams& m, float x, float y, float z) {
     const float ryz2 = y * y + z * z;
     const float r = __builtin_amdgcn_sqrtf(__builtin_fmaf(x, x, ryz2)), ryz = __builtin_amdgcn_sqrtf(ryz2);
@@ -1331,13 +1474,30 @@ __device__ __forceinline__ float cmem_fast(const CmemParams& m, float x, float y
     const bool z_sheath = !z_mp && r < rbs - h;
     const bool z_bs = !z_mp && !z_sheath && r >= rbs - h && r <= rbs + h;
     const float sd = 0.1f * r;
-    const float outer = m.A2 * __builtin_amdgcn_rcpf(sd * sd * sd);
+    const float outer = cmem_fast_outer(m, sd);
     if (!(z_mp || z_sheath || z_bs)) return outer;
-    const float ht = 0.5f * theta, ht2 = ht * ht;
-    const float inner = m.A1 * exp_fast(-m.B * (ht2 * ht2)) * pow_fast(sd, -m.alpha - m.beta * (st * st));
+    const float inner = cmem_fast_inner(m, sd, theta, st);
     if (z_mp) return ((r - (rmp - h)) * __builtin_amdgcn_rcpf(rmp + h)) * inner;  // lerp(0, inner, t)
     if (z_sheath) return inner;
     return __builtin_fmaf((r - (rbs - h)) * __builtin_amdgcn_rcpf(rbs + h), outer - inner, inner);
+}
+
+// cmem_fast with its surfaces left out where the bounds name the point's zone.
+__device__ __forceinline__ float cmem_fast_zoned(const CmemParams& m, const ZoneQuery& q, float x, float y, float z) {
+    const Zone zone = zone_of(q);
+    float val = 0.f;
+    if (zone == ZONE_EDGE) val = cmem_fast(m, x, y, z);
+    if (zone == ZONE_SHEATH || zone == ZONE_OUTER) {
+        const float ryz2 = y * y + z * z;
+        const float r = __builtin_amdgcn_sqrtf(__builtin_fmaf(x, x, ryz2)), sd = 0.1f * r;
+        if (zone == ZONE_OUTER) {
+            val = cmem_fast_outer(m, sd);
+        } else {
+            const float ir = __builtin_amdgcn_rcpf(r);
+            val = cmem_fast_inner(m, sd, acos_fast(x * ir), __builtin_amdgcn_sqrtf(ryz2) * ir);
+        }
+    }
+    return val;
 }
 
 // Keeps the FP32 march x(j) = RN(j d + i0), j = 0 .. last, inside [0, hi]. x(j) is one rounding of
@@ -1409,7 +1569,7 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
     constexpr bool SIGNED = CMEM || (KV & BIRP_KDT_SIGNED) != 0;
     const int tw = L.tw, th = L.th, ray = L.ray, ti = L.ti, tj = L.tj, sub = L.sub, sub_step = L.sub_step;
     const float K = (float)BIRP_SCALE_FOLDED;
-    const __amdgpu_buffer_rsrc_t rs = (DT == BIRP_DTYPE_F32) ? make_rsrc(V.quad, V.quad_bytes) : make_rsrc(V.oct, V.oct_bytes);
+    const __amdgpu_buffer_rsrc_t rs = CMEM ? make_rsrc(V.zones, BIRP_ZONE_BYTES) : (DT == BIRP_DTYPE_F32) ? make_rsrc(V.quad, V.quad_bytes) : make_rsrc(V.oct, V.oct_bytes);
     const int tx = tile % P.tiles_x, ty = tile / P.tiles_x;
     const int i = tx * tw + ti;
     const int j = ty * th + tj;
@@ -1500,7 +1660,7 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
             const float yd = __builtin_fmaf(fj, diy, iy0);
             const float zd = __builtin_fmaf(fj, diz, iz0);
             float x;
-            if constexpr (CMEM) x = cmem_fast(V.cmem, xd, yd, zd);
+            if constexpr (CMEM) x = cmem_fast_zoned(V.cmem, zone_fetch(rs, xd, yd, zd), xd, yd, zd);
             else x = fast_sample<DT>(V, rs, tab, xd, yd, zd);
             const unsigned long long neg = __ballot(act && x < 0.f);
             const unsigned grp = (unsigned)(neg >> gshift) & ((1u << S) - 1u);
@@ -1922,6 +2082,12 @@ int launch_check_div(const DevVolume& v, unsigned* bad_dev, void* stream) {
 static int brick_row_grid(const DevVolume& v, int nbz) {
     const long long rows = (long long)((v.nbx + kBrickRow - 1) / kBrickRow) * v.nby * nbz;
     return (int)((rows + 7) / 8 * 8);
+}
+
+int launch_cmem_zones(const CmemParams& m, void* zones, void* stream) {
+    hipLaunchKernelGGL(k_cmem_zones, dim3((BIRP_ZONE_CT * BIRP_ZONE_CP + BIRP_BLOCK - 1) / BIRP_BLOCK), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, m,
+                       (float4*)zones);
+    return hip_status(hipGetLastError());
 }
 
 int launch_build_quad(const DevVolume& v, void* quad, void* stream) {
