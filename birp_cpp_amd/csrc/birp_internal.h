@@ -189,10 +189,12 @@ int launch_sample_points(const DevVolume& v, const float* xyz, long long n, floa
 int launch_space_points(const ExactView& ev, int row0, int rows, float* xyz, void* stream);
 int launch_space_integrate(const ExactView& ev, int row0, int rows, const float* vals, float* img, void* stream);
 // tab_entries: the largest nx + ny + nz of the volumes the launch reads (<= 2048; any value for CMEM)
-int launch_fast_batch(const DevVolume* vols_dev, int dtype, const FastPose* poses_dev, const int* tile_prefix_dev,
-                      int npose, int total_tiles, unsigned* work_counter, int tile_w, int tile_h,
-                      int lanes_per_ray, int unroll, int grid, void* stream, int tab_entries);
-int launch_reset_counter(unsigned* counter, void* stream);
+// Many views: view k's tiles are blocks [block_prefix_dev[k], block_prefix_dev[k + 1]) of the launch, fast_blocks each.
+int launch_fast_batch(const DevVolume* vols_dev, int dtype, const FastPose* poses_dev, const int* block_prefix_dev,
+                      int npose, int total_blocks, int tile_w, int tile_h, int lanes_per_ray, int unroll, void* stream,
+                      int tab_entries);
+// blocks (of 4 wave tiles) of a view of `tiles` tiles
+inline int fast_blocks(int tiles) { return (int)(((long long)tiles + 3) / 4); }
 int launch_zero_f32(float* p, size_t n, void* stream);
 // Words of the class scan's flags (one cache line each), in a buffer of BIRP_SCAN_WORDS.
 #define BIRP_SCAN_CLASS 0
@@ -210,7 +212,7 @@ int launch_build_oct(const DevVolume& v, void* oct, float* bscale, void* stream)
 
 // Fast-path kernel variants: the storage dtype (BIRP_DTYPE_*), or F16 whose records share one
 // scale for the whole volume, which the kernel then applies once per ray instead of per sample;
-// plus BIRP_KDT_SIGNED for volumes with values <= 0, whose kernels stop each ray at its first
+// plus BIRP_KDT_SIGNED for volumes with negative values, whose kernels stop each ray at its first
 // negative sample (Camera.cpp:207-210) and take one sample per lane per trip. Positive volumes
 // use the kernels without the stop test.
 // BIRP_KDT_CMEM is the analytic model in the fast form (FP32 with the hardware exp2/log2 and
@@ -222,33 +224,25 @@ int launch_build_oct(const DevVolume& v, void* oct, float* bscale, void* stream)
 inline int fast_kernel_dtype(const DevVolume& d) {
     if (d.kind == SK_CMEM) return BIRP_KDT_CMEM;
     const int base = (d.dtype == BIRP_DTYPE_F16 && d.f16_uniform) ? BIRP_KDT_F16_UNIFORM : d.dtype;
-    return base | (d.vclass != VC_POSITIVE ? BIRP_KDT_SIGNED : 0);
+    return base | (d.vclass != VC_POSITIVE && d.vclass != VC_NONNEG ? BIRP_KDT_SIGNED : 0);
 }
-int fast_grid_size(int dtype, int lanes_per_ray, int unroll, int tab_entries);
-// per-wave LDS table words of a fast launch whose largest table has tab_entries entries
-int fast_tab_stride(int dtype, int tab_entries);
 inline int volume_tab_entries(const DevVolume& d) { return d.kind == SK_CMEM ? 0 : d.nx + d.ny + d.nz; }
 
 // birp_render_views_noalloc: its fast launches read their descriptors from a fixed device array
-// (render.hip) laid out as [DevVolume | FastPose x BIRP_NOALLOC_MAX_VIEWS | tile prefix sums of the
-// three lanes-per-ray groups | work-queue counters of the three groups, 256 each].
+// (render.hip) laid out as [DevVolume | FastPose x BIRP_NOALLOC_MAX_VIEWS | block prefix sums of the
+// three lanes-per-ray groups].
 #define BIRP_NOALLOC_MAX_VIEWS 64
 #define BIRP_NOALLOC_POSE_OFF 1024
 #define BIRP_NOALLOC_PREFIX_OFF (BIRP_NOALLOC_POSE_OFF + 256 * BIRP_NOALLOC_MAX_VIEWS)
-#define BIRP_NOALLOC_CTR_OFF (BIRP_NOALLOC_PREFIX_OFF + 1024)
-#define BIRP_NOALLOC_SCRATCH_BYTES (BIRP_NOALLOC_CTR_OFF + 3 * 256 * 4)
+#define BIRP_NOALLOC_SCRATCH_BYTES (BIRP_NOALLOC_PREFIX_OFF + 1024)
 // The device address of this GPU's array (the current device's), from hipGetSymbolAddress.
 int noalloc_scratch_address(void** out);
-// Stage the volume, the prefix sums (3 groups x (BIRP_NOALLOC_MAX_VIEWS + 1) ints) and cleared
-// counters, then poses [first, first + count) (count <= 4 per call), into the array at `scratch`
+// Stage the volume and the prefix sums (3 groups x (BIRP_NOALLOC_MAX_VIEWS + 1) ints), then poses [first, first + count) (count <= 4 per call), into the array at `scratch`
 // by kernels on `stream` (their arguments carry the data: no copy from host memory).
 int noalloc_stage_head(const DevVolume& v, const int* prefix, void* scratch, void* stream);
 int noalloc_stage_poses(const FastPose* poses, int first, int count, void* scratch, void* stream);
-// The grid of one persistent launch over `tiles` tiles: the occupancy-limited grid, or about one
-// wave per tile when that is smaller (idle waves cost serialized work-queue claims on exit).
 // One pose over one volume, both by value, as a plain grid of its tiles (k_render_fast_one): no
-// descriptors on the device and no work counters; the same per-tile arithmetic as launch_fast_batch.
+// descriptors on the device; the same per-tile arithmetic as launch_fast_batch.
 int launch_fast_one(const DevVolume& v, int dtype, const FastPose& pose, int total_tiles, int tile_w, int tile_h, int lanes_per_ray,
                     int unroll, void* stream, int tab_entries);
-int fast_grid_for(int dtype, int lanes_per_ray, int unroll, int tiles, int tab_entries);
 }  // namespace birp

@@ -1079,47 +1079,46 @@ int choose_tuning(const birp_volume* vol, const std::vector<birp_view>& views, b
     }
     if (!views.empty() && birp_autotune_lookup(vol->desc.dtype, views[bi].width, views[bi].height, views[bi].samples, &t) == BIRP_OK)
         return BIRP_OK;
-    // untuned default: the tuner's most frequent winner on the standard workloads
-    t.tile_w = 8;
-    t.tile_h = 8;
-    t.lanes_per_ray = 1;
-    t.unroll = 4;
+    long long rays = 0;
+    for (const birp_view& v : views) rays += (long long)v.width * v.height;
+    // untuned: signed cubes and CMEM models keep 8x8 rays per wave (their images depend on it)
+    t = tuning_is_free(fast_kernel_dtype(vol->dv)) ? launch_tuning(rays) : birp_tuning{8, 8, 1, 4};
     return BIRP_OK;
 }
 
-// The tuning of a fast render launched alone or in a server batch, chosen for latency from the
-// view and the volume's storage alone (so a request's result never depends on what it is batched
-// with): an image with few rays splits each ray over 2 or 4 lanes, shortening every lane's chain
-// of dependent sample gathers. Measured on back-to-back single launches of 6 orbit poses (256^3
-// cube), ms per render for 1 / 2 / 4 lanes per ray:
-//   144x84,  n = 160: F32 0.028 / 0.030 / 0.030, F16 0.027 / 0.024 / 0.027
-//   144x84,  n = 320: F32 0.036 / 0.039 / 0.033, F16 0.034 / 0.027 / 0.028
-//   144x84,  n = 800: F32 0.060 / 0.063 / 0.044, F16 0.054 / 0.037 / 0.032
-//   288x168, n = 800: F32 0.059 / 0.067 / 0.073, F16 0.054 / 0.049 / 0.063
-//   576x336 and 288x168 at n <= 320: 1 lane, by 20-70%
-// (BF16 as F32). A CMEM model costs about 25 transcendentals per sample, whose chains want more
-// waves per SIMD than a cube's gathers: its views take 4 lanes per ray over 4x4 rays whatever
-// their size (576x336 at n = 800: 0.724 ms, against 0.817 ms with 1 lane and 0.733 ms with 2).
-birp_tuning latency_tuning(const birp_view& v, const DevVolume& vol) {
-    const bool cmem = vol.kind == SK_CMEM;
+// A launch's fast render over a cube without negative values, by its rays (its images do not depend on the
+// tuning): few rays are a few waves waiting on each sample's loads, and 4 lanes per ray over 4x4 rays cut
+// the chain of each ray's samples by four; where the waves fill the SIMDs every lane's FP64 ray setup counts,
+// and fewer lanes per ray repeat it less. us per launch (FP16, 190^3 cube, orbit views), by lanes per ray
+// (tile):
+//                            rays    1 (8x8)  2 (4x8)  4 (4x4)
+//   144x84,  n = 320, 1       12 k    21.7     16.8     14.1
+//   288x168, n = 320, 2       97 k    22.7     19.3     19.6
+//   288x168, n = 800, 4      194 k    70.4     55.9     52.5
+//   576x336, n = 800, 1      194 k    43.4     39.3     39.6
+//   288x168, n = 320, 16     774 k    79.4     72.9     80.2
+//   576x336, n = 800, 16     3.1 M   505      487      521
+//   64 mixed orbit views     5.4 M   595      593      690   (BF16 616, 652, 759)
+//   256 mixed orbit views   21.7 M  2238     2308     2710
+birp_tuning launch_tuning(long long rays) {
+    if (rays <= 150000) return birp_tuning{4, 4, 4, 4};
+    if (rays <= 4000000) return birp_tuning{4, 8, 2, 4};
+    return birp_tuning{8, 8, 1, 4};
+}
+
+// A signed cube's view: an image with few rays splits each ray over 2 or 4 lanes (FP16 storage earlier), which
+// shortens each lane's chain of dependent gathers.
+// A CMEM model's chains of transcendentals want more waves per SIMD than a cube's gathers: its views take
+// 4 lanes per ray over 4x4 rays whatever their size (576x336 at n = 800: 0.724 ms, against 0.817 ms with
+// 1 lane and 0.733 ms with 2).
+birp_tuning view_tuning(const birp_view& v, const DevVolume& vol) {
+    if (vol.kind == SK_CMEM) return birp_tuning{4, 4, 4, 1};
     const bool f16 = vol.dtype == BIRP_DTYPE_F16;
-    birp_tuning t;
-    if (cmem) {
-        t.lanes_per_ray = 4;
-        t.unroll = 1;
-        t.tile_w = 4;
-        t.tile_h = 4;
-        return t;
-    }
     const long long rays = (long long)v.width * v.height;
     int lanes = 1;
     if (rays <= 20000) lanes = v.samples >= 600 ? 4 : (f16 ? 2 : (v.samples >= 240 ? 4 : 1));
     else if (rays <= 60000 && v.samples >= 600 && f16) lanes = 2;
-    t.lanes_per_ray = lanes;
-    t.unroll = 4;
-    t.tile_w = 8;
-    t.tile_h = 64 / (8 * lanes);
-    return t;
+    return birp_tuning{8, 64 / (8 * lanes), lanes, 4};
 }
 
 void batch_release(birp_batch* b) {
@@ -1332,6 +1331,13 @@ int exact_batch_setup(birp_batch* b) {
     return BIRP_OK;
 }
 
+// The kernel of a fast batch on stream st.
+static int fast_batch_launch(birp_batch* b, hipStream_t st) {
+    const birp_tuning& t = b->tuning;
+    return launch_fast_batch(b->d_vols, fast_kernel_dtype(b->vol->dv), b->d_poses, b->d_prefix, (int)b->views.size(), b->total_blocks,
+                             t.tile_w, t.tile_h, t.lanes_per_ray, t.unroll, st, volume_tab_entries(b->vol->dv));
+}
+
 int batch_setup(birp_batch* b) {
     if (b->exact) return exact_batch_setup(b);
     birp_device* dev = b->vol->dev;
@@ -1344,11 +1350,11 @@ int batch_setup(birp_batch* b) {
         float* out = (b->host_out_dev ? b->host_out_dev : b->d_images) + b->offsets[k];
         int rc = fast_pose(b->vol, &b->views[k], 0, out, t.tile_w, t.tile_h, poses[k]);
         if (rc) return rc;
-        const long long next = (long long)prefix[k] + tiles_of(b->views[k], t.tile_w, t.tile_h);
+        const long long next = (long long)prefix[k] + fast_blocks(tiles_of(b->views[k], t.tile_w, t.tile_h));
         if (next > INT32_MAX) return fail(BIRP_ERR_UNSUPPORTED, "batch of more than 2^31 - 1 tiles: split it");
         prefix[k + 1] = (int)next;
     }
-    b->total_tiles = prefix[n];
+    b->total_blocks = prefix[n];
     hipError_t e;
     if ((e = hipMalloc(&b->d_poses, sizeof(FastPose) * n)) != hipSuccess) return hip_fail(e, "hipMalloc(poses)");
     if ((e = hipMalloc(&b->d_prefix, sizeof(int) * (n + 1))) != hipSuccess) return hip_fail(e, "hipMalloc(prefix)");
@@ -1358,14 +1364,9 @@ int batch_setup(birp_batch* b) {
     if (e == hipSuccess) e = hipMemcpyAsync(b->d_vols, &b->vol->dv, sizeof(DevVolume), hipMemcpyHostToDevice, dev->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
     if (e != hipSuccess) return hip_fail(e, "batch upload");
-    b->grid = fast_grid_for(fast_kernel_dtype(b->vol->dv), t.lanes_per_ray, t.unroll, b->total_tiles, volume_tab_entries(b->vol->dv));
-    // capture: reset the work counter (a kernel, not a memset node), then the persistent kernel
     hipStream_t cs = b->capture_stream;
     if ((e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal)) != hipSuccess) return hip_fail(e, "begin capture");
-    int rc = launch_reset_counter(b->d_work, cs);
-    if (rc == BIRP_OK)
-        rc = launch_fast_batch(b->d_vols, fast_kernel_dtype(b->vol->dv), b->d_poses, b->d_prefix, n, b->total_tiles, b->d_work, t.tile_w,
-                               t.tile_h, t.lanes_per_ray, t.unroll, b->grid, cs, volume_tab_entries(b->vol->dv));
+    const int rc = fast_batch_launch(b, cs);
     e = hipStreamEndCapture(cs, &b->graph);
     if (rc != BIRP_OK) return fail(rc, "batch capture launch failed");
     if (e != hipSuccess) return hip_fail(e, "end capture");
@@ -1400,7 +1401,6 @@ extern "C" int birp_batch_create(birp_volume* vol, const birp_view* views, int c
     int rc;
     if ((e = hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking)) != hipSuccess) { rc = hip_fail(e, "stream"); goto bad; }
     if ((e = hipMalloc(&b->d_images, off * sizeof(float))) != hipSuccess) { rc = hip_fail(e, "hipMalloc(images)"); goto bad; }
-    if ((e = hipMalloc(&b->d_work, 1024)) != hipSuccess) { rc = hip_fail(e, "hipMalloc(counter)"); goto bad; }
     if ((e = hipEventCreate(&b->ev0)) != hipSuccess || (e = hipEventCreate(&b->ev1)) != hipSuccess) { rc = hip_fail(e, "event"); goto bad; }
     choose_tuning(vol, b->views, b->tuning);
     if ((rc = batch_setup(b)) != BIRP_OK) goto bad;
@@ -1485,7 +1485,6 @@ extern "C" int birp_batch_free(birp_batch* b) {
     batch_release(b);
     if (b->d_counts) (void)hipFree(b->d_counts);
     if (b->d_images) (void)hipFree(b->d_images);
-    if (b->d_work) (void)hipFree(b->d_work);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     if (b->capture_stream) (void)hipStreamDestroy(b->capture_stream);
@@ -1533,7 +1532,6 @@ extern "C" int birp_batch_launch_eager(birp_batch* b) {
     if (!b || (!b->d_poses && !b->d_evs)) return fail(BIRP_ERR_INVALID_ARGUMENT, "batch not ready");
     birp_device* dev = b->vol->dev;
     if (take_injected_failure(dev)) return fail(BIRP_ERR_INJECTED, "injected failure");
-    const birp_tuning& t = b->tuning;
     (void)hipEventRecord(b->ev0, dev->stream);
     if (b->exact) {
         int rc = exact_batch_launch(b, dev->stream);
@@ -1542,11 +1540,7 @@ extern "C" int birp_batch_launch_eager(birp_batch* b) {
         b->launched = true;
         return BIRP_OK;
     }
-    int rc = launch_reset_counter(b->d_work, dev->stream);
-    if (rc == BIRP_OK)
-        rc = launch_fast_batch(b->d_vols, fast_kernel_dtype(b->vol->dv), b->d_poses, b->d_prefix, (int)b->views.size(),
-                               b->total_tiles, b->d_work, t.tile_w, t.tile_h, t.lanes_per_ray, t.unroll, b->grid, dev->stream,
-                               volume_tab_entries(b->vol->dv));
+    const int rc = fast_batch_launch(b, dev->stream);
     if (rc) return fail(rc, "batch launch failed");
     (void)hipEventRecord(b->ev1, dev->stream);
     b->launched = true;
@@ -1601,10 +1595,9 @@ extern "C" int birp_batch_stats(birp_batch* b, long long* nominal, double* last_
 }
 
 // birp_render_views_noalloc: birp_render_async of each view without allocating. Exact views launch
-// the exact kernel (it needs no scratch); fast views are grouped by the lanes per ray of their
-// latency tuning (the tuning birp_render_async uses, so the images are the same bit for bit) and
-// each group is one persistent launch whose volume, poses, prefix sums and work counters are
-// staged by kernels into the device's fixed scratch array.
+// the exact kernel (it needs no scratch); fast views are one launch, over a signed cube one per lanes
+// per ray of the views' tunings (the tunings birp_render_async uses, so the images are the same bit for
+// bit), whose volume, poses and prefix sums are staged by kernels into the device's fixed scratch array.
 extern "C" int birp_render_views_noalloc(birp_volume* vol, const birp_view* views, int count, float* const* images_dev) {
     if (!vol || !views || !images_dev || count <= 0) return fail(BIRP_ERR_INVALID_ARGUMENT, "bad argument");
     if (count > BIRP_NOALLOC_MAX_VIEWS)
@@ -1624,15 +1617,19 @@ extern "C" int birp_render_views_noalloc(birp_volume* vol, const birp_view* view
     int nfast[3] = {0, 0, 0};
     birp_tuning gt[3] = {};
     int nf = 0;
+    const bool free_tuning = tuning_is_free(fast_kernel_dtype(vol->dv));  // then all fast views are one launch
+    long long rays = 0;
+    for (int k = 0; k < count; k++)
+        if (views[k].math == BIRP_MATH_FAST) rays += (long long)views[k].width * views[k].height;
     for (int g = 0; g < 3; g++) {  // lanes per ray 1, 2, 4: poses of group g are contiguous
         for (int k = 0; k < count; k++) {
             if (views[k].math != BIRP_MATH_FAST) continue;
-            const birp_tuning t = latency_tuning(views[k], vol->dv);
+            const birp_tuning t = free_tuning ? launch_tuning(rays) : view_tuning(views[k], vol->dv);
             if (t.lanes_per_ray != (1 << g)) continue;
             int rc = fast_pose(vol, &views[k], 0, images_dev[k], t.tile_w, t.tile_h, poses[nf]);
             if (rc) return rc;
             int* pre = prefix + g * (BIRP_NOALLOC_MAX_VIEWS + 1);
-            const long long next = (long long)pre[nfast[g]] + tiles_of(views[k], t.tile_w, t.tile_h);
+            const long long next = (long long)pre[nfast[g]] + fast_blocks(tiles_of(views[k], t.tile_w, t.tile_h));
             if (next > INT32_MAX) return fail(BIRP_ERR_UNSUPPORTED, "more than 2^31 - 1 tiles");
             pre[nfast[g] + 1] = (int)next;
             nfast[g]++;
@@ -1656,25 +1653,21 @@ extern "C" int birp_render_views_noalloc(birp_volume* vol, const birp_view* view
         const int* pre_dev = reinterpret_cast<const int*>(s + BIRP_NOALLOC_PREFIX_OFF) + g * (BIRP_NOALLOC_MAX_VIEWS + 1);
         const int total = prefix[g * (BIRP_NOALLOC_MAX_VIEWS + 1) + nfast[g]];
         const birp_tuning& t = gt[g];
-        const int grid = fast_grid_for(kdt, t.lanes_per_ray, t.unroll, total, volume_tab_entries(vol->dv));
         rc = launch_fast_batch(reinterpret_cast<const DevVolume*>(s), kdt, reinterpret_cast<const FastPose*>(s + BIRP_NOALLOC_POSE_OFF) + first,
-                               pre_dev, nfast[g], total, reinterpret_cast<unsigned*>(s + BIRP_NOALLOC_CTR_OFF) + g * 256, t.tile_w, t.tile_h,
-                               t.lanes_per_ray, t.unroll, grid, dev->stream, volume_tab_entries(vol->dv));
+                               pre_dev, nfast[g], total, t.tile_w, t.tile_h, t.lanes_per_ray, t.unroll, dev->stream,
+                               volume_tab_entries(vol->dv));
         if (rc) return fail(rc, "fast launch failed");
         first += nfast[g];
     }
     return BIRP_OK;
 }
 
-// A single fast render: a one-pose launch of the persistent kernel (no graph). Its descriptors go
-// through the device's ring of pinned slots, so the host waits only for the upload issued
-// kFastRing renders earlier, not for the work queued before this render.
 // A fast single render: its pose and volume go to the one-shot kernel by value, so the launch
-// needs nothing uploaded and no counters reset.
+// needs nothing uploaded.
 static int render_fast_into(birp_volume* vol, const birp_view* view, float* dimg) {
     birp_device* dev = vol->dev;
     if (view->flags & BIRP_RENDER_ACCUMULATE) return fail(BIRP_ERR_UNSUPPORTED, "fast renders do not accumulate");
-    const birp_tuning t = latency_tuning(*view, vol->dv);
+    const birp_tuning t = tuning_is_free(fast_kernel_dtype(vol->dv)) ? launch_tuning((long long)view->width * view->height) : view_tuning(*view, vol->dv);
     FastPose fp;
     int rc = fast_pose(vol, view, 0, dimg, t.tile_w, t.tile_h, fp);
     if (rc) return rc;

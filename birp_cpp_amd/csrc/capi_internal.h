@@ -85,9 +85,7 @@ struct birp_batch {
     birp::FastPose* d_poses = nullptr;
     int* d_prefix = nullptr;
     birp::DevVolume* d_vols = nullptr;
-    unsigned* d_work = nullptr;
-    int total_tiles = 0;
-    int grid = 0;
+    int total_blocks = 0;
     birp_tuning tuning{4, 4, 4, 2};
     hipStream_t capture_stream = nullptr;
     hipGraph_t graph = nullptr;
@@ -127,7 +125,12 @@ int default_exact_pipe();
 int tiles_of(const birp_view& v, int tile_w, int tile_h);
 bool take_injected_failure(birp_device* dev);
 int choose_tuning(const birp_volume* vol, const std::vector<birp_view>& views, birp_tuning& t);
-birp_tuning latency_tuning(const birp_view& v, const birp::DevVolume& vol);
+// The tuning of a fast render of `rays` rays over a cube without negative values, alone or as a launch of
+// several views (the images do not depend on it).
+birp_tuning launch_tuning(long long rays);
+// The tuning of a view's fast render over a signed cube or a CMEM model, whose images depend on it: from the view alone.
+birp_tuning view_tuning(const birp_view& v, const birp::DevVolume& vol);
+inline bool tuning_is_free(int kernel_dtype) { return !(kernel_dtype & (BIRP_KDT_SIGNED | BIRP_KDT_CMEM)); }
 // true when [p, p + bytes) lies inside one birp_host_alloc allocation (pinned host memory)
 bool pinned_range(const void* p, size_t bytes);
 // its device address when the allocation is mapped into the device's address space, else null

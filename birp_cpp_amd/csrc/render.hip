@@ -9,7 +9,7 @@
 //              scale chain via birp_scale_sample, std::lerp's branch structure, and the image sum
 //              in k order. Bit-identical to the reference CPU render for finite cubes.
 //  * fast   -- FP64 camera basis, ray origin and cube entry; FP32 FMA march in index space;
-//              BF16/F16/FP32 storage; FP32 Kahan sums. Batched in a persistent work-queue kernel.
+//              BF16/F16/FP32 storage; FP32 Kahan sums. Many views in one launch.
 //
 // Wave mapping: a wave64 owns a tile of 64/S rays; S lanes ("sub-lanes") share one ray and take
 // its samples k = kb + sub, kb advancing by S each trip. In the exact kernels every sub-lane then
@@ -24,7 +24,7 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
-#include <atomic>
+#include <type_traits>
 
 #include "../../include/birp.h"
 #include "birp_internal.h"
@@ -34,7 +34,7 @@ namespace birp {
 
 #define BIRP_BLOCK 256
 #define BIRP_MAX_EXACT_SAMPLES 8192
-#define BIRP_FAST_TAB 2048  // largest per-wave LDS table of the fast kernel (nx+ny+nz entries)
+#define BIRP_FAST_TAB 2048  // largest LDS table of the fast kernels (nx+ny+nz entries)
 #define BIRP_RSRC_WORD3 0x00020000
 
 // ------------------------------------------------------------------------------------------
@@ -1353,16 +1353,12 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_build_oct(DevVolume v, unsigned 
     }
 }
 
-__global__ void k_reset_counter(unsigned* c) {
-    if (blockIdx.x == 0 && threadIdx.x < 256) c[threadIdx.x] = 0u;
-}
-
 __global__ __launch_bounds__(BIRP_BLOCK) void k_zero_f32(float* p, size_t n) {
     for (size_t idx = (size_t)blockIdx.x * BIRP_BLOCK + threadIdx.x; idx < n; idx += (size_t)gridDim.x * BIRP_BLOCK) p[idx] = 0.f;
 }
 
 // ------------------------------------------------------------------------------------------
-// fast path: persistent work-queue kernel over (pose, tile) items
+// fast path: many views in one launch, or one by value
 // ------------------------------------------------------------------------------------------
 __device__ __forceinline__ float bf16lo(unsigned u) { return __uint_as_float(u << 16); }
 __device__ __forceinline__ float bf16hi(unsigned u) { return __uint_as_float(u & 0xFFFF0000u); }
@@ -1380,37 +1376,53 @@ __device__ __forceinline__ float xlerp_f16(unsigned u, float t) {
 }
 
 // Fast trilinear sample at index-space point (xd, yd, zd), already clamped into
-// [0, nextbelow(n-1)] per axis, so the truncation is a valid cell index (0 .. n-2).
+// [0, nextbelow(n-1)] per axis, so the truncation is a valid cell index (0 .. n-2): the record's
+// loads, then its lerps.
 template <int DT>
-__device__ __forceinline__ float fast_sample(const DevVolume& v, __amdgpu_buffer_rsrc_t rs, const unsigned* tab, float xd,
-                                             float yd, float zd) {
-    float fx = __builtin_amdgcn_fractf(xd), fy = __builtin_amdgcn_fractf(yd), fz = __builtin_amdgcn_fractf(zd);
-    int ix = (int)xd, iy = (int)yd, iz = (int)zd;
+struct FastFetch {
+    uint4 a;           // FP32: the z record; else the octet
+    float4 b;          // FP32: the z + 1 record
+    float fx, fy, fz;  // lerp weights
+    float scale;       // F16 with a scale per brick
+};
+template <int DT>
+__device__ __forceinline__ FastFetch<DT> fast_fetch(const DevVolume& v, __amdgpu_buffer_rsrc_t rs, const unsigned* tab, float xd, float yd, float zd) {
+    FastFetch<DT> q;
+    q.fx = __builtin_amdgcn_fractf(xd);
+    q.fy = __builtin_amdgcn_fractf(yd);
+    q.fz = __builtin_amdgcn_fractf(zd);
+    const unsigned xo = tab[(int)xd], yo = tab[v.nx + (int)yd];
+    const unsigned* zo = tab + v.nx + v.ny + (int)zd;
+    const unsigned off = add3(xo, yo, zo[0]);
+    q.a = load16u(rs, off);
+    if constexpr (DT == BIRP_DTYPE_F32) q.b = load16(rs, add3(xo, yo, zo[1]));
+    if constexpr (DT == BIRP_DTYPE_F16) q.scale = v.bscale[off >> 13];
+    return q;
+}
+template <int DT>
+__device__ __forceinline__ float fast_value(const FastFetch<DT>& q) {
     if constexpr (DT == BIRP_DTYPE_F32) {
-        const unsigned xo = tab[ix], yo = tab[v.nx + iy];
-        const unsigned* zo = tab + v.nx + v.ny + iz;
-        float4 a = load16(rs, add3(xo, yo, zo[0])), b = load16(rs, add3(xo, yo, zo[1]));
-        float ly = flerp(flerp(a.x, a.y, fx), flerp(a.z, a.w, fx), fy);
-        float hy = flerp(flerp(b.x, b.y, fx), flerp(b.z, b.w, fx), fy);
-        return flerp(ly, hy, fz);
+        const float4 a = __builtin_bit_cast(float4, q.a), b = q.b;
+        float ly = flerp(flerp(a.x, a.y, q.fx), flerp(a.z, a.w, q.fx), q.fy);
+        float hy = flerp(flerp(b.x, b.y, q.fx), flerp(b.z, b.w, q.fx), q.fy);
+        return flerp(ly, hy, q.fz);
     } else {  // BF16, F16 with per-brick scale, F16 with one scale (BIRP_KDT_F16_UNIFORM)
         // each dword of the record holds the x-pair (x0, x1) of one (y, z) corner row
-        const unsigned off = tab[ix] + tab[v.nx + iy] + tab[v.nx + v.ny + iz];
-        uint4 o = load16u(rs, off);
+        const uint4 o = q.a;
         float c00, c10, c01, c11;  // the four x-lerps, at (y0,z0), (y1,z0), (y0,z1), (y1,z1)
         if constexpr (DT == BIRP_DTYPE_BF16) {
-            c00 = flerp(bf16lo(o.x), bf16hi(o.x), fx);
-            c10 = flerp(bf16lo(o.y), bf16hi(o.y), fx);
-            c01 = flerp(bf16lo(o.z), bf16hi(o.z), fx);
-            c11 = flerp(bf16lo(o.w), bf16hi(o.w), fx);
+            c00 = flerp(bf16lo(o.x), bf16hi(o.x), q.fx);
+            c10 = flerp(bf16lo(o.y), bf16hi(o.y), q.fx);
+            c01 = flerp(bf16lo(o.z), bf16hi(o.z), q.fx);
+            c11 = flerp(bf16lo(o.w), bf16hi(o.w), q.fx);
         } else {
-            c00 = xlerp_f16(o.x, fx);
-            c10 = xlerp_f16(o.y, fx);
-            c01 = xlerp_f16(o.z, fx);
-            c11 = xlerp_f16(o.w, fx);
+            c00 = xlerp_f16(o.x, q.fx);
+            c10 = xlerp_f16(o.y, q.fx);
+            c01 = xlerp_f16(o.z, q.fx);
+            c11 = xlerp_f16(o.w, q.fx);
         }
-        float val = flerp(flerp(c00, c10, fy), flerp(c01, c11, fy), fz);
-        if constexpr (DT == BIRP_DTYPE_F16) val *= v.bscale[off >> 13];
+        float val = flerp(flerp(c00, c10, q.fy), flerp(c01, c11, q.fy), q.fz);
+        if constexpr (DT == BIRP_DTYPE_F16) val *= q.scale;
         return val;
     }
 }
@@ -1521,6 +1533,29 @@ __device__ __forceinline__ void fit_march(float& i0, float& d, float hi, int las
     if (!(e >= 0.f && e <= hi)) d = 0.f;
 }
 
+// 1/x and 1/sqrt(x) in double from the hardware's first approximations (within about 2^-23) and two Newton
+// steps each: within an ulp or two, a third of the IEEE sequences' instructions. x finite, normal, not 0.
+__device__ __forceinline__ double rcp64(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+    return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+__device__ __forceinline__ double rsqrt64(double x) {
+    double r = __builtin_amdgcn_rsq(x);
+    r = __builtin_fma(__builtin_fma(-0.5 * x * r, r, 0.5), r, r);
+    return __builtin_fma(__builtin_fma(-0.5 * x * r, r, 0.5), r, r);
+}
+// slab_axis with rcp64; a direction component below 2^-100 moves no sample by an FP32 ulp
+__device__ __forceinline__ void slab_axis_fast(double p, double d, double lo, double hi, double& tin, double& tout) {
+    if (fabs(d) < 0x1p-100) {
+        if (p < lo || p > hi) { tin = 1e300; tout = -1e300; }
+    } else {
+        const double inv = rcp64(d), t1 = (lo - p) * inv, t2 = (hi - p) * inv;
+        tin = fmax(tin, fmin(t1, t2));
+        tout = fmin(tout, fmax(t1, t2));
+    }
+}
+
 // x folded into a Kahan sum (sum, nc), nc holding the negated compensation -c:
 // y = x - c; t = sum + y; -c' = y - (t - sum); sum = t.
 __device__ __forceinline__ void kahan_add(float x, float& sum, float& nc) {
@@ -1583,12 +1618,12 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
         double sy = (1 - 2 * ((j + 0.5) * P.inv_h)) * P.tany;
         // (divisions by a norm or a spacing as products with its FP64 reciprocal: a relative
         // change of ~1e-16, far below the FP32 march)
-        const double ind = 1.0 / sqrt(sx * sx + sy * sy + 1.0);
+        const double ind = rsqrt64(sx * sx + sy * sy + 1.0);
         double u0 = sx * ind, u1 = sy * ind, u2 = -ind;
         double w0 = P.rinv[0] * u0 + P.rinv[1] * u1 + P.rinv[2] * u2;
         double w1 = P.rinv[3] * u0 + P.rinv[4] * u1 + P.rinv[5] * u2;
         double w2 = P.rinv[6] * u0 + P.rinv[7] * u1 + P.rinv[8] * u2;
-        const double iwd = 1.0 / sqrt(w0 * w0 + w1 * w1 + w2 * w2);
+        const double iwd = rsqrt64(w0 * w0 + w1 * w1 + w2 * w2);
         double dx = w0 * iwd, dy = w1 * iwd, dz = w2 * iwd;
         if constexpr (CMEM) {
             // the model has no bounds: every sample, marched in world coordinates
@@ -1604,9 +1639,9 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
         } else {
             // FP64 cube entry/exit: inside iff 0 <= (x - o)/s < n - 1 per axis
             double tin = -1e300, tout = 1e300;
-            slab_axis(P.px, dx, (double)V.ox, (double)V.ox + (double)(V.nx - 1) * V.sx, tin, tout);
-            slab_axis(P.py, dy, (double)V.oy, (double)V.oy + (double)(V.ny - 1) * V.sy, tin, tout);
-            slab_axis(P.pz, dz, (double)V.oz, (double)V.oz + (double)(V.nz - 1) * V.sz, tin, tout);
+            slab_axis_fast(P.px, dx, (double)V.ox, (double)V.ox + (double)(V.nx - 1) * V.sx, tin, tout);
+            slab_axis_fast(P.py, dy, (double)V.oy, (double)V.oy + (double)(V.ny - 1) * V.sy, tin, tout);
+            slab_axis_fast(P.pz, dz, (double)V.oz, (double)V.oz + (double)(V.nz - 1) * V.sz, tin, tout);
             if (tin <= tout) {
                 const double sc = P.sc;
                 double a = ceil(tin * sc - 0.5), b = ceil(tout * sc - 0.5) - 1.0;
@@ -1630,8 +1665,6 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
         }
     }
     const int cnt = (kl >= kf) ? (kl - kf + 1) : 0;
-    const int my = (cnt > sub) ? (cnt - sub + S - 1) / S : 0;  // samples of this sub-lane
-    const int trips = wave_max_i(my);
     if (!CMEM && cnt > 0) {
         // every sample inside [0, nextbelow(n - 1)] per axis, so that the cell index is the
         // truncation (0 .. n-2) with no clamp per sample; a sample rounded onto the far face
@@ -1640,16 +1673,15 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
         fit_march(iy0, diy, __uint_as_float(__float_as_uint(V.fny - 1.0f) - 1u), cnt - 1);
         fit_march(iz0, diz, __uint_as_float(__float_as_uint(V.fnz - 1.0f) - 1u), cnt - 1);
     }
-    // the U samples of an iteration (neighbours on the ray, of similar size) are added plainly,
-    // and their partial sum enters the running sum by one Kahan step. The trips that every lane
-    // of the wave fills completely need no clamp and no mask; the rest of the trips run below
-    // with both (the same samples in the same order and grouping either way).
-    float sum = 0.f, nc = 0.f;
+    float tot;
     if constexpr (SIGNED) {
         // Camera.cpp:207-210: a ray ends at its first negative sample. The S lanes of a ray take
         // samples q*S + sub in trip q, so the ray's first negative sample of a trip is the lowest
         // set bit of its S-bit group in the wave's ballot: a lane adds its sample unless its
         // group has a negative sample at or before it, and the ray dies with any in the group.
+        const int my = (cnt > sub) ? (cnt - sub + S - 1) / S : 0;  // samples of this sub-lane
+        const int trips = wave_max_i(my);
+        float sum = 0.f, nc = 0.f;
         const int gshift = ray * S;
         bool alive = true;  // the same in all S lanes of a ray
         for (int q = 0; q < trips; ++q) {
@@ -1661,7 +1693,7 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
             const float zd = __builtin_fmaf(fj, diz, iz0);
             float x;
             if constexpr (CMEM) x = cmem_fast_zoned(V.cmem, zone_fetch(rs, xd, yd, zd), xd, yd, zd);
-            else x = fast_sample<DT>(V, rs, tab, xd, yd, zd);
+            else x = fast_value<DT>(fast_fetch<DT>(V, rs, tab, xd, yd, zd));
             const unsigned long long neg = __ballot(act && x < 0.f);
             const unsigned grp = (unsigned)(neg >> gshift) & ((1u << S) - 1u);
             const bool cut = (grp & ((2u << sub) - 1u)) != 0u;
@@ -1669,139 +1701,157 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
             alive = alive && grp == 0u;
             if (__ballot(alive && (q + 1) * S < cnt) == 0ull) break;  // every ray of the wave is done
         }
+        // each sub-lane's Kahan total, then the S partials combined in sub order
+        tot = sum + nc;
+        if constexpr (S > 1) {
+            const float t1 = __shfl_xor(tot, sub_step, 64);
+            tot = (sub & 1) ? t1 + tot : tot + t1;
+            if constexpr (S == 4) {
+                const float t2 = __shfl_xor(tot, 2 * sub_step, 64);
+                tot = (sub & 2) ? t2 + tot : tot + t2;
+            }
+        }
     }
-    const int tfull = SIGNED ? 0 : wave_min_i(my) / U * U;
-    int q = SIGNED ? trips : 0;
-    for (; q < tfull; q += U) {
-        float part = 0.f;
+    if constexpr (!SIGNED) {
+        // A ray's samples go in groups of 16 from its first, sample 16 g + 4 b + r to residue r: the four
+        // of a residue (neighbours on the ray, of similar size) are added plainly and their sum enters the
+        // residue's running sum by one Kahan step. Lane `sub` takes the residues sub, sub + S, ..., so
+        // the image does not depend on S, on the tile or on U, and a launch may choose them
+        // (launch_tuning): single 300x170 x 500 FP16 renders 28.8 us with one lane per ray, 17.3 with four.
+        // Groups that every ray of the wave fills need no clamp and no mask; the others run below with
+        // both, and with the same sums: a masked sample adds 0, and a ray's sums rest after its last group.
+        constexpr int R = 4 / S, B = U > R ? U / R : 1;  // residues per lane; rows b in flight together
+        float sum[R] = {}, nc[R] = {}, part[R];
+        auto at = [&](float fj) {
+            return fast_fetch<DT>(V, rs, tab, __builtin_fmaf(fj, dix, ix0), __builtin_fmaf(fj, diy, iy0), __builtin_fmaf(fj, diz, iz0));
+        };
+        FastFetch<DT> f[B * R];
+        const int full = wave_min_i(cnt), most = wave_max_i(cnt);
+        int g = 0;
+        for (; g + 16 <= full; g += 16) {
+            // B rows (max(U, R) samples) per iteration, their loads in flight together: left to itself the
+            // compiler issues them one by one, each waited for before the next
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const float fj = (float)((q + u) * S + sub);
-            const float xd = __builtin_fmaf(fj, dix, ix0);
-            const float yd = __builtin_fmaf(fj, diy, iy0);
-            const float zd = __builtin_fmaf(fj, diz, iz0);
-            const float x = fast_sample<DT>(V, rs, tab, xd, yd, zd);
-            part = (u == 0) ? x : part + x;
-        }
-        kahan_add(part, sum, nc);
-    }
-    for (; q < trips; q += U) {
-        float part = 0.f;
+            for (int q = 0; q < R; ++q) part[q] = 0.f;
+            float fb = (float)(g + sub);
+#pragma unroll 1
+            for (int b = 0; b < 4; b += B, fb += 4.0f * B) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int js = (q + u) * S + sub;  // sample offset from kf
-            const bool act = js < cnt;
-            // a lane past its ray's last sample re-reads that sample (its result is masked); an
-            // empty ray has i0 = d = 0 and samples the grid origin
-            const float fj = (float)min(js, cnt - 1);
-            const float xd = __builtin_fmaf(fj, dix, ix0);
-            const float yd = __builtin_fmaf(fj, diy, iy0);
-            const float zd = __builtin_fmaf(fj, diz, iz0);
-            const float x = fast_sample<DT>(V, rs, tab, xd, yd, zd);
-            const float xa = act ? x : 0.f;
-            part = (u == 0) ? xa : part + xa;
+                for (int c = 0; c < B * R; ++c) f[c] = at(fb + (float)(4 * (c / R) + S * (c % R)));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int c = 0; c < B * R; ++c) part[c % R] += fast_value<DT>(f[c]);
+            }
+#pragma unroll
+            for (int q = 0; q < R; ++q) kahan_add(part[q], sum[q], nc[q]);
         }
-        kahan_add(part, sum, nc);
-    }
-    // each sub-lane's Kahan total, then the S partials combined in sub order; the step weight
-    // and the scale constant are applied once per ray (all in FP32)
-    float tot = sum + nc;
-    if constexpr (S > 1) {
-        float t1 = __shfl_xor(tot, sub_step, 64);
-        tot = (sub & 1) ? t1 + tot : tot + t1;
-        if constexpr (S == 4) {
-            float t2 = __shfl_xor(tot, 2 * sub_step, 64);
-            tot = (sub & 2) ? t2 + tot : tot + t2;
+        for (; g < most; g += 16) {
+#pragma unroll
+            for (int q = 0; q < R; ++q) part[q] = 0.f;
+#pragma unroll 1
+            for (int b = 0; b < 4 && g + 4 * b < most; b += B) {
+                // a lane past its ray's last sample re-reads that sample (its result is masked); an
+                // empty ray has i0 = d = 0 and samples the grid origin
+                const int js = g + 4 * b + sub;
+#pragma unroll
+                for (int c = 0; c < B * R; ++c) f[c] = at((float)min(js + 4 * (c / R) + S * (c % R), cnt - 1));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int c = 0; c < B * R; ++c) part[c % R] += js + 4 * (c / R) + S * (c % R) < cnt ? fast_value<DT>(f[c]) : 0.f;
+            }
+#pragma unroll
+            for (int q = 0; q < R; ++q)
+                if (g < cnt) kahan_add(part[q], sum[q], nc[q]);
+        }
+        // the residues' Kahan totals, (0 + 1) + (2 + 3)
+        float res[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            res[q] = sum[q] + nc[q];
+            if constexpr (S > 1) {
+                const float t1 = __shfl_xor(res[q], sub_step, 64);
+                res[q] = (sub & 1) ? t1 + res[q] : res[q] + t1;
+            }
+        }
+        if constexpr (S == 1) tot = (res[0] + res[1]) + (res[2] + res[3]);
+        else if constexpr (S == 2) tot = res[0] + res[1];
+        else {
+            const float t2 = __shfl_xor(res[0], 2 * sub_step, 64);
+            tot = (sub & 2) ? t2 + res[0] : res[0] + t2;
         }
     }
+    // the step weight and the scale constant are applied once per ray (all in FP32)
     if (valid && sub == 0) P.out[(size_t)j * P.W + i] = (tot * P.w) * K;
 }
 
-// Work distribution: items (pose-major, tiles row-major) are split into 8 contiguous ranges, one
-// per XCD queue. Block b starts on queue b % 8 (dispatch places consecutive blocks on successive
-// XCDs, so a queue's tiles -- neighbouring rays of one image -- meet in one L2) and moves on to
-// the other queues when its own is drained. Every wave leaves after finding all 8 queues empty.
-// KV is a kernel variant (fast_kernel_dtype): the storage kernel in its low bits, plus
-// BIRP_KDT_SIGNED for volumes with values <= 0, whose rays stop at their first negative sample.
-// Each wave keeps its volume's offset tables in tab_stride words of dynamic LDS, sized per launch
-// to the largest table it reads: 768 words for a 256^3 cube, 1536 for 512^3. With the tables sized
-// so, six blocks fit a CU where fixed 2048-word tables let five (the F16 orbit batch: 2.69 -> 2.51
-// ms), and the launch bound keeps the registers within six waves per SIMD.
+// The wave tiles of many views in one launch, as a plain grid: a block renders 4 consecutive tiles of one view
+// (prefix[k] = first block of view k), its waves sharing the view's offset tables in LDS, and the
+// dispatcher balances the load. Blocks go round-robin over the 8 XCDs; block b renders item
+// (c * 8 + b % 8) * chunk + i, its c-th chunk: each XCD renders runs of `chunk` neighbouring blocks, whose
+// rays meet the same records in its L2, and a fair share of every view.
+// A persistent grid whose waves claimed tiles from 8 atomic queues took 20-80 us more per launch (every wave
+// visits all queues before it leaves, and claims on one address serialize): 16 FP16 views of 288x168 x 320
+// 154 -> 73 us, 16 of 576x336 x 800 556 -> 487 us, 256 mixed orbit views 2.37 -> 2.24 ms.
+// KV is a kernel variant (fast_kernel_dtype): the storage kernel in its low bits, plus BIRP_KDT_SIGNED for
+// volumes with negative values, whose rays stop at their first negative sample. Six waves per SIMD: the
+// register allocation meets that with 4 samples in flight.
+__device__ __forceinline__ void load_fast_tables(const DevVolume& V, bool f32, unsigned* tab, int entries) {
+    const unsigned* src = f32 ? V.qtab : V.otab;
+    const int n = min(V.nx + V.ny + V.nz, entries);  // the host sizes the LDS to cover it
+    for (int q = threadIdx.x; q < n; q += BIRP_BLOCK) tab[q] = src[q];
+    __syncthreads();
+}
+
+// The last k < n with prefix[k] <= g (prefix[0] = 0 <= g < prefix[n]), searched by the wave 64 entries at a time.
+__device__ __forceinline__ int find_view(const int* __restrict__ prefix, int n, int g) {
+    int lo = 0;
+    for (int step = n; step > 1;) {  // the answer is in [lo, lo + step)
+        const int hi = min(lo + step, n);
+        step = (step + 63) / 64;
+        const int k = lo + lane_id() * step;
+        const unsigned long long below = __ballot(k < hi && prefix[min(k, n)] <= g);
+        lo += (__popcll(below) - 1) * step;
+    }
+    return __builtin_amdgcn_readfirstlane(lo);
+}
+
 template <int KV, int S, int U>
 __global__ __launch_bounds__(BIRP_BLOCK, 6) void k_render_fast(const DevVolume* __restrict__ vols, const FastPose* __restrict__ poses,
-                                                               const int* __restrict__ prefix, int npose, int total,
-                                                               unsigned* counters, int tw_log2, int tab_stride) {
+                                                               const int* __restrict__ prefix, int npose, int total, int chunk,
+                                                               int tw_log2, int tab_entries) {
     constexpr bool CMEM = KV == BIRP_KDT_CMEM;
     constexpr int DT = CMEM ? BIRP_DTYPE_F32 : (KV & 3);
     constexpr bool SIGNED = CMEM || (KV & BIRP_KDT_SIGNED) != 0;
     static_assert(!SIGNED || U == 1, "signed kernels take one sample per lane per trip");
     extern __shared__ unsigned s_tab[];
-    const int lane = lane_id();
-    const int wave = threadIdx.x >> 6;
-    unsigned* tab = s_tab + wave * tab_stride;
-    const FastLane fl = fast_lane<S, SIGNED>(lane, tw_log2);
-    int cached_vol = -1;
-    int queue = blockIdx.x & 7;
-    for (int tried = 0; tried < 8;) {
-        const int q_lo = (int)(((long long)total * queue) >> 3), q_hi = (int)(((long long)total * (queue + 1)) >> 3);
-        int item = 0;
-        if (lane == 0) item = q_lo + (int)atomicAdd(&counters[queue * 32], 1u);
-        item = __builtin_amdgcn_readfirstlane(item);
-        if (item >= q_hi) {
-            queue = (queue + 1) & 7;
-            tried++;
-            continue;
-        }
-        // pose = last p with prefix[p] <= item
-        int lo = 0, hi = npose - 1;
-        while (lo < hi) {
-            int mid = (lo + hi + 1) >> 1;
-            if (prefix[mid] <= item) lo = mid; else hi = mid - 1;
-        }
-        const int pidx = __builtin_amdgcn_readfirstlane(lo);
-        const FastPose& P = poses[pidx];
-        const DevVolume& V = vols[P.vol];
-        if (!CMEM && P.vol != cached_vol) {
-            const unsigned* src = (DT == BIRP_DTYPE_F32) ? V.qtab : V.otab;
-            const int ntab = min(V.nx + V.ny + V.nz, tab_stride);  // the host sizes tab_stride to cover it
-            for (int q = lane; q < ntab; q += 64) tab[q] = src[q];
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            cached_vol = P.vol;
-        }
-        const int tile = item - prefix[pidx];
-        fast_tile<KV, S, U>(V, P, tile, tab, fl);
-    }
+    const int turn = (int)(blockIdx.x >> 3), g = (turn / chunk * 8 + (int)(blockIdx.x & 7u)) * chunk + turn % chunk;
+    if (g >= total) return;
+    const int k = find_view(prefix, npose, g);
+    const FastPose& P = poses[k];
+    const DevVolume& V = vols[P.vol];
+    if constexpr (!CMEM) load_fast_tables(V, DT == BIRP_DTYPE_F32, s_tab, tab_entries);
+    const FastLane fl = fast_lane<S, SIGNED>(lane_id(), tw_log2);
+    const int tile = (g - prefix[k]) * (BIRP_BLOCK / 64) + (int)(threadIdx.x >> 6);
+    if (tile < P.tiles_x * ((P.H + fl.th - 1) / fl.th)) fast_tile<KV, S, U>(V, P, tile, s_tab, fl);
 }
 
 // One pose as a plain grid, with the pose and its volume by value: the launch needs no descriptor
-// upload and no work counters (single fast renders, a lone served request). Wave w of block b
-// renders tile 4 b' + w, where blocks go round-robin over the 8 XCDs and b' numbers them XCD by
-// XCD, so that each XCD renders a contiguous range of neighbouring tiles, as the work queues of
-// k_render_fast do. The grid is a multiple of 8 blocks; waves past the last tile leave at once.
+// upload (single fast renders, a lone served request). All its blocks run at once, so each XCD renders one
+// contiguous range of neighbouring tiles: its L2 then fetches each record once (with the blocks dealt out
+// one by one every XCD misses on nearly every record: 20-40% slower). The grid is a multiple of 8
+// blocks; waves past the last tile leave at once.
 template <int KV, int S, int U>
-__global__ __launch_bounds__(BIRP_BLOCK, 6) void k_render_fast_one(DevVolume V, FastPose P, int total, int tw_log2, int tab_stride) {
+__global__ __launch_bounds__(BIRP_BLOCK, 6) void k_render_fast_one(DevVolume V, FastPose P, int total, int tw_log2, int tab_entries) {
     constexpr bool CMEM = KV == BIRP_KDT_CMEM;
     constexpr int DT = CMEM ? BIRP_DTYPE_F32 : (KV & 3);
     constexpr bool SIGNED = CMEM || (KV & BIRP_KDT_SIGNED) != 0;
     static_assert(!SIGNED || U == 1, "signed kernels take one sample per lane per trip");
     extern __shared__ unsigned s_tab[];
-    const int lane = lane_id();
-    const int wave = threadIdx.x >> 6;
     const int b = (int)(blockIdx.x & 7u) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
-    const int item = b * (BIRP_BLOCK / 64) + wave;
+    const int item = b * (BIRP_BLOCK / 64) + (int)(threadIdx.x >> 6);
+    if constexpr (!CMEM) load_fast_tables(V, DT == BIRP_DTYPE_F32, s_tab, tab_entries);
     if (item >= total) return;
-    unsigned* tab = s_tab + wave * tab_stride;
-    if constexpr (!CMEM) {
-        const unsigned* src = (DT == BIRP_DTYPE_F32) ? V.qtab : V.otab;
-        const int ntab = min(V.nx + V.ny + V.nz, tab_stride);  // the host sizes tab_stride to cover it
-        for (int q = lane; q < ntab; q += 64) tab[q] = src[q];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    fast_tile<KV, S, U>(V, P, item, tab, fast_lane<S, SIGNED>(lane, tw_log2));
+    fast_tile<KV, S, U>(V, P, item, s_tab, fast_lane<S, SIGNED>(lane_id(), tw_log2));
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1814,7 +1864,7 @@ static __device__ __align__(256) unsigned char scratch[BIRP_NOALLOC_SCRATCH_BYTE
 static_assert(sizeof(DevVolume) <= BIRP_NOALLOC_POSE_OFF, "noalloc scratch: volume slot");
 static_assert(BIRP_NOALLOC_SCRATCH_BYTES <= BIRP_NOALLOC_SCRATCH_KIB * 1024, "noalloc scratch: stated size");
 static_assert(sizeof(FastPose) <= 256, "noalloc scratch: pose slot");
-static_assert(3 * (BIRP_NOALLOC_MAX_VIEWS + 1) * 4 <= BIRP_NOALLOC_CTR_OFF - BIRP_NOALLOC_PREFIX_OFF, "noalloc scratch: prefix");
+static_assert(3 * (BIRP_NOALLOC_MAX_VIEWS + 1) * 4 <= BIRP_NOALLOC_SCRATCH_BYTES - BIRP_NOALLOC_PREFIX_OFF, "noalloc scratch: prefix");
 
 struct NoallocHead {
     DevVolume v;
@@ -1829,8 +1879,6 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_noalloc_head(NoallocHead h, unsi
     if (threadIdx.x == 0) *reinterpret_cast<DevVolume*>(s) = h.v;
     int* pre = reinterpret_cast<int*>(s + BIRP_NOALLOC_PREFIX_OFF);
     for (int i = threadIdx.x; i < 3 * (BIRP_NOALLOC_MAX_VIEWS + 1); i += BIRP_BLOCK) pre[i] = h.prefix[i];
-    unsigned* ctr = reinterpret_cast<unsigned*>(s + BIRP_NOALLOC_CTR_OFF);
-    for (int i = threadIdx.x; i < 3 * 256; i += BIRP_BLOCK) ctr[i] = 0u;
 }
 
 __global__ void k_noalloc_poses(NoallocPoses c, unsigned char* s) {
@@ -2104,11 +2152,6 @@ int launch_build_oct(const DevVolume& v, void* oct, float* bscale, void* stream)
     return hip_status(hipGetLastError());
 }
 
-int launch_reset_counter(unsigned* counter, void* stream) {
-    hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(256), 0, (hipStream_t)stream, counter);
-    return hip_status(hipGetLastError());
-}
-
 int launch_zero_f32(float* p, size_t n, void* stream) {
     size_t blocks = (n + BIRP_BLOCK - 1) / BIRP_BLOCK;
     if (blocks > 4096) blocks = 4096;
@@ -2117,152 +2160,73 @@ int launch_zero_f32(float* p, size_t n, void* stream) {
     return hip_status(hipGetLastError());
 }
 
-template <int DT, int S, int U>
-static void* fast_kernel_ptr() { return (void*)k_render_fast<DT, S, U>; }
-
-template <int DT, int S>
-static int launch_fast_su(int unroll, int grid, hipStream_t st, const DevVolume* vols, const FastPose* poses, const int* prefix,
-                          int npose, int total, unsigned* counter, int twl, int ts) {
-    const size_t lds = (size_t)(BIRP_BLOCK / 64) * ts * sizeof(unsigned);
-    if constexpr ((DT & (BIRP_KDT_SIGNED | BIRP_KDT_CMEM)) != 0) {
-        hipLaunchKernelGGL((k_render_fast<DT, S, 1>), dim3(grid), dim3(BIRP_BLOCK), lds, st, vols, poses, prefix, npose, total, counter, twl, ts);
-    } else {
-        switch (unroll) {
-            case 4: hipLaunchKernelGGL((k_render_fast<DT, S, 4>), dim3(grid), dim3(BIRP_BLOCK), lds, st, vols, poses, prefix, npose, total, counter, twl, ts); break;
-            case 2: hipLaunchKernelGGL((k_render_fast<DT, S, 2>), dim3(grid), dim3(BIRP_BLOCK), lds, st, vols, poses, prefix, npose, total, counter, twl, ts); break;
-            default: hipLaunchKernelGGL((k_render_fast<DT, S, 1>), dim3(grid), dim3(BIRP_BLOCK), lds, st, vols, poses, prefix, npose, total, counter, twl, ts); break;
-        }
-    }
-    return hip_status(hipGetLastError());
+// U as the kernels take it: the signed and CMEM kernels one sample per lane per trip, the others at least a
+// lane's 4 / S residues.
+template <int KV, int S, int U>
+constexpr int fast_unroll() {
+    return (KV & (BIRP_KDT_SIGNED | BIRP_KDT_CMEM)) ? 1 : (U > 4 / S ? U : 4 / S);
 }
 
-template <int DT>
-static int launch_fast_d(int S, int unroll, int grid, hipStream_t st, const DevVolume* vols, const FastPose* poses,
-                         const int* prefix, int npose, int total, unsigned* counter, int twl, int ts) {
-    if (S == 4) return launch_fast_su<DT, 4>(unroll, grid, st, vols, poses, prefix, npose, total, counter, twl, ts);
-    if (S == 2) return launch_fast_su<DT, 2>(unroll, grid, st, vols, poses, prefix, npose, total, counter, twl, ts);
-    return launch_fast_su<DT, 1>(unroll, grid, st, vols, poses, prefix, npose, total, counter, twl, ts);
+// Calls launch(std::integral_constant KV, S, U) for the variant asked for.
+template <int KV, int S, class F>
+static int with_unroll(int u, F&& launch) {
+    if (u == 4) return launch(std::integral_constant<int, KV>(), std::integral_constant<int, S>(), std::integral_constant<int, fast_unroll<KV, S, 4>()>());
+    if (u == 2) return launch(std::integral_constant<int, KV>(), std::integral_constant<int, S>(), std::integral_constant<int, fast_unroll<KV, S, 2>()>());
+    return launch(std::integral_constant<int, KV>(), std::integral_constant<int, S>(), std::integral_constant<int, fast_unroll<KV, S, 1>()>());
 }
-
-int fast_tab_stride(int dtype, int tab_entries) {
-    if (dtype == BIRP_KDT_CMEM) return 0;  // the model has no tables
-    return ((std::max(tab_entries, 1) + 255) / 256) * 256;
+template <int KV, class F>
+static int with_lanes(int s, int u, F&& launch) {
+    return s == 4 ? with_unroll<KV, 4>(u, launch) : s == 2 ? with_unroll<KV, 2>(u, launch) : with_unroll<KV, 1>(u, launch);
 }
-
-// counters: 256 unsigned (8 queues, 128 B apart), reset by launch_reset_counter before each launch.
-int launch_fast_batch(const DevVolume* vols_dev, int dtype, const FastPose* poses_dev, const int* tile_prefix_dev, int npose,
-                      int total_tiles, unsigned* work_counter, int tile_w, int tile_h, int lanes_per_ray, int unroll,
-                      int grid, void* stream, int tab_entries) {
-    int twl = 0;
-    while ((1 << twl) < tile_w) twl++;
-    if ((1 << twl) != tile_w || tile_w * tile_h * lanes_per_ray != 64) return BIRP_ERR_INVALID_ARGUMENT;
-    if (dtype < 0 || dtype >= BIRP_KDT_COUNT) return BIRP_ERR_INVALID_ARGUMENT;
-    if (tab_entries < 0 || tab_entries > BIRP_FAST_TAB) return BIRP_ERR_INVALID_ARGUMENT;
-    const int ts = fast_tab_stride(dtype, tab_entries);
-    grid = ((grid + 7) / 8) * 8;
-    hipStream_t st = (hipStream_t)stream;
-    if (dtype & (BIRP_KDT_SIGNED | BIRP_KDT_CMEM)) unroll = 1;  // the signed and CMEM kernels take one sample per lane per trip
-#define BIRP_LFD(KV) \
-    case KV: return launch_fast_d<KV>(lanes_per_ray, unroll, grid, st, vols_dev, poses_dev, tile_prefix_dev, npose, total_tiles, work_counter, twl, ts);
+template <class F>
+static int with_variant(int dtype, int s, int u, F&& launch) {
     switch (dtype) {
-        BIRP_LFD(0) BIRP_LFD(1) BIRP_LFD(2) BIRP_LFD(3) BIRP_LFD(4) BIRP_LFD(5) BIRP_LFD(6) BIRP_LFD(7) BIRP_LFD(8)
+        case 0: return with_lanes<0>(s, u, launch);
+        case 1: return with_lanes<1>(s, u, launch);
+        case 2: return with_lanes<2>(s, u, launch);
+        case 3: return with_lanes<3>(s, u, launch);
+        case 4: return with_lanes<4>(s, u, launch);
+        case 5: return with_lanes<5>(s, u, launch);
+        case 6: return with_lanes<6>(s, u, launch);
+        case 7: return with_lanes<7>(s, u, launch);
+        case 8: return with_lanes<8>(s, u, launch);
         default: return BIRP_ERR_INVALID_ARGUMENT;
     }
-#undef BIRP_LFD
 }
 
-template <int DT, int S>
-static int launch_one_su(int unroll, int grid, hipStream_t st, const DevVolume& v, const FastPose& p, int total, int twl, int ts) {
-    const size_t lds = (size_t)(BIRP_BLOCK / 64) * ts * sizeof(unsigned);
-    if constexpr ((DT & (BIRP_KDT_SIGNED | BIRP_KDT_CMEM)) != 0) {
-        hipLaunchKernelGGL((k_render_fast_one<DT, S, 1>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, p, total, twl, ts);
-    } else {
-        switch (unroll) {
-            case 4: hipLaunchKernelGGL((k_render_fast_one<DT, S, 4>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, p, total, twl, ts); break;
-            case 2: hipLaunchKernelGGL((k_render_fast_one<DT, S, 2>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, p, total, twl, ts); break;
-            default: hipLaunchKernelGGL((k_render_fast_one<DT, S, 1>), dim3(grid), dim3(BIRP_BLOCK), lds, st, v, p, total, twl, ts); break;
-        }
-    }
-    return hip_status(hipGetLastError());
+// log2 of the tile's width, or -1 for a tile and lanes that do not make a wave
+static int tile_log2(int tile_w, int tile_h, int lanes_per_ray) {
+    int twl = 0;
+    while ((1 << twl) < tile_w) twl++;
+    return (1 << twl) == tile_w && tile_w * tile_h * lanes_per_ray == 64 ? twl : -1;
 }
+static size_t fast_lds_bytes(int dtype, int tab_entries) { return dtype == BIRP_KDT_CMEM ? 0 : (size_t)tab_entries * sizeof(unsigned); }
 
-template <int DT>
-static int launch_one_d(int S, int unroll, int grid, hipStream_t st, const DevVolume& v, const FastPose& p, int total, int twl, int ts) {
-    if (S == 4) return launch_one_su<DT, 4>(unroll, grid, st, v, p, total, twl, ts);
-    if (S == 2) return launch_one_su<DT, 2>(unroll, grid, st, v, p, total, twl, ts);
-    return launch_one_su<DT, 1>(unroll, grid, st, v, p, total, twl, ts);
+int launch_fast_batch(const DevVolume* vols_dev, int dtype, const FastPose* poses_dev, const int* block_prefix_dev, int npose,
+                      int total_blocks, int tile_w, int tile_h, int lanes_per_ray, int unroll, void* stream, int tab_entries) {
+    const int twl = tile_log2(tile_w, tile_h, lanes_per_ray);
+    if (twl < 0 || npose < 1 || total_blocks < 1 || tab_entries < 0 || tab_entries > BIRP_FAST_TAB) return BIRP_ERR_INVALID_ARGUMENT;
+    const int chunk = 16;  // 4 to 64 measured within 2% of each other, 1 up to 5% slower on small views
+    const long long grid = ((long long)total_blocks + 8 * chunk - 1) / (8 * chunk) * (8 * chunk);
+    if (grid > INT32_MAX) return BIRP_ERR_UNSUPPORTED;
+    return with_variant(dtype, lanes_per_ray, unroll, [&](auto kv, auto s, auto u) {
+        hipLaunchKernelGGL((k_render_fast<kv.value, s.value, u.value>), dim3((unsigned)grid), dim3(BIRP_BLOCK), fast_lds_bytes(dtype, tab_entries),
+                           (hipStream_t)stream, vols_dev, poses_dev, block_prefix_dev, npose, total_blocks, chunk, twl, tab_entries);
+        return hip_status(hipGetLastError());
+    });
 }
 
 int launch_fast_one(const DevVolume& v, int dtype, const FastPose& pose, int total_tiles, int tile_w, int tile_h, int lanes_per_ray,
                     int unroll, void* stream, int tab_entries) {
-    int twl = 0;
-    while ((1 << twl) < tile_w) twl++;
-    if ((1 << twl) != tile_w || tile_w * tile_h * lanes_per_ray != 64) return BIRP_ERR_INVALID_ARGUMENT;
-    if (dtype < 0 || dtype >= BIRP_KDT_COUNT) return BIRP_ERR_INVALID_ARGUMENT;
-    if (tab_entries < 0 || tab_entries > BIRP_FAST_TAB || total_tiles < 0) return BIRP_ERR_INVALID_ARGUMENT;
+    const int twl = tile_log2(tile_w, tile_h, lanes_per_ray);
+    if (twl < 0 || tab_entries < 0 || tab_entries > BIRP_FAST_TAB || total_tiles < 0) return BIRP_ERR_INVALID_ARGUMENT;
     if (total_tiles == 0) return BIRP_OK;
-    const int ts = fast_tab_stride(dtype, tab_entries);
-    const int blocks = (int)(((long long)total_tiles + BIRP_BLOCK / 64 - 1) / (BIRP_BLOCK / 64));
-    const int grid = ((blocks + 7) / 8) * 8;
-    hipStream_t st = (hipStream_t)stream;
-    if (dtype & (BIRP_KDT_SIGNED | BIRP_KDT_CMEM)) unroll = 1;  // the signed and CMEM kernels take one sample per lane per trip
-#define BIRP_LOD(KV) \
-    case KV: return launch_one_d<KV>(lanes_per_ray, unroll, grid, st, v, pose, total_tiles, twl, ts);
-    switch (dtype) {
-        BIRP_LOD(0) BIRP_LOD(1) BIRP_LOD(2) BIRP_LOD(3) BIRP_LOD(4) BIRP_LOD(5) BIRP_LOD(6) BIRP_LOD(7) BIRP_LOD(8)
-        default: return BIRP_ERR_INVALID_ARGUMENT;
-    }
-#undef BIRP_LOD
-}
-
-int fast_grid_for(int dtype, int lanes_per_ray, int unroll, int tiles, int tab_entries) {
-    // back-to-back single renders with the tuned tiles: 576x336 at n = 800 took 0.10-0.11 ms per
-    // render at one tile per wave, 0.12-0.13 ms at two waves per tile or on the full grid; 144x84
-    // at n = 160 took 0.033-0.036 ms against 0.086 ms on the full grid
-    return std::min(fast_grid_size(dtype, lanes_per_ray, unroll, tab_entries), (tiles + 3) / 4 + 1);
-}
-
-int fast_grid_size(int dtype, int lanes_per_ray, int unroll, int tab_entries) {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    // cached per device, kernel variant and table size: the occupancy query costs microseconds
-    if (dtype & (BIRP_KDT_SIGNED | BIRP_KDT_CMEM)) unroll = 1;
-    const int ts = fast_tab_stride(dtype, std::min(std::max(tab_entries, 0), BIRP_FAST_TAB));
-    const int tsb = ts / 256;  // 0..8
-    static std::atomic<int> cache[16][BIRP_KDT_COUNT][5][5][BIRP_FAST_TAB / 256 + 1];
-    const bool cacheable = dev >= 0 && dev < 16 && dtype >= 0 && dtype < BIRP_KDT_COUNT && lanes_per_ray <= 4 && unroll <= 4;
-    if (cacheable) {
-        const int c = cache[dev][dtype][lanes_per_ray][unroll][tsb].load(std::memory_order_relaxed);
-        if (c > 0) return c;
-    }
-    int cus = 0;
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (cus <= 0) cus = 256;
-    int per_cu = 0;
-    void* fn = nullptr;
-#define BIRP_FK(DT)                                                                          \
-    if (lanes_per_ray == 4) fn = unroll == 4 ? fast_kernel_ptr<DT, 4, 4>() : unroll == 2 ? fast_kernel_ptr<DT, 4, 2>() : fast_kernel_ptr<DT, 4, 1>(); \
-    else if (lanes_per_ray == 2) fn = unroll == 4 ? fast_kernel_ptr<DT, 2, 4>() : unroll == 2 ? fast_kernel_ptr<DT, 2, 2>() : fast_kernel_ptr<DT, 2, 1>(); \
-    else fn = unroll == 4 ? fast_kernel_ptr<DT, 1, 4>() : unroll == 2 ? fast_kernel_ptr<DT, 1, 2>() : fast_kernel_ptr<DT, 1, 1>();
-#define BIRP_FKS(DT) \
-    fn = lanes_per_ray == 4 ? fast_kernel_ptr<DT, 4, 1>() : lanes_per_ray == 2 ? fast_kernel_ptr<DT, 2, 1>() : fast_kernel_ptr<DT, 1, 1>();
-    switch (dtype) {
-        case 3: BIRP_FK(3) break;
-        case 2: BIRP_FK(2) break;
-        case 1: BIRP_FK(1) break;
-        case 4: BIRP_FKS(4) break;
-        case 5: BIRP_FKS(5) break;
-        case 6: BIRP_FKS(6) break;
-        case 7: BIRP_FKS(7) break;
-        case 8: BIRP_FKS(8) break;
-        default: BIRP_FK(0) break;
-    }
-#undef BIRP_FKS
-#undef BIRP_FK
-    const size_t lds = (size_t)(BIRP_BLOCK / 64) * ts * sizeof(unsigned);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, BIRP_BLOCK, lds) != hipSuccess || per_cu <= 0) per_cu = 4;
-    if (cacheable) cache[dev][dtype][lanes_per_ray][unroll][tsb].store(cus * per_cu, std::memory_order_relaxed);
-    return cus * per_cu;
+    const int blocks = fast_blocks(total_tiles), grid = (blocks + 7) / 8 * 8;
+    return with_variant(dtype, lanes_per_ray, unroll, [&](auto kv, auto s, auto u) {
+        hipLaunchKernelGGL((k_render_fast_one<kv.value, s.value, u.value>), dim3(grid), dim3(BIRP_BLOCK), fast_lds_bytes(dtype, tab_entries),
+                           (hipStream_t)stream, v, pose, total_tiles, twl, tab_entries);
+        return hip_status(hipGetLastError());
+    });
 }
 
 }  // namespace birp

@@ -7,16 +7,16 @@
 // batches). Requests queue on submission; whenever a slot is free the
 // dispatcher admits queued requests in arrival order while the slot's image buffer can hold them,
 // or can grow to hold them within the budget (releasing idle slots' buffers when that makes the
-// room), and launches them as one persistent-kernel batch (one launch per storage type and lanes
+// room), and launches them as one batch (one launch per storage type and lanes
 // per ray). A request that arrives while other batches are on the GPU is launched in the next
 // free slot, so its work overlaps theirs on the device. A result buffer from birp_host_alloc is
 // written by the kernel itself through its device address, the other images into the slot's
 // pinned staging the same way, and when a slot's device work is done a completion thread copies
 // those into the callers' buffers (split over a pool of helper threads for large batches) and
 // releases the slot, so the dispatcher keeps launching meanwhile.
-// Every request in BIRP_MATH_FAST is rendered with the tuning its own view selects (the one fast
-// single renders use) and the same per-tile arithmetic whatever it is batched with, so results do
-// not depend on the mix and equal birp_render's. Requests in BIRP_MATH_EXACT (FP32 cubes of any
+// A request in BIRP_MATH_FAST renders the same whatever it is batched with, and as birp_render: over a
+// signed cube or a CMEM model with the tuning its own view selects, over other cubes with the launch's,
+// on which their images do not depend. Requests in BIRP_MATH_EXACT (FP32 cubes of any
 // interpolation and sign, CMEM models) render with the exact arithmetic through the multi-view
 // exact kernel, one launch per sample mode in the same slot, and equal birp_render's exact images
 // bit for bit.
@@ -179,15 +179,13 @@ private:
 };
 
 // A launch's descriptors live in one block, pinned on the host and mirrored on the device, and go
-// to the device in one copy (desc_layout): the work-queue counters first, kept zero on the host so
-// that the copy resets them, then the tile prefix sums, the fast poses and the exact views, each
+// to the device in one copy (desc_layout): the prefix sums, the fast poses and the exact views, each
 // region sized for the launch's requests.
 struct Slot {
     hipStream_t stream = nullptr;
     hipEvent_t done = nullptr;
     unsigned char* h_desc = nullptr;  // pinned descriptor block, sized for max_batch requests
     unsigned char* d_desc = nullptr;  // its device copy
-    unsigned* d_work = nullptr;       // work-queue counters, 256 per kernel group, at d_desc
     // this launch's regions in h_desc / d_desc
     FastPose* h_poses = nullptr;  // poses packed by kernel group
     FastPose* d_poses = nullptr;
@@ -273,35 +271,36 @@ int slot_alloc_images(Slot& s, size_t pixels) {
     return BIRP_OK;
 }
 
-// Kernel groups of a batch: storage kernel x lanes per ray (1, 2, 4). Every request's tuning comes
-// from its own view (latency_tuning), so a group has one tuning and a request renders the same
-// whatever shares its launch.
+// Kernel groups of a batch: storage kernel x lanes per ray (1, 2, 4). A request over a signed cube or a CMEM
+// model has its tuning from its own view (view_tuning), so that it renders the same whatever shares its
+// launch; the others' images do not depend on the tuning, and all of a storage kernel are one group
+// (lane index 0) tuned for its rays (launch_tuning).
 constexpr int kGroups = BIRP_KDT_COUNT * 3;
 int lane_index(int lanes) { return lanes == 4 ? 2 : (lanes == 2 ? 1 : 0); }
 int request_group(const Request* r, birp_tuning* t) {
-    *t = latency_tuning(r->req.view, r->vol->dv);
-    return fast_kernel_dtype(r->vol->dv) * 3 + lane_index(t->lanes_per_ray);
+    const int kdt = fast_kernel_dtype(r->vol->dv);
+    if (tuning_is_free(kdt)) return kdt * 3;
+    *t = view_tuning(r->req.view, r->vol->dv);
+    return kdt * 3 + lane_index(t->lanes_per_ray);
 }
 // Requests in BIRP_MATH_EXACT render with the exact arithmetic of birp_render through the
 // multi-view exact kernel, one launch per sample mode present; the others take the fast kernels.
 bool exact_request(const Request* r) { return r->req.view.math == BIRP_MATH_EXACT; }
 constexpr int kModes = SM_CMEM + 1;
-constexpr size_t kCounterBytes = sizeof(unsigned) * kGroups * 256;
 
 // Offsets of a launch's descriptor regions for n fast and nexact exact requests, 256-byte aligned,
-// and the span that one copy uploads: the counters only when fast requests use them.
+// and the span that one copy uploads.
 struct DescLayout {
-    size_t prefix, eprefix, poses, evs, lo, hi;
+    size_t prefix, eprefix, poses, evs, hi;
 };
 DescLayout desc_layout(int n, int nexact) {
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     DescLayout L;
-    L.prefix = kCounterBytes;
+    L.prefix = 0;
     L.eprefix = L.prefix + up(sizeof(int) * (n + kGroups));
     L.poses = L.eprefix + up(sizeof(int) * (nexact + kModes));
     L.evs = L.poses + up(sizeof(FastPose) * n);
     L.hi = L.evs + up(sizeof(ExactView) * nexact);
-    L.lo = n ? 0 : L.prefix;
     return L;
 }
 
@@ -318,12 +317,14 @@ int launch_slot(birp_server* S, Slot& s) {
     if (rc) return rc;
     int base[kGroups + 1] = {}, fill[kGroups];
     birp_tuning gt[kGroups];
+    long long rays[kGroups] = {};
     for (Request* r : s.reqs) {
         if (exact_request(r)) continue;
-        birp_tuning t;
+        birp_tuning t{};
         const int g = request_group(r, &t);
         base[g + 1]++;
-        gt[g] = t;
+        rays[g] += (long long)r->req.view.width * r->req.view.height;
+        gt[g] = tuning_is_free(g / 3) ? launch_tuning(rays[g]) : t;
     }
     for (int g = 0; g < kGroups; g++) {
         base[g + 1] += base[g];
@@ -401,6 +402,7 @@ int launch_slot(birp_server* S, Slot& s) {
         }
         birp_tuning t;
         const int g = request_group(r, &t);
+        t = gt[g];
         tabs[g] = std::max(tabs[g], volume_tab_entries(r->vol->dv));
         rc = fast_pose(r->vol, &r->req.view, r->req.volume, out, t.tile_w, t.tile_h, s.h_poses[fill[g]++]);
         if (rc) return rc;
@@ -412,7 +414,7 @@ int launch_slot(birp_server* S, Slot& s) {
             birp_view tmp{};
             tmp.width = s.h_poses[k].W;
             tmp.height = s.h_poses[k].H;
-            const long long next = (long long)pre[k - base[g]] + tiles_of(tmp, gt[g].tile_w, gt[g].tile_h);
+            const long long next = (long long)pre[k - base[g]] + fast_blocks(tiles_of(tmp, gt[g].tile_w, gt[g].tile_h));
             if (next > INT32_MAX) return fail(BIRP_ERR_UNSUPPORTED, "launch of more than 2^31 - 1 tiles");
             pre[k - base[g] + 1] = (int)next;
         }
@@ -430,7 +432,7 @@ int launch_slot(birp_server* S, Slot& s) {
     }
     hipError_t e = hipSuccess;
     if ((n && !lone_fast) || (nexact && !lone))
-        e = hipMemcpyAsync(s.d_desc + L.lo, s.h_desc + L.lo, L.hi - L.lo, hipMemcpyHostToDevice, s.stream);
+        e = hipMemcpyAsync(s.d_desc, s.h_desc, L.hi, hipMemcpyHostToDevice, s.stream);
     if (e != hipSuccess) return hip_fail(e, "server descriptor upload");
     if (lone) {
         const DevVolume& dv = lone->vol->dv;
@@ -450,16 +452,15 @@ int launch_slot(birp_server* S, Slot& s) {
         if (!count) continue;
         const birp_tuning& t = gt[g];
         const int kdt = g / 3;
-        const int total_tiles = s.h_prefix[base[g] + g + count];
+        const int total_blocks = s.h_prefix[base[g] + g + count];
         if (lone_fast) {
-            rc = launch_fast_one(lone_fast->vol->dv, kdt, s.h_poses[base[g]], total_tiles, t.tile_w, t.tile_h, t.lanes_per_ray,
+            rc = launch_fast_one(lone_fast->vol->dv, kdt, s.h_poses[base[g]], tiles_of(lone_fast->req.view, t.tile_w, t.tile_h), t.tile_w, t.tile_h, t.lanes_per_ray,
                                  t.unroll, s.stream, tabs[g]);
             if (rc) return fail(rc, "fast launch failed");
             continue;
         }
-        const int grid = fast_grid_for(kdt, t.lanes_per_ray, t.unroll, total_tiles, tabs[g]);
-        rc = launch_fast_batch(S->d_vols, kdt, s.d_poses + base[g], s.d_prefix + base[g] + g, count, total_tiles, s.d_work + g * 256,
-                               t.tile_w, t.tile_h, t.lanes_per_ray, t.unroll, grid, s.stream, tabs[g]);
+        rc = launch_fast_batch(S->d_vols, kdt, s.d_poses + base[g], s.d_prefix + base[g] + g, count, total_blocks, t.tile_w, t.tile_h,
+                               t.lanes_per_ray, t.unroll, s.stream, tabs[g]);
         if (rc) return rc;
     }
     // without a mapped staging, the other results come back to it in one DMA; the completion thread
@@ -702,8 +703,6 @@ extern "C" int birp_server_create(birp_device* dev, const birp_server_config* cf
         const size_t bytes = desc_layout(nb, nb).hi;
         if ((e = hipHostMalloc(&s.h_desc, bytes, hipHostMallocDefault)) != hipSuccess) { rc = hip_fail(e, "pinned"); break; }
         if ((e = hipMalloc(&s.d_desc, bytes)) != hipSuccess) { rc = hip_fail(e, "descriptors"); break; }
-        memset(s.h_desc, 0, kCounterBytes);  // the counters stay zero on the host
-        s.d_work = (unsigned*)s.d_desc;
         if (cfg->reserve_pixels) {
             if ((rc = slot_alloc_images(s, cfg->reserve_pixels))) break;
             s.held = cfg->reserve_pixels * 4;
