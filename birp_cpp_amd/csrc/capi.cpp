@@ -569,18 +569,17 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
         d.otab = v->otab;
         d.oct_bytes = (unsigned)oct_bytes;
         d.bscale = v->bscale;
-        if (desc->dtype == BIRP_DTYPE_F16) {
-            // One power-of-two scale for the whole volume when every nonzero |v| then lands in
-            // F16's normal range [2^-14, 2^15): no per-sample scale lookup in the kernel.
-            double s = 1.0;
-            if (d.vmax > 0.f) {
-                int ex = 0;
-                std::frexp((double)d.vmax, &ex);  // vmax = f * 2^ex, f in [0.5, 1)
-                s = std::ldexp(1.0, ex - 15);     // vmax / s < 2^15
-            }
-            d.f16_uniform = (d.vmax == 0.f || (double)d.vmin / s >= 0x1p-14) && s >= 0x1p-126 && s <= 0x1p120;
-            d.f16_scale = d.f16_uniform ? (float)s : 1.f;
+        // One power-of-two scale for the whole volume when every nonzero |v| then lands in F16's normal
+        // range [2^-14, 2^15): no per-sample scale lookup in the kernel. BF16 values (8 significant bits) are
+        // then exact in F16 too, and their records hold them as F16, whose x-lerps need no conversions.
+        double s = 1.0;
+        if (d.vmax > 0.f) {
+            int ex = 0;
+            std::frexp((double)d.vmax, &ex);  // vmax = f * 2^ex, f in [0.5, 1)
+            s = std::ldexp(1.0, ex - 15);     // vmax / s < 2^15
         }
+        d.f16_uniform = (d.vmax == 0.f || (double)d.vmin / s >= 0x1p-14) && s >= 0x1p-126 && s <= 0x1p120;
+        d.f16_scale = d.f16_uniform ? (float)s : 1.f;
         if ((rc = launch_build_oct(d, v->oct, v->bscale, dev->stream)) != BIRP_OK) goto fail_out;
     }
     if ((e = hipStreamSynchronize(dev->stream)) != hipSuccess) { rc = hip_fail(e, "layout build"); goto fail_out; }

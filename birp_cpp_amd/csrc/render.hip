@@ -1354,8 +1354,10 @@ __device__ __forceinline__ unsigned short f32_to_f16_bits(float x) {
 }
 
 // F16 records hold v / scale, a power of two per brick: max|v| over the brick's corners maps to < 2^15. With
-// v.f16_uniform every brick gets the volume's scale v.f16_scale instead.
-template <bool F16>
+// v.f16_uniform every brick gets the volume's scale v.f16_scale instead, and BF16 volumes hold their
+// values, rounded to BF16, as F16 too (exactly).
+enum OctForm { OCT_BF16, OCT_F16, OCT_BF16_AS_F16 };
+template <int FORM>
 __global__ __launch_bounds__(BIRP_BLOCK) void k_build_oct(DevVolume v, unsigned char* oct, float* bscale) {
     __shared__ float s[kTileX * 9 * 9];
     int bx, by, bz;
@@ -1364,8 +1366,8 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_build_oct(DevVolume v, unsigned 
     const int w = threadIdx.x >> 6;  // one wave per brick
     if (bx + w >= v.nbx) return;
     const unsigned base = v.otab[(bx + w) * 8] + v.otab[v.nx + by * 8] + v.otab[v.nx + v.ny + bz * 8];
-    float inv = 1.f;
-    if constexpr (F16) {
+    float inv = FORM == OCT_BF16_AS_F16 ? 1.f / v.f16_scale : 1.f;  // powers of two: exact
+    if constexpr (FORM == OCT_F16) {
         float scale = v.f16_scale;
         if (!v.f16_uniform) {
             float m = 0.f;
@@ -1379,7 +1381,7 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_build_oct(DevVolume v, unsigned 
             }
         }
         if (lane_id() == 0) bscale[base >> 13] = scale;
-        inv = 1.f / scale;  // power of two: exact
+        inv = 1.f / scale;
     }
     for (int r = lane_id(); r < 512; r += 64) {
         const float* c0 = s + brick_cell(w, r);
@@ -1387,7 +1389,10 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_build_oct(DevVolume v, unsigned 
         const float c[8] = {c0[0], c0[1], c0[kTileX], c0[kTileX + 1], c1[0], c1[1], c1[kTileX], c1[kTileX + 1]};
         unsigned short h[8];
 #pragma unroll
-        for (int q = 0; q < 8; q++) h[q] = F16 ? f32_to_f16_bits(c[q] * inv) : f32_to_bf16_bits(c[q]);
+        for (int q = 0; q < 8; q++) {
+            const unsigned short b = f32_to_bf16_bits(c[q]);
+            h[q] = FORM == OCT_F16 ? f32_to_f16_bits(c[q] * inv) : FORM == OCT_BF16 ? b : f32_to_f16_bits(__uint_as_float((unsigned)b << 16) * inv);
+        }
         uint4 o;
         o.x = (unsigned)h[0] | ((unsigned)h[1] << 16);
         o.y = (unsigned)h[2] | ((unsigned)h[3] << 16);
@@ -2153,10 +2158,8 @@ int launch_build_quad(const DevVolume& v, void* quad, void* stream) {
 
 int launch_build_oct(const DevVolume& v, void* oct, float* bscale, void* stream) {
     const dim3 grid(brick_row_grid(v, v.nbz));
-    if (v.dtype == BIRP_DTYPE_F16)
-        hipLaunchKernelGGL((k_build_oct<true>), grid, dim3(BIRP_BLOCK), 0, (hipStream_t)stream, v, (unsigned char*)oct, bscale);
-    else
-        hipLaunchKernelGGL((k_build_oct<false>), grid, dim3(BIRP_BLOCK), 0, (hipStream_t)stream, v, (unsigned char*)oct, bscale);
+    auto kernel = v.dtype == BIRP_DTYPE_F16 ? k_build_oct<OCT_F16> : v.f16_uniform ? k_build_oct<OCT_BF16_AS_F16> : k_build_oct<OCT_BF16>;
+    hipLaunchKernelGGL(kernel, grid, dim3(BIRP_BLOCK), 0, (hipStream_t)stream, v, (unsigned char*)oct, bscale);
     return hip_status(hipGetLastError());
 }
 

@@ -72,3 +72,19 @@ def test_bitwise(device, oracle, interp, kind, spacing, centred):
     ref, _ = oracle_image(oracle, vals, org, (spacing,) * 3, interp, v, v.semantics, init=init)
     assert np.array_equal(img.view(np.uint32), ref.view(np.uint32))
     vol.free()
+
+
+@pytest.mark.parametrize("spread", [3.0, 40.0])  # BF16 records as F16 values with one scale, and as BF16
+def test_bf16_storage_is_bf16(device, spread):
+    rng = np.random.default_rng(4)
+    vals = np.exp(rng.uniform(-spread, 0, SHAPE)).astype(np.float32)
+    near = (vals.view(np.uint32) + 0x7FFF + (vals.view(np.uint32) >> 16 & 1)) & np.uint32(0xFFFF0000)  # rounded to BF16
+    org, spacing = (2.0, -7.0, -6.0), (0.4, 0.4, 0.4)
+    v = capi.make_view(97, 61, 40.0, 30.0, (5.0, -20.0, 6.0), (10.0, 0.0, 0.0), 40.0, 300, math=capi.MATH_FAST)
+    stored = capi.Volume.upload(device, vals, org, spacing, dtype=capi.DTYPE_BF16)
+    rounded = capi.Volume.upload(device, near.view(np.float32), org, spacing)
+    a, _ = stored.render(v)
+    b = rounded.render_f64(v)
+    stored.free()
+    rounded.free()
+    assert b.any() and np.linalg.norm(a - b) <= 1e-6 * np.linalg.norm(b)
