@@ -1204,6 +1204,10 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_space_integrate(ExactView ev, in
 // ------------------------------------------------------------------------------------------
 // GetSample at arbitrary points (DataCube.cpp:203-277 / Cmem.cpp:117-186), exact arithmetic
 // ------------------------------------------------------------------------------------------
+// A trilinear sample of a cube without negative values reads its two quad records, which share a 128-byte
+// line every other time, instead of four pairs of values in four lines of the [z][y][x] copy: random
+// points wait on lines (1,000,003 points over a 200^3 cube: 66 -> 32 us). Other cubes keep the copy: on a
+// grid point the records' lerps give +0 where a value is -0.
 __global__ __launch_bounds__(BIRP_BLOCK) void k_sample_points(DevVolume v, const float* xyz, long long n, float* out) {
     long long p = (long long)blockIdx.x * BIRP_BLOCK + threadIdx.x;
     if (p >= n) return;
@@ -1223,7 +1227,14 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_sample_points(DevVolume v, const
         out[p] = -1.f;
         return;
     }
-    out[p] = (v.interp == BIRP_INTERP_TRILINEAR) ? sample_linear_tri(v, r) : sample_linear_nearest(v, r);
+    if (v.interp == BIRP_INTERP_NEAREST) {
+        out[p] = sample_linear_nearest(v, r);
+    } else if (v.quad && v.qtab && (v.vclass == VC_POSITIVE || v.vclass == VC_NONNEG)) {
+        const QuadCtx qc{make_rsrc(v.quad, v.quad_bytes), v.qtab, v.qtab + v.nx, v.qtab + v.nx + v.ny, 0.f, 0.f, 0.f, 0u, 0u};
+        out[p] = quad_lerp<LERP_NONNEG>(quad_fetch_inside(qc, r.xd, r.yd, r.zd));
+    } else {
+        out[p] = sample_linear_tri(v, r);
+    }
 }
 
 // ------------------------------------------------------------------------------------------

@@ -74,6 +74,25 @@ def test_bitwise(device, oracle, interp, kind, spacing, centred):
     vol.free()
 
 
+@pytest.mark.parametrize("interp", [capi.INTERP_TRILINEAR, capi.INTERP_NEAREST])
+@pytest.mark.parametrize("kind", ["positive", "cavity", "scattered", "minus_zero", "tiny", "signed"])
+def test_point_samples_bitwise(device, oracle, interp, kind):
+    rng = np.random.default_rng(3)
+    vals = field(kind, rng)
+    org, spacing = (-3.0, 0.0, 2.0), (0.25, 0.3, 0.12)
+    hi = np.array([n - 1 for n in SHAPE[::-1]])
+    idx = rng.uniform(-0.5, 1.0, (3000, 3)) * (hi + 0.5)
+    idx[:1500] = np.floor(idx[:1500] * 2) / 2  # grid points and midpoints, faces among them
+    xyz = (np.array(org) + idx * np.array(spacing)).astype(np.float32)
+    vol = capi.Volume.upload(device, vals, org, spacing, interp)
+    got = vol.sample(xyz)
+    vol.free()
+    cube = oracle.OracleCube(vals, org, spacing, interp)
+    want = np.array([cube.sample(float(x), float(y), float(z)) for x, y, z in xyz], np.float32)
+    assert (want >= 0).any() and (want == -1).any()
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("spread", [3.0, 40.0])  # BF16 records as F16 values with one scale, and as BF16
 def test_bf16_storage_is_bf16(device, spread):
     rng = np.random.default_rng(4)
