@@ -205,7 +205,8 @@ int launch_zero_f32(float* p, size_t n, void* stream);
 #define BIRP_SCAN_MAX 128
 #define BIRP_SCAN_DIV 192 /* launch_check_div */
 #define BIRP_SCAN_WORDS 193
-int launch_scan_class(const float* values, size_t n, unsigned* flags_dev, void* stream);
+// With copy_to, `values` may be mapped host memory; both 16-byte aligned.
+int launch_scan_class(const float* values, size_t n, unsigned* flags_dev, void* stream, float* copy_to = nullptr);
 // Checks birp_div_fma2 for the volume's spacings over every significand: ORs bit `axis` into *bad_dev for
 // an axis with a mismatch.
 int launch_check_div(const DevVolume& v, unsigned* bad_dev, void* stream);

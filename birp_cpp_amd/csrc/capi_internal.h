@@ -32,6 +32,12 @@ struct birp_device {
     void* pinned = nullptr;            // pinned host staging for birp_render's image copy
     void* pinned_dev = nullptr;        // its device address (null when the device does not map it)
     size_t pinned_bytes = 0;
+    // large uploads: a ring of kRing chunks of kRingChunk bytes, pinned and mapped (upload_values)
+    static constexpr int kRing = 4;
+    static constexpr size_t kRingChunk = (size_t)4 << 20;
+    char* ring = nullptr;
+    char* ring_dev = nullptr;
+    hipEvent_t ring_done[kRing] = {};
     void* rbuf = nullptr;              // birp_render: [u64 sample counter | pad to 256 B | image]
     size_t rbuf_bytes = 0;
     unsigned long long count_base = 0; // the counter's value at its last read (it only grows)

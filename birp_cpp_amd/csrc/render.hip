@@ -1246,7 +1246,9 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_sample_points(DevVolume v, const
 // two blocks per CU, each with one atomic per word, and the words in cache lines of their own (an
 // atomic on a contended line takes about 8 ns: three per wave on one line took 376 us for 256^3
 // values, whose read takes 13 us at 5.2 TB/s; 27 us now).
-__global__ __launch_bounds__(BIRP_BLOCK) void k_scan_class(const float* vals, size_t n, unsigned* flags) {
+// COPY: vals is a mapped host buffer, and the values go to `out` on the way.
+template <bool COPY>
+__global__ __launch_bounds__(BIRP_BLOCK) void k_scan_class(const float* vals, size_t n, unsigned* flags, float* out) {
     unsigned f = 0, mn = 0x7F7FFFFFu, mx = 0u;
     auto look = [&](float x) {
         const unsigned u = __float_as_uint(x) & 0x7FFFFFFFu;
@@ -1260,13 +1262,18 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_scan_class(const float* vals, si
     };
     const size_t n4 = n / 4, step = (size_t)gridDim.x * BIRP_BLOCK, first = (size_t)blockIdx.x * BIRP_BLOCK + threadIdx.x;
     for (size_t k = first; k < n4; k += step) {
-        const float4 x = reinterpret_cast<const float4*>(vals)[k];  // hipMalloc'ed: aligned
+        const float4 x = reinterpret_cast<const float4*>(vals)[k];  // allocations and chunks of 16 B: aligned
+        if constexpr (COPY) reinterpret_cast<float4*>(out)[k] = x;
         look(x.x);
         look(x.y);
         look(x.z);
         look(x.w);
     }
-    for (size_t k = 4 * n4 + first; k < n; k += step) look(vals[k]);
+    for (size_t k = 4 * n4 + first; k < n; k += step) {
+        const float x = vals[k];
+        if constexpr (COPY) out[k] = x;
+        look(x);
+    }
     __shared__ unsigned s_f, s_mn, s_mx;
     if (threadIdx.x == 0) {
         s_f = 0u;
@@ -2139,9 +2146,10 @@ int launch_sample_points(const DevVolume& v, const float* xyz, long long n, floa
     return hip_status(hipGetLastError());
 }
 
-int launch_scan_class(const float* values, size_t n, unsigned* flags_dev, void* stream) {
+int launch_scan_class(const float* values, size_t n, unsigned* flags_dev, void* stream, float* copy_to) {
     const size_t blocks = std::min<size_t>((n / 4 + BIRP_BLOCK) / BIRP_BLOCK, 512);
-    hipLaunchKernelGGL(k_scan_class, dim3((unsigned)blocks), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, values, n, flags_dev);
+    if (copy_to) hipLaunchKernelGGL((k_scan_class<true>), dim3((unsigned)blocks), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, values, n, flags_dev, copy_to);
+    else hipLaunchKernelGGL((k_scan_class<false>), dim3((unsigned)blocks), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, values, n, flags_dev, nullptr);
     return hip_status(hipGetLastError());
 }
 
