@@ -697,8 +697,8 @@ extern "C" int birp_cmem_create(birp_device* dev, const birp_cmem_state* s, birp
     v->dv.interp = BIRP_INTERP_TRILINEAR;
     (void)hipSetDevice(dev->ordinal);
     hipError_t e = hipMalloc(&v->zones, BIRP_ZONE_BYTES);
+    // renders follow on the device's stream; a server, whose slots have streams of their own, waits for it
     int rc = e == hipSuccess ? launch_cmem_zones(c, v->zones, dev->stream) : hip_fail(e, "hipMalloc(zone bounds)");
-    if (rc == BIRP_OK && (e = hipStreamSynchronize(dev->stream)) != hipSuccess) rc = hip_fail(e, "zone bounds");
     if (rc) {
         free_volume_buffers(v);
         delete v;
@@ -1158,8 +1158,11 @@ int choose_tuning(const birp_volume* vol, const std::vector<birp_view>& views, b
         return BIRP_OK;
     long long rays = 0;
     for (const birp_view& v : views) rays += (long long)v.width * v.height;
-    // untuned: signed cubes and CMEM models keep 8x8 rays per wave (their images depend on it)
-    t = tuning_is_free(fast_kernel_dtype(vol->dv)) ? launch_tuning(rays) : birp_tuning{8, 8, 1, 4};
+    // Untuned: the images of signed cubes and CMEM models depend on the lanes per ray, which no number of views
+    // changes. us with 1 / 2 / 4 lanes, signed cube: 16 of 144x84 n = 200 60 / 43 / 44, 16 of 288x168 n = 320
+    // 133 / 119 / 140; CMEM model: 4 of 72x42 n = 200 133 / 71 / 42, 16 of 288x168 n = 320 365 / 350 / 346.
+    const int kind = fast_kernel_dtype(vol->dv);
+    t = tuning_is_free(kind) ? launch_tuning(rays) : kind == BIRP_KDT_CMEM ? birp_tuning{4, 4, 4, 1} : birp_tuning{4, 8, 2, 1};
     return BIRP_OK;
 }
 
@@ -1183,19 +1186,17 @@ birp_tuning launch_tuning(long long rays) {
     return birp_tuning{8, 8, 1, 4};
 }
 
-// A signed cube's view: an image with few rays splits each ray over 2 or 4 lanes (FP16 storage earlier), which
-// shortens each lane's chain of dependent gathers.
+// A signed cube's view takes 4 lanes per ray up to 20,000 rays and 2 above, where a launch of many views would
+// pay for 4 (us per single view with 1 / 2 / 4 lanes: 144x84 n = 800 69 / 40 / 27, 288x168 n = 320 36 / 24 /
+// 19, 576x336 n = 400 42 / 36 / 43; of many, choose_tuning).
 // A CMEM model's chains of transcendentals want more waves per SIMD than a cube's gathers: its views take
-// 4 lanes per ray over 4x4 rays whatever their size (576x336 at n = 800: 0.724 ms, against 0.817 ms with
-// 1 lane and 0.733 ms with 2).
+// 4 lanes per ray over 4x4 rays whatever their size (576x336 at n = 800 without the zone bounds: 0.724 ms,
+// against 0.817 ms with 1 lane and 0.733 ms with 2). Its unroll is how a single view's kernel asks the zone
+// bounds (fast_tile).
 birp_tuning view_tuning(const birp_view& v, const DevVolume& vol) {
-    if (vol.kind == SK_CMEM) return birp_tuning{4, 4, 4, 1};
-    const bool f16 = vol.dtype == BIRP_DTYPE_F16;
     const long long rays = (long long)v.width * v.height;
-    int lanes = 1;
-    if (rays <= 20000) lanes = v.samples >= 600 ? 4 : (f16 ? 2 : (v.samples >= 240 ? 4 : 1));
-    else if (rays <= 60000 && v.samples >= 600 && f16) lanes = 2;
-    return birp_tuning{8, 64 / (8 * lanes), lanes, 4};
+    if (vol.kind == SK_CMEM) return birp_tuning{4, 4, 4, rays <= 10000 ? 4 : (rays <= 60000 ? 2 : 1)};
+    return rays <= 20000 ? birp_tuning{4, 4, 4, 1} : birp_tuning{4, 8, 2, 1};
 }
 
 void batch_release(birp_batch* b) {

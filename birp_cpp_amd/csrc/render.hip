@@ -1728,16 +1728,41 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
         float sum = 0.f, nc = 0.f;
         const int gshift = ray * S;
         bool alive = true;  // the same in all S lanes of a ray
+        float xd = 0.f, yd = 0.f, zd = 0.f, xn, yn, zn;
+        auto place = [&](int js, float& x, float& y, float& z) {
+            const float fj = (float)min(js, cnt - 1);
+            x = __builtin_fmaf(fj, dix, ix0);
+            y = __builtin_fmaf(fj, diy, iy0);
+            z = __builtin_fmaf(fj, diz, iz0);
+        };
+        // CMEM: U = 1 asks the zone bounds before each sample, U = 2 a trip ahead, U = 4 takes the model in full;
+        // the samples are the same. With a wave per SIMD or less nothing hides the table's load and the zone's
+        // branches, with a few only the load; with many the plain form has the most waves. us with U = 1 / 2 / 4:
+        // 120x70 n = 300 51.5 / 45.2 / 40.3, 144x84 n = 320 39.7 / 33.8 / 42.9, 300x170 n = 300 64.7 / 63.6 / 92.8,
+        // 576x336 n = 800 262 / 275 / 653.
+        constexpr bool AHEAD = CMEM && U == 2;
+        ZoneQuery zone{};
+        if constexpr (AHEAD) {
+            place(sub, xn, yn, zn);
+            zone = zone_fetch(rs, xn, yn, zn);
+        }
         for (int q = 0; q < trips; ++q) {
             const int js = q * S + sub;
             const bool act = alive && js < cnt;
-            const float fj = (float)min(js, cnt - 1);
-            const float xd = __builtin_fmaf(fj, dix, ix0);
-            const float yd = __builtin_fmaf(fj, diy, iy0);
-            const float zd = __builtin_fmaf(fj, diz, iz0);
             float x;
-            if constexpr (CMEM) x = cmem_fast_zoned(V.cmem, zone_fetch(rs, xd, yd, zd), xd, yd, zd);
-            else x = fast_value<DT>(fast_fetch<DT>(V, rs, tab, xd, yd, zd));
+            if constexpr (AHEAD) {
+                xd = xn;
+                yd = yn;
+                zd = zn;
+                place(js + S, xn, yn, zn);
+                const ZoneQuery next = zone_fetch(rs, xn, yn, zn);
+                x = cmem_fast_zoned(V.cmem, zone, xd, yd, zd);
+                zone = next;
+            } else {
+                place(js, xd, yd, zd);
+                if constexpr (!CMEM) x = fast_value<DT>(fast_fetch<DT>(V, rs, tab, xd, yd, zd));
+                else x = U == 4 ? cmem_fast(V.cmem, xd, yd, zd) : cmem_fast_zoned(V.cmem, zone_fetch(rs, xd, yd, zd), xd, yd, zd);
+            }
             const unsigned long long neg = __ballot(act && x < 0.f);
             const unsigned grp = (unsigned)(neg >> gshift) & ((1u << S) - 1u);
             const bool cut = (grp & ((2u << sub) - 1u)) != 0u;
@@ -1876,7 +1901,7 @@ __global__ __launch_bounds__(BIRP_BLOCK, 6) void k_render_fast_one(DevVolume V, 
     constexpr bool CMEM = KV == BIRP_KDT_CMEM;
     constexpr int DT = CMEM ? BIRP_DTYPE_F32 : (KV & 3);
     constexpr bool SIGNED = CMEM || (KV & BIRP_KDT_SIGNED) != 0;
-    static_assert(!SIGNED || U == 1, "signed kernels take one sample per lane per trip");
+    static_assert(CMEM || !SIGNED || U == 1, "signed kernels take one sample per lane per trip");
     extern __shared__ unsigned s_tab[];
     const int b = (int)(blockIdx.x & 7u) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
     const int item = b * (BIRP_BLOCK / 64) + (int)(threadIdx.x >> 6);
@@ -2190,11 +2215,12 @@ int launch_zero_f32(float* p, size_t n, void* stream) {
     return hip_status(hipGetLastError());
 }
 
-// U as the kernels take it: the signed and CMEM kernels one sample per lane per trip, the others at least a
-// lane's 4 / S residues.
+// U as the kernels take it: the signed kernels one sample per lane per trip, a single CMEM view's kernel its way
+// of asking the zone bounds (many views' have the waves for the plain one), the others at least a lane's 4 / S
+// residues.
 template <int KV, int S, int U>
 constexpr int fast_unroll() {
-    return (KV & (BIRP_KDT_SIGNED | BIRP_KDT_CMEM)) ? 1 : (U > 4 / S ? U : 4 / S);
+    return (KV & BIRP_KDT_SIGNED) ? 1 : (KV & BIRP_KDT_CMEM) ? U : (U > 4 / S ? U : 4 / S);
 }
 
 // Calls launch(std::integral_constant KV, S, U) for the variant asked for.
@@ -2240,7 +2266,8 @@ int launch_fast_batch(const DevVolume* vols_dev, int dtype, const FastPose* pose
     const long long grid = ((long long)total_blocks + 8 * chunk - 1) / (8 * chunk) * (8 * chunk);
     if (grid > INT32_MAX) return BIRP_ERR_UNSUPPORTED;
     return with_variant(dtype, lanes_per_ray, unroll, [&](auto kv, auto s, auto u) {
-        hipLaunchKernelGGL((k_render_fast<kv.value, s.value, u.value>), dim3((unsigned)grid), dim3(BIRP_BLOCK), fast_lds_bytes(dtype, tab_entries),
+        constexpr int U = kv.value == BIRP_KDT_CMEM ? 1 : u.value;
+        hipLaunchKernelGGL((k_render_fast<kv.value, s.value, U>), dim3((unsigned)grid), dim3(BIRP_BLOCK), fast_lds_bytes(dtype, tab_entries),
                            (hipStream_t)stream, vols_dev, poses_dev, block_prefix_dev, npose, total_blocks, chunk, twl, tab_entries);
         return hip_status(hipGetLastError());
     });

@@ -53,3 +53,22 @@ def test_every_lanes_per_ray_class(device, size):
     assert st.samples_in_cube == batch.samples()[0] == size[0] * size[1] * 61
     batch.free()
     vol.free()
+
+
+@pytest.mark.parametrize("params", PARAMS)
+def test_fast_views_of_every_size_equal_the_batch(device, params):
+    """A single fast view asks the zone bounds in the way of its size (in full up to 10,000 rays, a trip ahead up
+    to 60,000, before each sample above), a launch of many before each sample: with the same lanes
+    per ray, which order a ray's sum, the images are the same bits."""
+    vol = capi.Volume.cmem(device, capi.cmem_init(capi.cmem_params(**params)))
+    views = [capi.make_view(w, h, 70.0, 50.0, pos, aim, 70.0, n, capi.SEM_EXTENDED, capi.MATH_FAST)
+             for (pos, aim) in POSES for (w, h, n) in ((1, 1, 2), (33, 21, 67), (100, 100, 41), (101, 100, 66), (240, 250, 30), (241, 250, 31))]
+    batch = capi.Batch(vol, views)
+    batch.set_tuning(capi.Tuning(4, 4, 4, 1))
+    batch.launch()
+    batch.wait()
+    for k, v in enumerate(views):
+        got = vol.render(v)[0]
+        assert np.array_equal(got.view(np.uint32), batch.image(k).view(np.uint32)), k
+    batch.free()
+    vol.free()
