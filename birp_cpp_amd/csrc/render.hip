@@ -375,7 +375,8 @@ __device__ __forceinline__ float sample_linear_nearest(const DevVolume& v, const
 
 // ------------------------------------------------------------------------------------------
 // CMEM::GetSample (Cmem.cpp:117-288) on the device: the reference's float/double types and
-// order; the transcendental functions are ROCm's device libm (within ~1 ulp of glibc's).
+// order; the transcendental functions are ROCm's device libm (within ~1 ulp of glibc's) and, for the sheath's
+// power, birp_powf.
 // ------------------------------------------------------------------------------------------
 // (float)acos(c) for a double c, to float accuracy without an FP64 arc cosine: acos(c) =
 // 2 asin(sqrt((1 - c) / 2)) for c >= 0 and pi - 2 asin(sqrt((1 + c) / 2)) below, with 1 -/+ c formed
@@ -389,12 +390,14 @@ __device__ __forceinline__ float acos_to_float(double c) {
 
 // Emissivity outside the bow shock (Cmem.cpp:172-175) and in the sheath (:148-152).
 __device__ __forceinline__ float cmem_outer(const CmemParams& m, float r) {
-    double sd = r / 10;
+    double sd = birp_div_rn64(r, 0.1);
     return (float)(m.A2 * (1 / (sd * sd * sd)));
 }
 __device__ __forceinline__ float cmem_inner(const CmemParams& m, float r, float theta, float st) {
     float half_t = theta / 2;
-    return m.A1 * (expf(-m.B * (half_t * half_t * half_t * half_t))) * powf(r / 10, (-m.alpha - (m.beta * (st * st))));
+    const float sd = birp_div_rn64(r, 0.1), e = -m.alpha - (m.beta * (st * st));
+    const float fall = birp_powf_takes(sd, e) ? birp_powf(sd, e) : powf(sd, e);
+    return m.A1 * (expf(-m.B * (half_t * half_t * half_t * half_t))) * fall;
 }
 
 __device__ __forceinline__ float cmem_sample(const CmemParams& m, float x, float y, float z) {
@@ -519,17 +522,19 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_cmem_zones(CmemParams m, float4*
 enum Zone { ZONE_INSIDE, ZONE_SHEATH, ZONE_OUTER, ZONE_EDGE };
 struct ZoneQuery {
     float4 t;
-    float r;
+    float r, ir, iyz;  // |(x, y, z)| and the reciprocals of it and of |(y, z)|, to a few ulps
     bool axis;
 };
 __device__ __forceinline__ ZoneQuery zone_fetch(__amdgpu_buffer_rsrc_t rs, float x, float y, float z) {
     ZoneQuery q;
-    const float yz2 = __builtin_fmaf(y, y, z * z), r2 = __builtin_fmaf(x, x, yz2), ir = __builtin_amdgcn_rsqf(r2);
-    const float u = __builtin_fmaf(x * ir, 0.5f * BIRP_ZONE_CT, 0.5f * BIRP_ZONE_CT);
-    const float v = __builtin_fmaf(y * __builtin_amdgcn_rsqf(yz2), 0.5f * BIRP_ZONE_CP, 0.5f * BIRP_ZONE_CP);
+    const float yz2 = __builtin_fmaf(y, y, z * z), r2 = __builtin_fmaf(x, x, yz2);
+    q.ir = __builtin_amdgcn_rsqf(r2);
+    q.iyz = __builtin_amdgcn_rsqf(yz2);
+    const float u = __builtin_fmaf(x * q.ir, 0.5f * BIRP_ZONE_CT, 0.5f * BIRP_ZONE_CT);
+    const float v = __builtin_fmaf(y * q.iyz, 0.5f * BIRP_ZONE_CP, 0.5f * BIRP_ZONE_CP);
     const unsigned iu = (unsigned)__builtin_amdgcn_fmed3f(u, 0.0f, BIRP_ZONE_CT - 1.0f), iv = (unsigned)__builtin_amdgcn_fmed3f(v, 0.0f, BIRP_ZONE_CP - 1.0f);
     q.t = load16(rs, (iu * BIRP_ZONE_CP + iv) * 16u);
-    q.r = r2 * ir;
+    q.r = r2 * q.ir;
     q.axis = !(fabsf(x * y) > 0.0f);
     return q;
 }
@@ -540,20 +545,32 @@ __device__ __forceinline__ Zone zone_of(const ZoneQuery& q) {
     return q.r < q.t.z ? ZONE_SHEATH : q.r > q.t.w ? ZONE_OUTER : ZONE_EDGE;
 }
 
+// RN(sqrt(a)) from the query's estimate of 1 / sqrt(a), which is off by another rounding of a.
+__device__ __forceinline__ float sqrt_from(float a, float y) {
+    if (__builtin_expect(!(a >= 0x1p-96f), 0)) return sqrtf(a);
+    return birp_sqrt_rn(a, y);
+}
+
 // cmem_sample with its surfaces left out where the bounds name the point's zone: the same value, bit for bit.
 // The surfaces are the model's cost (about 900 of 1,100 VALU instructions per sample in libm calls) and a
 // zone is all that most samples need of them: a query is 35 instructions and one 16-byte load. 576x336 x
-// 800: 3.45 -> 0.65 ms; fast form 0.662 -> 0.264 ms. A table of half the cells per axis gives 0.70 and
-// 0.270 ms, of twice 0.64 and 0.262 (2 MB): what is left is the sheath's powf and the outer zone's
-// FP64 cube, not the cells on a surface.
+// 800: 3.45 -> 0.62 ms; fast form 0.662 -> 0.264 ms. A table of half the cells per axis gives 0.67 and
+// 0.270 ms, of twice 0.61 and 0.262 (2 MB): the cells on a surface are not what is left.
+// The roots start from the query's reciprocals, the quotients by r share one in FP64, and the sheath's power
+// is birp_powf: 0.62 -> 0.51 ms (138 VALU instructions per sample, 97% of the issue slots; 8 orbit views of
+// 288x168 at n = 320 0.359 -> 0.325). birp_powf is within 0.502 ulp of the power, powf within 1.3.
 __device__ __forceinline__ float cmem_sample_zoned(const CmemParams& m, const ZoneQuery& q, float x, float y, float z) {
     const Zone zone = zone_of(q);
     float val = 0.f;
     if (zone == ZONE_EDGE) val = cmem_sample(m, x, y, z);
     if (zone == ZONE_SHEATH || zone == ZONE_OUTER) {
-        const float r = sqrtf(x * x + y * y + z * z);
-        if (zone == ZONE_OUTER) val = cmem_outer(m, r);
-        else val = cmem_inner(m, r, acosf(x / r), sqrtf(y * y + z * z) / r);
+        const float r = sqrt_from(x * x + y * y + z * z, q.ir);
+        if (zone == ZONE_OUTER) {
+            val = cmem_outer(m, r);
+        } else {
+            const double rc = rcp64((double)r);
+            val = cmem_inner(m, r, acosf(birp_div_rn64(x, rc)), birp_div_rn64(sqrt_from(y * y + z * z, q.iyz), rc));
+        }
     }
     return val;
 }
