@@ -1,5 +1,5 @@
 """Tune the fast-path kernels (tile shape, lanes per ray, unroll) for the standard workloads and
-write the table that batches, fast single renders and the server read:
+write a table that batches read after birp_autotune_load:
 
     python -m birp_cpp_amd.tune [--out birp_cpp_amd/tuning.jsonl]
 
@@ -7,7 +7,10 @@ The views cover every (image-size class, samples class) the workloads use: the 2
 of the batched workload (three image sizes, steps 0.1 and 0.25 RE), the 1600-sample views
 of the precision workload, and 0.5 RE steps as the serving workload draws them. Each
 class is tuned for FP32, BF16 and F16 storage on the 256^3 shell cube, by birp_autotune (every
-candidate timed with HIP events on a batch of that class's views).
+candidate timed with HIP events on a batch of that class's views). No table ships with the package: without
+one a batch's tuning follows its number of rays, which a table of per-view classes does not know, and that
+measured no slower in any class (8 orbit views of F16 97 us against 104, two of 512^3 at 1,600 samples
+150 against 165, 256 orbit views the same).
 """
 from __future__ import annotations
 
