@@ -400,17 +400,9 @@ __device__ __forceinline__ float cmem_inner(const CmemParams& m, float r, float 
     return m.A1 * (expf(-m.B * (half_t * half_t * half_t * half_t))) * fall;
 }
 
-__device__ __forceinline__ float cmem_sample(const CmemParams& m, float x, float y, float z) {
-    float r = sqrtf(x * x + y * y + z * z);
-    const float ryz = sqrtf(y * y + z * z);
-    float theta = (x != 0) ? acosf(x / r) : 0.f;
-    // phi = acos(y / ryz) (0 when y == 0) enters only through its cosine and sine, and theta's
-    // cosine and sine are needed too: all four from the ratios that are their arc cosines' arguments
-    // (theta, phi in [0, pi], so both sines are >= 0; x == 0 and y == 0 give the reference's angle
-    // 0), within an ulp or two of cos(acos(u)) and sin(acos(u)), with no trigonometric call
-    const float ct = (x != 0) ? x / r : 1.f, st = (x != 0) ? ryz / r : 0.f;
-    const float cos_phi = (y != 0) ? y / ryz : 1.f, sin_phi = (y != 0) ? fabsf(z) / ryz : 0.f;
-    // LinScaled (Cmem.cpp:188-222)
+// The magnetopause's radius in a direction (LinScaled, Cmem.cpp:188-222): ct, st and cos_phi, sin_phi of its
+// angles, theta itself.
+__device__ __forceinline__ float cmem_mp(const CmemParams& m, float ct, float st, float theta, float cos_phi, float sin_phi, float y, float z) {
     // cos(phi - pi/2) and cos(phi - 3 pi/2) in double (Cmem.cpp:205, 209) are sin(phi) and
     // -sin(phi), formed here in double from the coordinates
     const double sphi = (y != 0) ? (double)fabsf(z) / sqrt((double)y * y + (double)z * z) : 0.0;
@@ -420,29 +412,53 @@ __device__ __forceinline__ float cmem_sample(const CmemParams& m, float x, float
                    (m.p1 * (m.beta_c[0] + m.beta_c[1] * cos_phi + m.beta_c[3] * (sin_phi * sin_phi))));
     float q = m.p2 * m.charlie * expf(m.p3 * m.dn * (powf(phi_n, m.a21))) +
               m.p2 * m.charlie * expf(m.p3 * m.ds * (powf(phi_s, m.a21)));
-    float radius_mp = m.p0 * m.r0_lin * f + q;
-    float h = 0.05f / 2;
-    if (r < radius_mp - h) return 0;  // inside the magnetopause: the bow shock is not needed
-    // ShueModel (Cmem.cpp:280-288)
+    return m.p0 * m.r0_lin * f + q;
+}
+
+// The bow shock's (ShueModel, Cmem.cpp:280-288).
+__device__ __forceinline__ float cmem_bs(const CmemParams& m, float ct, float cos_phi, float sin_phi) {
     float base = 2 / (1 + ct);
     float ry = m.bs * powf(base, m.ay_bs);
     float rz = (m.az_bs == m.ay_bs) ? ry : m.bs * powf(base, m.az_bs);  // equal unless set apart
     float rzc = rz * cos_phi, rys = ry * sin_phi;
-    float radius_bs = (ry * rz) / sqrtf((rzc * rzc) + (rys * rys));
+    return (ry * rz) / sqrtf((rzc * rzc) + (rys * rys));
+}
+
+// ask_mp, ask_bs: false where the point is known to lie outside the magnetopause (beyond its band), inside the bow
+// shock (below its band).
+__device__ __forceinline__ float cmem_sample(const CmemParams& m, float x, float y, float z, bool ask_mp = true, bool ask_bs = true) {
+    float r = sqrtf(x * x + y * y + z * z);
+    const float ryz = sqrtf(y * y + z * z);
+    float theta = (x != 0) ? acosf(x / r) : 0.f;
+    // phi = acos(y / ryz) (0 when y == 0) enters only through its cosine and sine, and theta's
+    // cosine and sine are needed too: all four from the ratios that are their arc cosines' arguments
+    // (theta, phi in [0, pi], so both sines are >= 0; x == 0 and y == 0 give the reference's angle
+    // 0), within an ulp or two of cos(acos(u)) and sin(acos(u)), with no trigonometric call
+    const float ct = (x != 0) ? x / r : 1.f, st = (x != 0) ? ryz / r : 0.f;
+    const float cos_phi = (y != 0) ? y / ryz : 1.f, sin_phi = (y != 0) ? fabsf(z) / ryz : 0.f;
     // the reference's zone tests in its order (Cmem.cpp:136-176); the sheath emissivity is
     // evaluated only for the three zones that use it
-    const bool z_mp = r >= radius_mp - h && r <= radius_mp + h;
-    const bool z_sheath = !z_mp && r > radius_mp + h && r < radius_bs - h;
-    const bool z_bs = !z_mp && !z_sheath && r >= radius_bs - h && r <= radius_bs + h;
-    if (!(z_mp || z_sheath || z_bs)) return cmem_outer(m, r);
-    float inner = cmem_inner(m, r, theta, st);
-    if (z_mp) {
-        float norm = (r - (radius_mp - h)) / (radius_mp + h);
-        return lerp_general(0.f, inner, norm);
+    const float h = 0.05f / 2;
+    bool z_mp = false, past = true;
+    float norm = 0.f;
+    if (ask_mp) {
+        const float radius_mp = cmem_mp(m, ct, st, theta, cos_phi, sin_phi, y, z);
+        if (r < radius_mp - h) return 0;  // inside the magnetopause: the bow shock is not needed
+        z_mp = r >= radius_mp - h && r <= radius_mp + h;
+        past = r > radius_mp + h;
+        norm = (r - (radius_mp - h)) / (radius_mp + h);
     }
+    bool z_sheath = !z_mp && past, z_bs = false;
+    if (ask_bs && !z_mp) {
+        const float radius_bs = cmem_bs(m, ct, cos_phi, sin_phi);
+        z_sheath = past && r < radius_bs - h;
+        z_bs = !z_sheath && r >= radius_bs - h && r <= radius_bs + h;
+        norm = (r - (radius_bs - h)) / (radius_bs + h);
+    }
+    if (!(z_mp || z_sheath || z_bs)) return cmem_outer(m, r);
+    const float inner = cmem_inner(m, r, theta, st);
     if (z_sheath) return inner;
-    float norm = (r - (radius_bs - h)) / (radius_bs + h);
-    return lerp_general(inner, cmem_outer(m, r), norm);
+    return lerp_general(z_mp ? 0.f : inner, z_mp ? inner : cmem_outer(m, r), norm);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -517,9 +533,9 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_cmem_zones(CmemParams m, float4*
     zones[cell] = t;
 }
 
-// What the bounds say of a point. ZONE_EDGE: nothing; also for points on x = 0 or y = 0, where the
-// reference takes an angle of 0 (Cmem.cpp:224-246).
-enum Zone { ZONE_INSIDE, ZONE_SHEATH, ZONE_OUTER, ZONE_EDGE };
+// What the bounds say of a point: its zone, or (SPLIT) which of the surfaces it takes to know (ZONE_EDGE: both;
+// also for points on x = 0 or y = 0, where the reference takes an angle of 0, Cmem.cpp:224-246).
+enum Zone { ZONE_INSIDE, ZONE_OUTER, ZONE_SHEATH, ZONE_EDGE_MP, ZONE_EDGE_BS, ZONE_EDGE };
 struct ZoneQuery {
     float4 t;
     float r, ir, iyz;  // |(x, y, z)| and the reciprocals of it and of |(y, z)|, to a few ulps
@@ -538,11 +554,12 @@ __device__ __forceinline__ ZoneQuery zone_fetch(__amdgpu_buffer_rsrc_t rs, float
     q.axis = !(fabsf(x * y) > 0.0f);
     return q;
 }
+template <bool SPLIT>
 __device__ __forceinline__ Zone zone_of(const ZoneQuery& q) {
     if (q.axis) return ZONE_EDGE;
     if (q.r < q.t.x) return ZONE_INSIDE;
-    if (!(q.r > q.t.y)) return ZONE_EDGE;
-    return q.r < q.t.z ? ZONE_SHEATH : q.r > q.t.w ? ZONE_OUTER : ZONE_EDGE;
+    if (!(q.r > q.t.y)) return SPLIT && q.r < q.t.z ? ZONE_EDGE_MP : ZONE_EDGE;
+    return q.r < q.t.z ? ZONE_SHEATH : q.r > q.t.w ? ZONE_OUTER : SPLIT ? ZONE_EDGE_BS : ZONE_EDGE;
 }
 
 // RN(sqrt(a)) from the query's estimate of 1 / sqrt(a), which is off by another rounding of a.
@@ -557,13 +574,16 @@ __device__ __forceinline__ float sqrt_from(float a, float y) {
 // 800: 3.45 -> 0.62 ms; fast form 0.662 -> 0.264 ms. A table of half the cells per axis gives 0.67 and
 // 0.270 ms, of twice 0.61 and 0.262 (2 MB): the cells on a surface are not what is left.
 // The roots start from the query's reciprocals, the quotients by r share one in FP64, and the sheath's power
-// is birp_powf: 0.62 -> 0.51 ms (138 VALU instructions per sample, 97% of the issue slots; 8 orbit views of
-// 288x168 at n = 320 0.359 -> 0.325). birp_powf is within 0.502 ulp of the power, powf within 1.3.
+// is birp_powf: 0.62 -> 0.51 ms. birp_powf is within 0.502 ulp of the power, powf within 1.3.
+// A sample near one surface takes that one only (about 900 instructions for the magnetopause, 200 for the bow
+// shock; a trip's lanes seldom meet both): 0.505 -> 0.476 ms, 300x170 n = 300 103 -> 84 us, 144x84 n = 320
+// 46 -> 38, the 8 views 0.325 -> 0.314 ms.
 __device__ __forceinline__ float cmem_sample_zoned(const CmemParams& m, const ZoneQuery& q, float x, float y, float z) {
-    const Zone zone = zone_of(q);
+    const Zone zone = zone_of<true>(q);
     float val = 0.f;
-    if (zone == ZONE_EDGE) val = cmem_sample(m, x, y, z);
-    if (zone == ZONE_SHEATH || zone == ZONE_OUTER) {
+    if (zone >= ZONE_EDGE_MP) {
+        val = cmem_sample(m, x, y, z, zone != ZONE_EDGE_BS, zone != ZONE_EDGE_MP);
+    } else if (zone != ZONE_INSIDE) {
         const float r = sqrt_from(x * x + y * y + z * z, q.ir);
         if (zone == ZONE_OUTER) {
             val = cmem_outer(m, r);
@@ -1539,6 +1559,26 @@ __device__ __forceinline__ float cmem_fast_inner(const CmemParams& m, float sd, 
 }
 __device__ __forceinline__ float cmem_fast_outer(const CmemParams& m, float sd) { return m.A2 * __builtin_amdgcn_rcpf(sd * sd * sd); }
 
+// cmem_mp and cmem_bs in this arithmetic.
+__device__ __forceinline__ float cmem_fast_mp(const CmemParams& m, float ct, float st, float theta, float cphi, float sphi) {
+    // LinScaled (Cmem.cpp:188-222): cos(phi - pi/2) = sin(phi), cos(phi - 3 pi/2) = -sin(phi)
+    const float phi_n = acos_fast(ct * m.cos_theta_n + st * m.sin_theta_n * sphi);
+    const float phi_s = acos_fast(ct * m.cos_theta_s - st * m.sin_theta_s * sphi);
+    const float cos_half = __builtin_amdgcn_sqrtf(0.5f * (1.f + ct));  // cos(theta / 2), theta in [0, pi]
+    const float sin_2t = 2.f * st * ct;
+    const float f = pow_fast(cos_half + m.a5 * sin_2t * (1.f - exp_fast(-theta)),
+                             m.p1 * (m.beta_c[0] + m.beta_c[1] * cphi + m.beta_c[3] * (sphi * sphi)));
+    const float q = m.p2 * m.charlie * (exp_fast(m.p3 * m.dn * pow_fast(phi_n, m.a21)) + exp_fast(m.p3 * m.ds * pow_fast(phi_s, m.a21)));
+    return m.p0 * m.r0_lin * f + q;
+}
+__device__ __forceinline__ float cmem_fast_bs(const CmemParams& m, float ct, float cphi, float sphi) {
+    const float base = 2.f * __builtin_amdgcn_rcpf(1.f + ct);
+    const float ry = m.bs * pow_fast(base, m.ay_bs);
+    const float rz = (m.az_bs == m.ay_bs) ? ry : m.bs * pow_fast(base, m.az_bs);
+    const float rzc = rz * cphi, rys = ry * sphi;
+    return ry * rz * __builtin_amdgcn_rsqf(rzc * rzc + rys * rys);
+}
+
 __device__ __forceinline__ float cmem_fast(const CmemParams& m, float x, float y, float z) {
     const float ryz2 = y * y + z * z;
     const float r = __builtin_amdgcn_sqrtf(__builtin_fmaf(x, x, ryz2)), ryz = __builtin_amdgcn_sqrtf(ryz2);
@@ -1548,23 +1588,10 @@ __device__ __forceinline__ float cmem_fast(const CmemParams& m, float x, float y
     const float ct = xs ? x * ir : 1.f, st = xs ? ryz * ir : 0.f;
     const float theta = xs ? acos_fast(ct) : 0.f;
     const float cphi = ys ? y * iyz : 1.f, sphi = ys ? fabsf(z) * iyz : 0.f;
-    // LinScaled (Cmem.cpp:188-222): cos(phi - pi/2) = sin(phi), cos(phi - 3 pi/2) = -sin(phi)
-    const float phi_n = acos_fast(ct * m.cos_theta_n + st * m.sin_theta_n * sphi);
-    const float phi_s = acos_fast(ct * m.cos_theta_s - st * m.sin_theta_s * sphi);
-    const float cos_half = __builtin_amdgcn_sqrtf(0.5f * (1.f + ct));  // cos(theta / 2), theta in [0, pi]
-    const float sin_2t = 2.f * st * ct;
-    const float f = pow_fast(cos_half + m.a5 * sin_2t * (1.f - exp_fast(-theta)),
-                             m.p1 * (m.beta_c[0] + m.beta_c[1] * cphi + m.beta_c[3] * (sphi * sphi)));
-    const float q = m.p2 * m.charlie * (exp_fast(m.p3 * m.dn * pow_fast(phi_n, m.a21)) + exp_fast(m.p3 * m.ds * pow_fast(phi_s, m.a21)));
-    const float rmp = m.p0 * m.r0_lin * f + q;
+    const float rmp = cmem_fast_mp(m, ct, st, theta, cphi, sphi);
     const float h = 0.025f;
     if (r < rmp - h) return 0.f;
-    // ShueModel (Cmem.cpp:280-288)
-    const float base = 2.f * __builtin_amdgcn_rcpf(1.f + ct);
-    const float ry = m.bs * pow_fast(base, m.ay_bs);
-    const float rz = (m.az_bs == m.ay_bs) ? ry : m.bs * pow_fast(base, m.az_bs);
-    const float rzc = rz * cphi, rys = ry * sphi;
-    const float rbs = ry * rz * __builtin_amdgcn_rsqf(rzc * rzc + rys * rys);
+    const float rbs = cmem_fast_bs(m, ct, cphi, sphi);
     // the zones of Cmem.cpp:132-176 (r >= rmp - h here)
     const bool z_mp = r <= rmp + h;
     const bool z_sheath = !z_mp && r < rbs - h;
@@ -1578,9 +1605,10 @@ __device__ __forceinline__ float cmem_fast(const CmemParams& m, float x, float y
     return __builtin_fmaf((r - (rbs - h)) * __builtin_amdgcn_rcpf(rbs + h), outer - inner, inner);
 }
 
-// cmem_fast with its surfaces left out where the bounds name the point's zone.
+// cmem_fast with its surfaces left out where the bounds name the point's zone. (Only the surface near a sample, as
+// cmem_sample_zoned asks it: 8% slower, its selects weigh as much as the hardware's transcendentals.)
 __device__ __forceinline__ float cmem_fast_zoned(const CmemParams& m, const ZoneQuery& q, float x, float y, float z) {
-    const Zone zone = zone_of(q);
+    const Zone zone = zone_of<false>(q);
     float val = 0.f;
     if (zone == ZONE_EDGE) val = cmem_fast(m, x, y, z);
     if (zone == ZONE_SHEATH || zone == ZONE_OUTER) {
