@@ -5,15 +5,15 @@
 //
 // Two arithmetic families:
 //  * exact  -- FP32 in the reference's operation order (no FMA contraction: the file is built
-//              with -ffp-contract=off), correctly rounded divisions via birp_div_rn, the double
-//              scale chain via birp_scale_sample, std::lerp's branch structure, and the image sum
+//              with -ffp-contract=off), correctly rounded divisions and the scale chain in the
+//              short forms of exact_math.h, std::lerp's branch structure, and the image sum
 //              in k order. Bit-identical to the reference CPU render for finite cubes.
 //  * fast   -- FP64 camera basis, ray origin and cube entry; FP32 FMA march in index space;
-//              BF16/F16/FP32 storage; FP32 Kahan sums. Many views in one launch.
+//              BF16/F16/FP32 storage; FP32 Kahan sums over groups of 16 samples. Many views in one launch.
 //
 // Wave mapping: a wave64 owns a tile of 64/S rays; S lanes ("sub-lanes") share one ray and take
 // its samples k = kb + sub, kb advancing by S each trip. In the exact kernels every sub-lane then
-// reads its quad-mates' samples through DPP quad_perm operands and all of them add the S samples
+// reads its ray's other samples through DPP operands and all of them add the S samples
 // in k order, so the sequential FP32 sum of the reference is kept while S lanes sample in
 // parallel. A masked-off sample contributes -0.0f, which leaves every partial sum unchanged.
 //

@@ -191,13 +191,13 @@ int birp_render_async(birp_volume* vol, const birp_view* view, birp_image* img);
  * serving loops, harnesses that forbid hipMalloc): birp_render_async of each of `count` views of
  * one volume into images_dev[k] (device memory the caller owns, views[k].height * width floats),
  * the same images bit for bit, with no allocation of any kind. Exact views run the exact kernel;
- * fast views are grouped by lanes per ray and each group is one persistent launch whose volume,
- * poses, tile prefix sums and work-queue counters live in a fixed device array of the library,
+ * fast views are one launch (signed cubes and CMEM models: one per lanes per ray) whose volume,
+ * poses and tile prefix sums live in a fixed device array of the library,
  * BIRP_NOALLOC_SCRATCH_KIB per GPU, set up by birp_device_open and held until the process ends. At
  * most BIRP_NOALLOC_MAX_VIEWS views per call (BIRP_ERR_UNSUPPORTED beyond: the array holds that
  * many poses). Asynchronous on
  * the device's stream, like birp_render_async. Every call on a GPU shares that GPU's array, which
- * keeps the last call's descriptors (the counters are cleared by each call): calls on one device
+ * keeps the last call's descriptors: calls on one device
  * from different threads or streams that overlap race on it. */
 #define BIRP_NOALLOC_SCRATCH_KIB 21
 #define BIRP_NOALLOC_MAX_VIEWS 64
@@ -214,7 +214,7 @@ int birp_render_f64(birp_volume* vol, const birp_view* view, double* image);
 int birp_view_basis(const birp_view* view, float* angle_sun, float rot[9], float rinv[9]);
 
 /* ------------------------------------------------------------------ batched renders */
-/* Many poses (and image sizes, sample counts) over one volume in one persistent-kernel launch,
+/* Many poses (and image sizes, sample counts) over one volume in one launch,
  * also captured in a HIP graph that can be replayed. Images are written into one device buffer; image i
  * starts at offset[i] floats. No reference counterpart: the reference renders one pose per
  * Camera (Camera.cpp:63) and batches cubes serially (main.cpp:242-264). */
@@ -226,7 +226,8 @@ typedef struct birp_tuning {
 
 int birp_batch_create(birp_volume* vol, const birp_view* views, int count, birp_batch** out);
 int birp_batch_free(birp_batch* b);
-/* Selects kernel tuning for the batch: an explicit choice, or NULL for the autotuner's. */
+/* Selects kernel tuning for the batch: an explicit choice, or NULL for a loaded tuning table's or, without
+ * one for the batch's class, the one that suits its number of rays. */
 int birp_batch_set_tuning(birp_batch* b, const birp_tuning* tuning);
 /* Launch without waiting (birp_batch_wait waits for completion): the batch's kernels go straight
  * onto the device stream, which measured faster per launch than replaying the captured graph. */
