@@ -14,21 +14,21 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def exe(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fma") / "exact_fma_check")
     subprocess.run(["g++", "-O2", "-std=c++20", "-ffp-contract=off", os.path.join(HERE, "cpu", "exact_fma_check.cpp"), "-o", out], check=True)
     return out
 
 
 @pytest.mark.parametrize("args", [["scale"], ["lerp", "1"], ["lerp", "2"]] + [["div", repr(b)] for b in (30 / 255, 30 / 127, 0.1, 0.25, 7.0)])
-def test_fma_forms_equal_the_operations(checker, args):
-    r = subprocess.run([checker] + args, capture_output=True, text=True)
+def test_fma_forms_equal_the_operations(exe, args):
+    r = subprocess.run([exe] + args, capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
 
 
-def test_the_division_form_fails_for_some_spacings(checker):
+def test_the_division_form_fails_for_some_spacings(exe):
     # 0.12 is one of them: the upload's check is needed
-    assert subprocess.run([checker, "div", "0.12"], capture_output=True).returncode == 1
+    assert subprocess.run([exe, "div", "0.12"], capture_output=True).returncode == 1
 
 
 @pytest.mark.gpu

@@ -9,13 +9,13 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def exe(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("pow") / "exact_pow_check")
     subprocess.run(["g++", "-O2", "-std=c++20", "-mfma", "-ffp-contract=off", os.path.join(HERE, "cpu", "exact_pow_check.cpp"), "-o", out], check=True)
     return out
 
 
 @pytest.mark.parametrize("args", [["sqrt", "0"], ["sqrt", "-96"], ["sqrt", "124"], ["pow", "1"], ["pow", "2"]])
-def test_within_the_stated_error(checker, args):
-    r = subprocess.run([checker] + args, capture_output=True, text=True)
+def test_within_the_stated_error(exe, args):
+    r = subprocess.run([exe] + args, capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
