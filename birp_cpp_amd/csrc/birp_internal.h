@@ -198,6 +198,19 @@ int launch_fast_batch(const DevVolume* vols_dev, int dtype, const FastPose* pose
                       int tab_entries);
 // blocks (of 4 wave tiles) of a view of `tiles` tiles
 inline int fast_blocks(int tiles) { return (int)(((long long)tiles + 3) / 4); }
+// The launches of such a list: each covers the blocks [first, first + count), with a grid of `grid` blocks.
+// HIP takes fewer than 2^32 threads along an axis, 2^24 blocks of 256; a launch here has at most 2^23.
+#define BIRP_FAST_CHUNK 16
+#define BIRP_FAST_PIECE (1 << 23)
+struct FastPiece {
+    int first, count;
+    unsigned grid;  // count rounded up to whole chunks on each of the 8 XCDs
+};
+inline FastPiece fast_piece(int total_blocks, int first) {
+    const int left = total_blocks - first, count = left < BIRP_FAST_PIECE ? left : BIRP_FAST_PIECE;
+    const unsigned round = 8 * BIRP_FAST_CHUNK;
+    return FastPiece{first, count, ((unsigned)count + round - 1) / round * round};
+}
 int launch_zero_f32(float* p, size_t n, void* stream);
 // Words of the class scan's flags (one cache line each), in a buffer of BIRP_SCAN_WORDS.
 #define BIRP_SCAN_CLASS 0

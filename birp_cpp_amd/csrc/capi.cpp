@@ -1429,7 +1429,7 @@ int batch_setup(birp_batch* b) {
         int rc = fast_pose(b->vol, &b->views[k], 0, out, t.tile_w, t.tile_h, poses[k]);
         if (rc) return rc;
         const long long next = (long long)prefix[k] + fast_blocks(tiles_of(b->views[k], t.tile_w, t.tile_h));
-        if (next > INT32_MAX) return fail(BIRP_ERR_UNSUPPORTED, "batch of more than 2^31 - 1 tiles: split it");
+        if (next > INT32_MAX) return fail(BIRP_ERR_UNSUPPORTED, "batch of more than 2^31 - 1 blocks of 4 tiles: split it");
         prefix[k + 1] = (int)next;
     }
     b->total_blocks = prefix[n];
@@ -1708,7 +1708,7 @@ extern "C" int birp_render_views_noalloc(birp_volume* vol, const birp_view* view
             if (rc) return rc;
             int* pre = prefix + g * (BIRP_NOALLOC_MAX_VIEWS + 1);
             const long long next = (long long)pre[nfast[g]] + fast_blocks(tiles_of(views[k], t.tile_w, t.tile_h));
-            if (next > INT32_MAX) return fail(BIRP_ERR_UNSUPPORTED, "more than 2^31 - 1 tiles");
+            if (next > INT32_MAX) return fail(BIRP_ERR_UNSUPPORTED, "more than 2^31 - 1 blocks of 4 tiles");
             pre[nfast[g] + 1] = (int)next;
             nfast[g]++;
             gt[g] = t;

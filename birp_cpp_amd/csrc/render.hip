@@ -1905,8 +1905,10 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
 // The wave tiles of many views in one launch, as a plain grid: a block renders 4 consecutive tiles of one view
 // (prefix[k] = first block of view k), its waves sharing the view's offset tables in LDS, and the
 // dispatcher balances the load. Blocks go round-robin over the 8 XCDs; block b renders item
-// (c * 8 + b % 8) * chunk + i, its c-th chunk: each XCD renders runs of `chunk` neighbouring blocks, whose
-// rays meet the same records in its L2, and a fair share of every view.
+// first + (c * 8 + b % 8) * chunk + i, its c-th chunk of BIRP_FAST_CHUNK: each XCD renders runs of neighbouring
+// blocks, whose rays meet the same records in its L2, and a fair share of every view (chunks of 4 to 64
+// measured within 2% of each other, 1 up to 5% slower on small views). A list of more blocks than a
+// grid may have takes several launches (fast_piece).
 // A persistent grid whose waves claimed tiles from 8 atomic queues took 20-80 us more per launch (every wave
 // visits all queues before it leaves, and claims on one address serialize): 16 FP16 views of 288x168 x 320
 // 154 -> 73 us, 16 of 576x336 x 800 556 -> 487 us, 256 mixed orbit views 2.37 -> 2.24 ms.
@@ -1922,15 +1924,17 @@ __device__ __forceinline__ void load_fast_tables(const DevVolume& V, bool f32, u
 
 template <int KV, int S, int U>
 __global__ __launch_bounds__(BIRP_BLOCK, 6) void k_render_fast(const DevVolume* __restrict__ vols, const FastPose* __restrict__ poses,
-                                                               const int* __restrict__ prefix, int npose, int total, int chunk,
+                                                               const int* __restrict__ prefix, int npose, int first, int count,
                                                                int tw_log2, int tab_entries) {
     constexpr bool CMEM = KV == BIRP_KDT_CMEM;
     constexpr int DT = CMEM ? BIRP_DTYPE_F32 : (KV & 3);
     constexpr bool SIGNED = CMEM || (KV & BIRP_KDT_SIGNED) != 0;
     static_assert(!SIGNED || U == 1, "signed kernels take one sample per lane per trip");
     extern __shared__ unsigned s_tab[];
-    const int turn = (int)(blockIdx.x >> 3), g = (turn / chunk * 8 + (int)(blockIdx.x & 7u)) * chunk + turn % chunk;
-    if (g >= total) return;
+    constexpr int chunk = BIRP_FAST_CHUNK;
+    const int turn = (int)(blockIdx.x >> 3), at = (turn / chunk * 8 + (int)(blockIdx.x & 7u)) * chunk + turn % chunk;
+    if (at >= count) return;
+    const int g = first + at;
     const int k = find_view(prefix, npose, g);
     const FastPose& P = poses[k];
     const DevVolume& V = vols[P.vol];
@@ -2311,14 +2315,18 @@ int launch_fast_batch(const DevVolume* vols_dev, int dtype, const FastPose* pose
                       int total_blocks, int tile_w, int tile_h, int lanes_per_ray, int unroll, void* stream, int tab_entries) {
     const int twl = tile_log2(tile_w, tile_h, lanes_per_ray);
     if (twl < 0 || npose < 1 || total_blocks < 1 || tab_entries < 0 || tab_entries > BIRP_FAST_TAB) return BIRP_ERR_INVALID_ARGUMENT;
-    const int chunk = 16;  // 4 to 64 measured within 2% of each other, 1 up to 5% slower on small views
-    const long long grid = ((long long)total_blocks + 8 * chunk - 1) / (8 * chunk) * (8 * chunk);
-    if (grid > INT32_MAX) return BIRP_ERR_UNSUPPORTED;
     return with_variant(dtype, lanes_per_ray, unroll, [&](auto kv, auto s, auto u) {
         constexpr int U = kv.value == BIRP_KDT_CMEM ? 1 : u.value;
-        hipLaunchKernelGGL((k_render_fast<kv.value, s.value, U>), dim3((unsigned)grid), dim3(BIRP_BLOCK), fast_lds_bytes(dtype, tab_entries),
-                           (hipStream_t)stream, vols_dev, poses_dev, block_prefix_dev, npose, total_blocks, chunk, twl, tab_entries);
-        return hip_status(hipGetLastError());
+        int rc = BIRP_OK;
+        for (int first = 0; first < total_blocks && rc == BIRP_OK;) {
+            const FastPiece p = fast_piece(total_blocks, first);
+            hipLaunchKernelGGL((k_render_fast<kv.value, s.value, U>), dim3(p.grid), dim3(BIRP_BLOCK), fast_lds_bytes(dtype, tab_entries),
+                               (hipStream_t)stream, vols_dev, poses_dev, block_prefix_dev, npose, p.first, p.count, twl, tab_entries);
+            rc = hip_status(hipGetLastError());
+            if (total_blocks - first <= p.count) break;
+            first += p.count;
+        }
+        return rc;
     });
 }
 

@@ -415,7 +415,7 @@ int launch_slot(birp_server* S, Slot& s) {
             tmp.width = s.h_poses[k].W;
             tmp.height = s.h_poses[k].H;
             const long long next = (long long)pre[k - base[g]] + fast_blocks(tiles_of(tmp, gt[g].tile_w, gt[g].tile_h));
-            if (next > INT32_MAX) return fail(BIRP_ERR_UNSUPPORTED, "launch of more than 2^31 - 1 tiles");
+            if (next > INT32_MAX) return fail(BIRP_ERR_UNSUPPORTED, "launch of more than 2^31 - 1 blocks of 4 tiles");
             pre[k - base[g] + 1] = (int)next;
         }
     }
