@@ -9,7 +9,8 @@
 //              short forms of exact_math.h, std::lerp's branch structure, and the image sum
 //              in k order. Bit-identical to the reference CPU render for finite cubes.
 //  * fast   -- FP64 camera basis, ray origin and cube entry; FP32 FMA march in index space;
-//              BF16/F16/FP32 storage; FP32 Kahan sums over groups of 16 samples. Many views in one launch.
+//              BF16/F16/FP32 storage; sums in FP64 (signed cubes and CMEM: FP32 Kahan sums), rounded once.
+//              Many views in one launch.
 //
 // Wave mapping: a wave64 owns a tile of 64/S rays; S lanes ("sub-lanes") share one ray and take
 // its samples k = kb + sub, kb advancing by S each trip. In the exact kernels every sub-lane then
@@ -1688,6 +1689,16 @@ __device__ __forceinline__ FastLane fast_lane(int lane, int tw_log2) {
     return f;
 }
 
+// x + the x of the lane `step` away, and the sum of the S lanes of a ray, (0 + 1) + (2 + 3): the same bits on
+// each of its lanes (an addition of two commutes).
+__device__ __forceinline__ double pair_sum(double x, int step) { return x + __shfl_xor(x, step, 64); }
+template <int S>
+__device__ __forceinline__ double sum_lanes(double x, int sub_step) {
+    if constexpr (S >= 2) x = pair_sum(x, sub_step);
+    if constexpr (S == 4) x = pair_sum(x, 2 * sub_step);
+    return x;
+}
+
 // One wave renders tile `tile` (row-major over the image's tiles) of pose P over volume V, whose
 // offset tables the wave holds in `tab`; every lane of the wave calls it.
 template <int KV, int S, int U>
@@ -1819,84 +1830,54 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
             alive = alive && grp == 0u;
             if (__ballot(alive && (q + 1) * S < cnt) == 0ull) break;  // every ray of the wave is done
         }
-        // each sub-lane's Kahan total, then the S partials combined in sub order
-        tot = sum + nc;
-        if constexpr (S > 1) {
-            const float t1 = __shfl_xor(tot, sub_step, 64);
-            tot = (sub & 1) ? t1 + tot : tot + t1;
-            if constexpr (S == 4) {
-                const float t2 = __shfl_xor(tot, 2 * sub_step, 64);
-                tot = (sub & 2) ? t2 + tot : tot + t2;
-            }
-        }
+        // each sub-lane's sum with its compensation, the S of them in FP64: the ray's total is rounded once
+        tot = (float)sum_lanes<S>((double)sum + (double)nc, sub_step);
     }
     if constexpr (!SIGNED) {
-        // A ray's samples go in groups of 16 from its first, sample 16 g + 4 b + r to residue r: the four
-        // of a residue (neighbours on the ray, of similar size) are added plainly and their sum enters the
-        // residue's running sum by one Kahan step. Lane `sub` takes the residues sub, sub + S, ..., so
-        // the image does not depend on S, on the tile or on U, and a launch may choose them
-        // (launch_tuning): single 300x170 x 500 FP16 renders 28.8 us with one lane per ray, 17.3 with four.
-        // Groups that every ray of the wave fills need no clamp and no mask; the others run below with
-        // both, and with the same sums: a masked sample adds 0, and a ray's sums rest after its last group.
-        constexpr int R = 4 / S, B = U > R ? U / R : 1;  // residues per lane; rows b in flight together
-        float sum[R] = {}, nc[R] = {}, part[R];
+        // Sample k of a ray, from its first, belongs to residue k mod 4; the samples of a residue are added in
+        // order in FP64, then the four sums, and the total is rounded once. Lane `sub` takes the residues sub,
+        // sub + S, ..., so the image does not depend on S, on the tile or on U, and a launch may choose
+        // them (launch_tuning): single 300x170 x 500 FP16 renders 28.8 us with one lane per ray, 17.3 with
+        // four. No number of samples loses a bit of the total: relative RMS error of the sum of 17 / 150 / 400
+        // samples 2.4e-8 / 2.3e-8 / 1.8e-8, all of it the last rounding. Sums of four samples in FP32, one Kahan
+        // step each and a rounded total per residue, gave 3.8e-8 / 3.4e-8 / 2.7e-8 and were 0.5% faster (256
+        // mixed orbit views of F16 2.305 ms, 2.314 now; FP32 the same).
+        // Rows that every ray of the wave fills need no clamp and no mask; the others run below with both,
+        // and with the same sums: a masked sample adds 0.
+        constexpr int R = 4 / S, B = U > R ? U / R : 1;  // residues per lane; rows of 4 samples in flight together
+        double sum[R] = {};
         auto at = [&](float fj) {
             return fast_fetch<DT>(V, rs, tab, __builtin_fmaf(fj, dix, ix0), __builtin_fmaf(fj, diy, iy0), __builtin_fmaf(fj, diz, iz0));
         };
         FastFetch<DT> f[B * R];
         const int full = wave_min_i(cnt), most = wave_max_i(cnt);
-        int g = 0;
-        for (; g + 16 <= full; g += 16) {
-            // B rows (max(U, R) samples) per iteration, their loads in flight together: left to itself the
-            // compiler issues them one by one, each waited for before the next
+        int row = 0;
+        float fj = (float)sub;
+        for (; row + 4 * B <= full; row += 4 * B, fj += 4.0f * B) {
 #pragma unroll
-            for (int q = 0; q < R; ++q) part[q] = 0.f;
-            float fb = (float)(g + sub);
-#pragma unroll 1
-            for (int b = 0; b < 4; b += B, fb += 4.0f * B) {
+            for (int c = 0; c < B * R; ++c) f[c] = at(fj + (float)(4 * (c / R) + S * (c % R)));
+            // The next row's loads may rise above these lerps, which the few waves of 4 lanes per ray need (144x84 n =
+            // 2000 FP32 42.7 -> 38.5 us); with 2 lanes and 16-bit records the registers that takes cost more
+            // than it gives (1000x600 n = 2000 343 us with the barrier, 351 without).
+            if constexpr (DT != BIRP_DTYPE_F32 && S == 2) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int c = 0; c < B * R; ++c) f[c] = at(fb + (float)(4 * (c / R) + S * (c % R)));
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int c = 0; c < B * R; ++c) part[c % R] += fast_value<DT>(f[c]);
-            }
-#pragma unroll
-            for (int q = 0; q < R; ++q) kahan_add(part[q], sum[q], nc[q]);
+            for (int c = 0; c < B * R; ++c) sum[c % R] += (double)fast_value<DT>(f[c]);
         }
-        for (; g < most; g += 16) {
+        for (; row < most; row += 4 * B) {
+            // a lane past its ray's last sample re-reads that sample (its result is masked); an
+            // empty ray has i0 = d = 0 and samples the grid origin
+            const int js = row + sub;
 #pragma unroll
-            for (int q = 0; q < R; ++q) part[q] = 0.f;
-#pragma unroll 1
-            for (int b = 0; b < 4 && g + 4 * b < most; b += B) {
-                // a lane past its ray's last sample re-reads that sample (its result is masked); an
-                // empty ray has i0 = d = 0 and samples the grid origin
-                const int js = g + 4 * b + sub;
+            for (int c = 0; c < B * R; ++c) f[c] = at((float)min(js + 4 * (c / R) + S * (c % R), cnt - 1));
+            // here the compiler would issue the loads one by one, each waited for before the next (40x30 n = 2000
+            // 41.2 -> 54.1 us)
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int c = 0; c < B * R; ++c) f[c] = at((float)min(js + 4 * (c / R) + S * (c % R), cnt - 1));
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int c = 0; c < B * R; ++c) part[c % R] += js + 4 * (c / R) + S * (c % R) < cnt ? fast_value<DT>(f[c]) : 0.f;
-            }
-#pragma unroll
-            for (int q = 0; q < R; ++q)
-                if (g < cnt) kahan_add(part[q], sum[q], nc[q]);
+            for (int c = 0; c < B * R; ++c) sum[c % R] += (double)(js + 4 * (c / R) + S * (c % R) < cnt ? fast_value<DT>(f[c]) : 0.f);
         }
-        // the residues' Kahan totals, (0 + 1) + (2 + 3)
-        float res[R];
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-            res[q] = sum[q] + nc[q];
-            if constexpr (S > 1) {
-                const float t1 = __shfl_xor(res[q], sub_step, 64);
-                res[q] = (sub & 1) ? t1 + res[q] : res[q] + t1;
-            }
-        }
-        if constexpr (S == 1) tot = (res[0] + res[1]) + (res[2] + res[3]);
-        else if constexpr (S == 2) tot = res[0] + res[1];
-        else {
-            const float t2 = __shfl_xor(res[0], 2 * sub_step, 64);
-            tot = (sub & 2) ? t2 + res[0] : res[0] + t2;
-        }
+        if constexpr (S == 1) tot = (float)((sum[0] + sum[1]) + (sum[2] + sum[3]));
+        else if constexpr (S == 2) tot = (float)(pair_sum(sum[0], sub_step) + pair_sum(sum[1], sub_step));
+        else tot = (float)sum_lanes<4>(sum[0], sub_step);
     }
     // the step weight and the scale constant are applied once per ray (all in FP32)
     if (valid && sub == 0) P.out[(size_t)j * P.W + i] = (tot * P.w) * K;
@@ -1931,8 +1912,9 @@ __global__ __launch_bounds__(BIRP_BLOCK, 6) void k_render_fast(const DevVolume* 
     constexpr bool SIGNED = CMEM || (KV & BIRP_KDT_SIGNED) != 0;
     static_assert(!SIGNED || U == 1, "signed kernels take one sample per lane per trip");
     extern __shared__ unsigned s_tab[];
-    constexpr int chunk = BIRP_FAST_CHUNK;
-    const int turn = (int)(blockIdx.x >> 3), at = (turn / chunk * 8 + (int)(blockIdx.x & 7u)) * chunk + turn % chunk;
+    constexpr unsigned chunk = BIRP_FAST_CHUNK;
+    const unsigned turn = blockIdx.x >> 3;
+    const int at = (int)((turn / chunk * 8 + (blockIdx.x & 7u)) * chunk + turn % chunk);
     if (at >= count) return;
     const int g = first + at;
     const int k = find_view(prefix, npose, g);
