@@ -535,7 +535,10 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_cmem_zones(CmemParams m, float4*
 }
 
 // What the bounds say of a point: its zone, or (SPLIT) which of the surfaces it takes to know (ZONE_EDGE: both;
-// also for points on x = 0 or y = 0, where the reference takes an angle of 0, Cmem.cpp:224-246).
+// also for points on x = 0 or y = 0, where the reference takes an angle of 0, Cmem.cpp:224-246, and where |x y| is
+// so small that r^2 may leave the normal floats, whose reciprocal root the hardware takes for 0's). y^2 + z^2 may
+// leave them elsewhere too, beside the Sun's line: the surfaces are round there, and any cell that
+// touches ct = 1 bounds them, so it does not matter which phi the query then finds.
 enum Zone { ZONE_INSIDE, ZONE_OUTER, ZONE_SHEATH, ZONE_EDGE_MP, ZONE_EDGE_BS, ZONE_EDGE };
 struct ZoneQuery {
     float4 t;
@@ -552,7 +555,7 @@ __device__ __forceinline__ ZoneQuery zone_fetch(__amdgpu_buffer_rsrc_t rs, float
     const unsigned iu = (unsigned)__builtin_amdgcn_fmed3f(u, 0.0f, BIRP_ZONE_CT - 1.0f), iv = (unsigned)__builtin_amdgcn_fmed3f(v, 0.0f, BIRP_ZONE_CP - 1.0f);
     q.t = load16(rs, (iu * BIRP_ZONE_CP + iv) * 16u);
     q.r = r2 * q.ir;
-    q.axis = !(fabsf(x * y) > 0.0f);
+    q.axis = !(fabsf(x * y) > 0x1p-60f);
     return q;
 }
 template <bool SPLIT>
