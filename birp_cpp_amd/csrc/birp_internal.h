@@ -102,7 +102,7 @@ struct ExactView {
     int semantics;    // BIRP_SEM_*
     int vol;          // multi-view launches: index of the view's volume in the volume table
     int accumulate;   // start from out's values
-    double inv_w, inv_h;  // RN64(1 / W), RN64(1 / H)
+    double inv_w, inv_h;  // RN64(1 / (float)W), RN64(1 / (float)H)
     float per_t;      // n / L: samples per unit of t
     float margin;     // slab expansion (RE) that covers FP32 position error
     int fast_guards;  // cube without negative values whose scaled samples stay normal floats: 1: only the scale's

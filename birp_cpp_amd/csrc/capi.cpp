@@ -88,8 +88,8 @@ int exact_view(const birp_volume* vol, const birp_view* v, float* out_dev, Exact
     ev.W = v->width;
     ev.H = v->height;
     ev.n = v->samples;
-    ev.inv_w = 1.0 / v->width;
-    ev.inv_h = 1.0 / v->height;
+    ev.inv_w = 1.0 / (double)(float)v->width;  // Camera.cpp:148 divides by the size as a float
+    ev.inv_h = 1.0 / (double)(float)v->height;
     ev.per_t = (float)((double)v->samples / v->ray_length);
     ev.semantics = v->semantics;
     ev.accumulate = (v->flags & BIRP_RENDER_ACCUMULATE) ? 1 : 0;
