@@ -126,7 +126,7 @@ struct FastPose {
     int vol;          // index into the volume table
     int tiles_x;      // wave tiles across
     float w;          // step weight (t1 - t0 in double, rounded)
-    float pad;
+    float scale;      // of BIRP_KDT_F16_UNIFORM records, a power of two; else 1
     float* out;       // device image
 };
 

@@ -139,8 +139,7 @@ int fast_pose(const birp_volume* vol, const birp_view* v, int vol_index, float* 
     fp.vol = vol_index;
     fp.tiles_x = (v->width + tile_w - 1) / tile_w;
     fp.w = (float)((double)v->ray_length / v->samples);
-    if ((fast_kernel_dtype(vol->dv) & ~BIRP_KDT_SIGNED) == BIRP_KDT_F16_UNIFORM) fp.w *= vol->dv.f16_scale;  // power of two: exact
-    fp.pad = 0.f;
+    fp.scale = (fast_kernel_dtype(vol->dv) & ~BIRP_KDT_SIGNED) == BIRP_KDT_F16_UNIFORM ? vol->dv.f16_scale : 1.f;
     fp.out = out_dev;
     (void)tile_h;
     return BIRP_OK;

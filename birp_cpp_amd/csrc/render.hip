@@ -1882,8 +1882,13 @@ __device__ __forceinline__ void fast_tile(const DevVolume& V, const FastPose& P,
         else if constexpr (S == 2) tot = (float)(pair_sum(sum[0], sub_step) + pair_sum(sum[1], sub_step));
         else tot = (float)sum_lanes<4>(sum[0], sub_step);
     }
-    // the step weight and the scale constant are applied once per ray (all in FP32)
-    if (valid && sub == 0) P.out[(size_t)j * P.W + i] = (tot * P.w) * K;
+    // the step weight and the scale constant are applied once per ray (all in FP32), the records' scale last: a
+    // power of two changes no bit of a normal result, where scale * w could be subnormal
+    if (valid && sub == 0) {
+        float out = (tot * P.w) * K;
+        if constexpr (!CMEM && DT == BIRP_KDT_F16_UNIFORM) out *= P.scale;
+        P.out[(size_t)j * P.W + i] = out;
+    }
 }
 
 // The wave tiles of many views in one launch, as a plain grid: a block renders 4 consecutive tiles of one view
