@@ -760,12 +760,13 @@ extern "C" int birp_server_add_volume(birp_server* S, birp_volume* vol, int* ind
     if (vol->dev != S->dev) return fail(BIRP_ERR_INVALID_ARGUMENT, "volume on another device");
     std::lock_guard<std::mutex> lk(S->mu);
     if ((int)S->vols.size() >= S->vol_cap) return fail(BIRP_ERR_OUT_OF_MEMORY, "volume table full");
-    if (S->resident + S->held + vol->bytes > S->cfg.memory_budget)
+    const size_t charge = vol->dv.kind == SK_CMEM ? 0 : vol->bytes;  // a model's fixed table is not charged
+    if (S->resident + S->held + charge > S->cfg.memory_budget)
         return fail(BIRP_ERR_ADMISSION, "volume does not fit the memory budget");
     hipError_t e = hipStreamSynchronize(vol->dev->stream);  // a CMEM model's zone bounds are made there
     if (e == hipSuccess) e = hipMemcpy(S->d_vols + S->vols.size(), &vol->dv, sizeof(DevVolume), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(e, "volume table upload");
-    S->resident += vol->bytes;
+    S->resident += charge;
     *index = (int)S->vols.size();
     S->vols.push_back(vol);
     return BIRP_OK;

@@ -305,9 +305,9 @@ typedef struct birp_result_info {
 int birp_server_create(birp_device* dev, const birp_server_config* cfg, birp_server** out);
 int birp_server_destroy(birp_server* s);
 /* Registers a resident volume, a cube or a CMEM model (owned by the caller; must outlive the
- * server). Its device bytes
- * count against the budget; fails with BIRP_ERR_ADMISSION when it does not fit beside the
- * volumes already registered and the image buffers the slots hold. A request whose image alone
+ * server). A cube's device bytes
+ * count against the budget (a model's fixed 512 KiB do not); fails with BIRP_ERR_ADMISSION when
+ * it does not fit beside the volumes already registered and the image buffers the slots hold. A request whose image alone
  * exceeds the budget left after the volumes completes with BIRP_ERR_ADMISSION. */
 int birp_server_add_volume(birp_server* s, birp_volume* vol, int* index);
 /* Queues a request; the result buffer (H*W floats, host) must stay valid until it completes. */
