@@ -397,6 +397,7 @@ static void free_volume_buffers(birp_volume* v) {
     if (v->qtab) (void)hipFree(v->qtab);
     if (v->otab) (void)hipFree(v->otab);
     if (v->zones) (void)hipFree(v->zones);
+    if (v->zones_made) (void)hipEventDestroy(v->zones_made);
     v->linear = nullptr;
     v->quad = nullptr;
     v->oct = nullptr;
@@ -404,6 +405,7 @@ static void free_volume_buffers(birp_volume* v) {
     v->qtab = nullptr;
     v->otab = nullptr;
     v->zones = nullptr;
+    v->zones_made = nullptr;
 }
 
 namespace birp {
@@ -696,8 +698,10 @@ extern "C" int birp_cmem_create(birp_device* dev, const birp_cmem_state* s, birp
     v->dv.interp = BIRP_INTERP_TRILINEAR;
     (void)hipSetDevice(dev->ordinal);
     hipError_t e = hipMalloc(&v->zones, BIRP_ZONE_BYTES);
-    // renders follow on the device's stream; a server, whose slots have streams of their own, waits for it
-    int rc = e == hipSuccess ? launch_cmem_zones(c, v->zones, dev->stream) : hip_fail(e, "hipMalloc(zone bounds)");
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&v->zones_made, hipEventDisableTiming);
+    // renders follow on the device's stream; a server, whose slots have streams of their own, waits for the event
+    int rc = e == hipSuccess ? launch_cmem_zones(c, v->zones, dev->stream) : hip_fail(e, "zone bounds");
+    if (rc == BIRP_OK && (e = hipEventRecord(v->zones_made, dev->stream)) != hipSuccess) rc = hip_fail(e, "zone bounds");
     if (rc) {
         free_volume_buffers(v);
         delete v;

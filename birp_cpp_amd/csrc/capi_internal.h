@@ -68,7 +68,8 @@ struct birp_volume {
     float* bscale = nullptr;
     unsigned* qtab = nullptr;
     unsigned* otab = nullptr;
-    void* zones = nullptr;  // CMEM: the zone bounds
+    void* zones = nullptr;  // CMEM: the zone bounds, and the event that follows their making on the device's stream
+    hipEvent_t zones_made = nullptr;
     bool morton = false;
     size_t bytes = 0;
 };

@@ -758,13 +758,16 @@ extern "C" int birp_server_destroy(birp_server* S) {
 extern "C" int birp_server_add_volume(birp_server* S, birp_volume* vol, int* index) {
     if (!S || !vol || !index) return fail(BIRP_ERR_INVALID_ARGUMENT, "null argument");
     if (vol->dev != S->dev) return fail(BIRP_ERR_INVALID_ARGUMENT, "volume on another device");
+    // a CMEM model's zone bounds are made on the device's stream, the slots have streams of their own; what else the
+    // stream holds is not waited for, and nothing is with the lock held
+    hipError_t e = vol->zones_made ? hipEventSynchronize(vol->zones_made) : hipSuccess;
+    if (e != hipSuccess) return hip_fail(e, "zone bounds");
     std::lock_guard<std::mutex> lk(S->mu);
     if ((int)S->vols.size() >= S->vol_cap) return fail(BIRP_ERR_OUT_OF_MEMORY, "volume table full");
     const size_t charge = vol->dv.kind == SK_CMEM ? 0 : vol->bytes;  // a model's fixed table is not charged
     if (S->resident + S->held + charge > S->cfg.memory_budget)
         return fail(BIRP_ERR_ADMISSION, "volume does not fit the memory budget");
-    hipError_t e = hipStreamSynchronize(vol->dev->stream);  // a CMEM model's zone bounds are made there
-    if (e == hipSuccess) e = hipMemcpy(S->d_vols + S->vols.size(), &vol->dv, sizeof(DevVolume), hipMemcpyHostToDevice);
+    e = hipMemcpy(S->d_vols + S->vols.size(), &vol->dv, sizeof(DevVolume), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(e, "volume table upload");
     S->resident += charge;
     *index = (int)S->vols.size();

@@ -22,3 +22,65 @@ def test_models_cost_no_budget(device):
         srv.destroy()
         for v in vols:
             v.free()
+
+
+def test_registering_does_not_wait_for_the_device_stream(device):
+    """With a long queue of renders on the device's stream, volumes whose making has finished are registered, and
+    requests over them served, before the queue ends."""
+    rng = np.random.default_rng(2)
+    cube = capi.Volume.upload(device, (1e-5 * np.exp(rng.standard_normal((20, 22, 24)))).astype(np.float32), (2.0, -5.0, -4.5), (0.5,) * 3)
+    model = capi.Volume.cmem(device, capi.cmem_init())
+    image = capi.Image(device, 576, 336)
+    long = capi.make_view(576, 336, 26.5, 15.5, (0.0, -20.0, 10.0), (10.0, 0.0, 0.0), 80.0, 8000)
+    device.synchronize()
+
+    def queue():
+        t = capi.clock_s()
+        for _ in range(30):
+            capi.render_async(model, long, image)
+        return t
+
+    srv = capi.Server(device, memory_budget=1 << 30, max_batch=4, max_inflight=1, reserve_pixels=4096)
+    try:
+        t = queue()
+        device.synchronize()
+        whole = capi.clock_s() - t  # about 0.13 s
+        assert whole > 0.05
+        t = queue()
+        srv.add_volume(cube)
+        srv.add_volume(model)
+        registered = capi.clock_s() - t
+        device.synchronize()
+        total = capi.clock_s() - t
+        assert registered < 0.5 * total, (registered, total)
+    finally:
+        srv.destroy()
+        image.free()
+        model.free()
+        cube.free()
+
+
+def test_a_model_made_behind_other_work_is_served_whole(device):
+    other = capi.Volume.cmem(device, capi.cmem_init())
+    image = capi.Image(device, 576, 336)
+    long = capi.make_view(576, 336, 26.5, 15.5, (0.0, -20.0, 10.0), (10.0, 0.0, 0.0), 80.0, 2000)
+    views = [capi.make_view(190, 120, 26.5, 15.5, (0.0, -20.0, 10.0), (10.0, 0.0, 0.0), 60.0, 90, capi.SEM_EXTENDED, m)
+             for m in (capi.MATH_EXACT, capi.MATH_FAST)]
+    srv = capi.Server(device, memory_budget=1 << 30, max_batch=4, max_inflight=2)
+    models = []
+    try:
+        for density in (5.0, 9.0, 14.0):
+            for _ in range(10):
+                capi.render_async(other, long, image)
+            models.append(capi.Volume.cmem(device, capi.cmem_init(capi.cmem_params(density=density))))
+            index = srv.add_volume(models[-1])
+            ids = [srv.submit(index, v) for v in views]
+            got = [srv.wait(i, 20000) for i in ids]
+            for (status, img, _), v in zip(got, views):
+                assert status == capi.OK
+                assert np.array_equal(img.view(np.uint32), models[-1].render(v)[0].view(np.uint32))
+    finally:
+        srv.destroy()
+        image.free()
+        for m in models + [other]:
+            m.free()
