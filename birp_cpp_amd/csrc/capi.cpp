@@ -397,7 +397,6 @@ static void free_volume_buffers(birp_volume* v) {
     if (v->qtab) (void)hipFree(v->qtab);
     if (v->otab) (void)hipFree(v->otab);
     if (v->zones) (void)hipFree(v->zones);
-    if (v->zones_made) (void)hipEventDestroy(v->zones_made);
     v->linear = nullptr;
     v->quad = nullptr;
     v->oct = nullptr;
@@ -405,7 +404,6 @@ static void free_volume_buffers(birp_volume* v) {
     v->qtab = nullptr;
     v->otab = nullptr;
     v->zones = nullptr;
-    v->zones_made = nullptr;
 }
 
 namespace birp {
@@ -697,13 +695,10 @@ extern "C" int birp_cmem_create(birp_device* dev, const birp_cmem_state* s, birp
     v->dv.dtype = BIRP_DTYPE_F32;
     v->dv.interp = BIRP_INTERP_TRILINEAR;
     (void)hipSetDevice(dev->ordinal);
-    hipError_t e = hipMalloc(&v->zones, BIRP_ZONE_BYTES);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&v->zones_made, hipEventDisableTiming);
-    // renders follow on the device's stream; a server, whose slots have streams of their own, waits for the event
-    int rc = e == hipSuccess ? launch_cmem_zones(c, v->zones, dev->stream) : hip_fail(e, "zone bounds");
-    if (rc == BIRP_OK && (e = hipEventRecord(v->zones_made, dev->stream)) != hipSuccess) rc = hip_fail(e, "zone bounds");
-    if (rc) {
-        free_volume_buffers(v);
+    // allocated here, since some renders may not allocate; filled for the first render that asks the bounds
+    const hipError_t e = hipMalloc(&v->zones, BIRP_ZONE_BYTES);
+    if (e != hipSuccess) {
+        const int rc = hip_fail(e, "hipMalloc(zone bounds)");
         delete v;
         return rc;
     }
@@ -712,6 +707,23 @@ extern "C" int birp_cmem_create(birp_device* dev, const birp_cmem_state* s, birp
     *out = v;
     return BIRP_OK;
 }
+
+namespace birp {
+// A model's bounds are made once, 12 us of the stream's time, and not for models none of whose views ask them
+// (small fast ones take the model in full). In a stream capture the kernel becomes a part of the graph, and
+// the next eager launch still has to make them.
+int need_zones(birp_volume* v) {
+    if (v->dv.kind != SK_CMEM) return BIRP_OK;
+    std::lock_guard<std::mutex> lk(v->zones_mu);
+    if (v->zones_made) return BIRP_OK;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(v->dev->stream, &capture);
+    if (e != hipSuccess) return hip_fail(e, "zone bounds");
+    const int rc = launch_cmem_zones(v->dv.cmem, v->zones, v->dev->stream);
+    v->zones_made = rc == BIRP_OK && capture == hipStreamCaptureStatusNone;
+    return rc ? fail(rc, "zone bounds launch failed") : BIRP_OK;
+}
+}  // namespace birp
 
 extern "C" int birp_volume_free(birp_volume* v) {
     if (!v) return BIRP_OK;
@@ -914,6 +926,7 @@ static int render_exact_into(birp_volume* vol, const birp_view* view, float* dim
     if (take_injected_failure(dev)) return fail(BIRP_ERR_INJECTED, "injected failure");
     DevVolume dv = vol->dv;
     if (exact_force_linear() && dv.vclass != VC_NONFINITE && dv.kind == SK_CUBE) dv.vclass = VC_NONFINITE;
+    if ((rc = need_zones(vol))) return rc;
     const int lanes = default_exact_lanes(dv.kind == SK_CMEM, ev.W, ev.H);
     ExactOrder ord{};
     const ExactOrder* use = exact_order(dev, dv, ev, lanes, ord);
@@ -1320,6 +1333,8 @@ int exact_batch_setup(birp_batch* b) {
     const int n = (int)b->views.size();
     std::vector<ExactView> evs(n);
     std::vector<int> mode(n);
+    for (birp_volume* vol : b->evols)
+        if ((rc = need_zones(vol))) return rc;
     for (int k = 0; k < n; k++) {
         const birp_volume* vol = b->evols[b->vol_of[k]];
         float* out = (b->host_out_dev ? b->host_out_dev : b->d_images) + b->offsets[k];
@@ -1423,6 +1438,7 @@ int batch_setup(birp_batch* b) {
     if (b->exact) return exact_batch_setup(b);
     birp_device* dev = b->vol->dev;
     batch_release(b);
+    if (const int rc = need_zones(b->vol)) return rc;
     const birp_tuning& t = b->tuning;
     const int n = (int)b->views.size();
     std::vector<FastPose> poses(n);
@@ -1723,6 +1739,7 @@ extern "C" int birp_render_views_noalloc(birp_volume* vol, const birp_view* view
     for (int k = 0; k < count && rc == BIRP_OK; k++)
         if (views[k].math == BIRP_MATH_EXACT) rc = render_exact_into(vol, &views[k], images_dev[k], nullptr);
     if (rc || nf == 0) return rc;
+    if ((rc = need_zones(vol))) return rc;
     char* s = static_cast<char*>(dev->noalloc_scratch);
     if ((rc = noalloc_stage_head(vol->dv, prefix, s, dev->stream))) return fail(rc, "scratch staging failed");
     for (int q = 0; q < nf; q += 4)
@@ -1753,6 +1770,7 @@ static int render_fast_into(birp_volume* vol, const birp_view* view, float* dimg
     int rc = fast_pose(vol, view, 0, dimg, t.tile_w, t.tile_h, fp);
     if (rc) return rc;
     if (take_injected_failure(dev)) return fail(BIRP_ERR_INJECTED, "injected failure");
+    if (t.unroll != 4 && (rc = need_zones(vol))) return rc;  // 4: the model in full (view_tuning)
     rc = launch_fast_one(vol->dv, fast_kernel_dtype(vol->dv), fp, tiles_of(*view, t.tile_w, t.tile_h), t.tile_w, t.tile_h,
                          t.lanes_per_ray, t.unroll, dev->stream, volume_tab_entries(vol->dv));
     return rc ? fail(rc, "fast render launch failed") : BIRP_OK;

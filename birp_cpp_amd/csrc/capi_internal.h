@@ -5,6 +5,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <atomic>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -68,8 +69,9 @@ struct birp_volume {
     float* bscale = nullptr;
     unsigned* qtab = nullptr;
     unsigned* otab = nullptr;
-    void* zones = nullptr;  // CMEM: the zone bounds, and the event that follows their making on the device's stream
-    hipEvent_t zones_made = nullptr;
+    void* zones = nullptr;     // CMEM: the zone bounds
+    bool zones_made = false;   // their kernel is on the device's stream (need_zones), under zones_mu
+    std::mutex zones_mu;
     bool morton = false;
     size_t bytes = 0;
 };
@@ -127,6 +129,8 @@ int hip_fail(hipError_t e, const char* what);
 int validate_view(const birp_view* v, bool exact);
 int fast_pose(const birp_volume* vol, const birp_view* v, int vol_index, float* out_dev, int tile_w, int tile_h, FastPose& fp);
 int exact_view(const birp_volume* vol, const birp_view* v, float* out_dev, ExactView& ev);
+// Before a launch on the device's stream that asks a CMEM model's zone bounds: puts the kernel that makes them there.
+int need_zones(birp_volume* v);
 int default_exact_lanes(bool cmem, int W, int H);
 int default_exact_pipe();
 int tiles_of(const birp_view& v, int tile_w, int tile_h);

@@ -113,6 +113,7 @@ struct Request {
     uint64_t id = 0;
     birp_request req{};
     birp_volume* vol = nullptr;  // captured at submission
+    const DevVolume* dv = nullptr;
     float* result = nullptr;
     size_t pixels = 0;
     float* dev_out = nullptr;  // result lies in a birp_host_alloc buffer: its device address
@@ -211,6 +212,7 @@ struct birp_server {
     birp_device* dev = nullptr;
     birp_server_config cfg{};
     std::vector<birp_volume*> vols;
+    std::deque<DevVolume> dvols;  // theirs as in d_vols (a model with the server's zone bounds); a deque: they never move
     DevVolume* d_vols = nullptr;
     int vol_cap = 64;
     size_t resident = 0;  // device bytes of the registered volumes (under mu)
@@ -435,7 +437,7 @@ int launch_slot(birp_server* S, Slot& s) {
         e = hipMemcpyAsync(s.d_desc, s.h_desc, L.hi, hipMemcpyHostToDevice, s.stream);
     if (e != hipSuccess) return hip_fail(e, "server descriptor upload");
     if (lone) {
-        const DevVolume& dv = lone->vol->dv;
+        const DevVolume& dv = *lone->dv;
         rc = launch_exact(dv, s.h_evs[0], default_exact_lanes(dv.kind == SK_CMEM, lone->req.view.width, lone->req.view.height),
                           default_exact_pipe(), s.stream, nullptr);
         if (rc) return fail(rc, "exact launch failed");
@@ -454,7 +456,7 @@ int launch_slot(birp_server* S, Slot& s) {
         const int kdt = g / 3;
         const int total_blocks = s.h_prefix[base[g] + g + count];
         if (lone_fast) {
-            rc = launch_fast_one(lone_fast->vol->dv, kdt, s.h_poses[base[g]], tiles_of(lone_fast->req.view, t.tile_w, t.tile_h), t.tile_w, t.tile_h, t.lanes_per_ray,
+            rc = launch_fast_one(*lone_fast->dv, kdt, s.h_poses[base[g]], tiles_of(lone_fast->req.view, t.tile_w, t.tile_h), t.tile_w, t.tile_h, t.lanes_per_ray,
                                  t.unroll, s.stream, tabs[g]);
             if (rc) return fail(rc, "fast launch failed");
             continue;
@@ -750,29 +752,49 @@ extern "C" int birp_server_destroy(birp_server* S) {
         if (s.stream) (void)hipStreamDestroy(s.stream);
     }
     if (S->d_vols) (void)hipFree(S->d_vols);
+    for (const DevVolume& dv : S->dvols)
+        if (dv.kind == SK_CMEM) (void)hipFree(const_cast<void*>(dv.zones));
     for (auto& kv : S->reqs) delete kv.second;
     delete S;
+    return BIRP_OK;
+}
+
+static int register_volume(birp_server* S, birp_volume* vol, const DevVolume& dv, int* index) {
+    std::lock_guard<std::mutex> lk(S->mu);
+    if ((int)S->vols.size() >= S->vol_cap) return fail(BIRP_ERR_OUT_OF_MEMORY, "volume table full");
+    const size_t charge = vol->dv.kind == SK_CMEM ? 0 : vol->bytes;  // a model's fixed table is not charged
+    if (S->resident + S->held + charge > S->cfg.memory_budget)
+        return fail(BIRP_ERR_ADMISSION, "volume does not fit the memory budget");
+    const hipError_t e = hipMemcpy(S->d_vols + S->vols.size(), &dv, sizeof(DevVolume), hipMemcpyHostToDevice);
+    if (e != hipSuccess) return hip_fail(e, "volume table upload");
+    S->resident += charge;
+    *index = (int)S->vols.size();
+    S->vols.push_back(vol);
+    S->dvols.push_back(dv);
     return BIRP_OK;
 }
 
 extern "C" int birp_server_add_volume(birp_server* S, birp_volume* vol, int* index) {
     if (!S || !vol || !index) return fail(BIRP_ERR_INVALID_ARGUMENT, "null argument");
     if (vol->dev != S->dev) return fail(BIRP_ERR_INVALID_ARGUMENT, "volume on another device");
-    // a CMEM model's zone bounds are made on the device's stream, the slots have streams of their own; what else the
-    // stream holds is not waited for, and nothing is with the lock held
-    hipError_t e = vol->zones_made ? hipEventSynchronize(vol->zones_made) : hipSuccess;
-    if (e != hipSuccess) return hip_fail(e, "zone bounds");
-    std::lock_guard<std::mutex> lk(S->mu);
-    if ((int)S->vols.size() >= S->vol_cap) return fail(BIRP_ERR_OUT_OF_MEMORY, "volume table full");
-    const size_t charge = vol->dv.kind == SK_CMEM ? 0 : vol->bytes;  // a model's fixed table is not charged
-    if (S->resident + S->held + charge > S->cfg.memory_budget)
-        return fail(BIRP_ERR_ADMISSION, "volume does not fit the memory budget");
-    e = hipMemcpy(S->d_vols + S->vols.size(), &vol->dv, sizeof(DevVolume), hipMemcpyHostToDevice);
-    if (e != hipSuccess) return hip_fail(e, "volume table upload");
-    S->resident += charge;
-    *index = (int)S->vols.size();
-    S->vols.push_back(vol);
-    return BIRP_OK;
+    // The slots have streams of their own: a CMEM model gets a table of its own here, made before the lock is taken,
+    // whatever the device's stream holds.
+    DevVolume dv = vol->dv;
+    void* zones = nullptr;
+    if (dv.kind == SK_CMEM) {
+        (void)hipSetDevice(S->dev->ordinal);
+        hipError_t e = hipMalloc(&zones, BIRP_ZONE_BYTES);
+        if (e == hipSuccess && launch_cmem_zones(dv.cmem, zones, nullptr) != BIRP_OK) e = hipErrorLaunchFailure;
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+        if (e != hipSuccess) {
+            if (zones) (void)hipFree(zones);
+            return hip_fail(e, "zone bounds");
+        }
+        dv.zones = zones;
+    }
+    const int rc = register_volume(S, vol, dv, index);
+    if (rc && zones) (void)hipFree(zones);
+    return rc;
 }
 
 extern "C" int birp_server_submit(birp_server* S, const birp_request* req, float* result, uint64_t* id) {
@@ -811,6 +833,7 @@ extern "C" int birp_server_submit(birp_server* S, const birp_request* req, float
             return fail(BIRP_ERR_NOT_FOUND, "unknown volume index");
         }
         r->vol = S->vols[req->volume];
+        r->dv = &S->dvols[req->volume];
         r->id = S->next_id++;
         S->reqs[r->id] = r;
         S->pending.push_back(r);

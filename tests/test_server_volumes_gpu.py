@@ -84,3 +84,4 @@ def test_a_model_made_behind_other_work_is_served_whole(device):
         image.free()
         for m in models + [other]:
             m.free()
+
