@@ -220,8 +220,7 @@ int launch_zero_f32(float* p, size_t n, void* stream);
 #define BIRP_SCAN_WORDS 193
 // With copy_to, `values` may be mapped host memory; both 16-byte aligned.
 int launch_scan_class(const float* values, size_t n, unsigned* flags_dev, void* stream, float* copy_to = nullptr);
-// Checks birp_div_fma2 for the volume's spacings over every significand: ORs bit `axis` into *bad_dev for
-// an axis with a mismatch.
+// Checks birp_div_fma2 for the volume's spacings over every significand: sets *bad_dev to 1 on a mismatch.
 int launch_check_div(const DevVolume& v, unsigned* bad_dev, void* stream);
 int launch_cmem_zones(const CmemParams& m, void* zones, void* stream);
 int launch_build_quad(const DevVolume& v, void* quad, void* stream);

@@ -604,8 +604,9 @@ extern "C" int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc
         rc = hip_fail(e, "class scan init");
         goto fail_out;
     }
-    if ((rc = upload_values(dev, values, nvox, v->linear, dflags)) != BIRP_OK) goto fail_out;
+    // before the values: it runs while the host prepares their copy
     if (splits && desc->dtype == BIRP_DTYPE_F32 && (rc = launch_check_div(d, dflags + BIRP_SCAN_DIV, dev->stream)) != BIRP_OK) goto fail_out;
+    if ((rc = upload_values(dev, values, nvox, v->linear, dflags)) != BIRP_OK) goto fail_out;
     if ((e = hipMemcpyAsync(flags, dflags, sizeof(flags), hipMemcpyDeviceToHost, dev->stream)) != hipSuccess ||
         (e = hipStreamSynchronize(dev->stream)) != hipSuccess) {
         rc = hip_fail(e, "class scan");

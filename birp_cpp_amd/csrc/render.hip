@@ -1344,17 +1344,27 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_scan_class(const float* vals, si
     }
 }
 
-// birp_div_fma2 against the correctly rounded birp_div_rn64 for every significand of the dividend and
-// the three spacings; a mismatch sets bit `axis` of *bad.
-__global__ __launch_bounds__(BIRP_BLOCK) void k_check_div(DevVolume v, unsigned* bad) {
-    const unsigned m = blockIdx.x * BIRP_BLOCK + threadIdx.x;
-    if (m >= (1u << 23)) return;
-    const float a = __uint_as_float(0x3F800000u | m);
-    unsigned f = 0;
-    f |= birp_div_fma2(a, v.rhx, v.rlx) != birp_div_rn64(a, v.rdx) ? 1u : 0u;
-    f |= birp_div_fma2(a, v.rhy, v.rly) != birp_div_rn64(a, v.rdy) ? 2u : 0u;
-    f |= birp_div_fma2(a, v.rhz, v.rlz) != birp_div_rn64(a, v.rdz) ? 4u : 0u;
-    if (f) atomicOr(bad, f);
+// birp_div_fma2 against the correctly rounded birp_div_rn64 for every significand of the dividend and each of
+// the n different spacings; a mismatch sets bit 0 of *bad. 16 significands to a thread and one atomic per wave at
+// most: a grid of 2^23 threads that checked three spacings, equal or not, and counted every mismatch took 9 us
+// of a small cube's upload, 43 where a spacing has many (30 / 31).
+struct DivCheck {
+    float rh[3], rl[3];
+    double rd[3];
+    int n;
+};
+constexpr int kDivPerThread = 16;
+__global__ __launch_bounds__(BIRP_BLOCK) void k_check_div(DivCheck c, unsigned* bad) {
+    const unsigned first = blockIdx.x * BIRP_BLOCK + threadIdx.x, step = (1u << 23) / kDivPerThread;
+    bool f = false;
+    for (int k = 0; k < c.n; ++k) {
+#pragma unroll
+        for (int q = 0; q < kDivPerThread; ++q) {
+            const float a = __uint_as_float(0x3F800000u | (first + q * step));
+            f = f || birp_div_fma2(a, c.rh[k], c.rl[k]) != birp_div_rn64(a, c.rd[k]);
+        }
+    }
+    if (__ballot(f) != 0ull && lane_id() == 0 && __hip_atomic_load(bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) atomicOr(bad, 1u);
 }
 
 // The layout builders: a block makes the records of 4 bricks in a row along x. It reads their corners
@@ -2222,7 +2232,18 @@ int launch_scan_class(const float* values, size_t n, unsigned* flags_dev, void* 
 }
 
 int launch_check_div(const DevVolume& v, unsigned* bad_dev, void* stream) {
-    hipLaunchKernelGGL(k_check_div, dim3((1u << 23) / BIRP_BLOCK), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, v, bad_dev);
+    DivCheck c{{v.rhx}, {v.rlx}, {v.rdx}, 1};
+    auto add = [&](float rh, float rl, double rd) {
+        for (int k = 0; k < c.n; k++)
+            if (c.rd[k] == rd) return;  // RN64(1 / spacing) tells floats apart
+        c.rh[c.n] = rh;
+        c.rl[c.n] = rl;
+        c.rd[c.n++] = rd;
+    };
+    add(v.rhy, v.rly, v.rdy);
+    add(v.rhz, v.rlz, v.rdz);
+    const unsigned grid = (1u << 23) / kDivPerThread / BIRP_BLOCK;
+    hipLaunchKernelGGL(k_check_div, dim3(grid), dim3(BIRP_BLOCK), 0, (hipStream_t)stream, c, bad_dev);
     return hip_status(hipGetLastError());
 }
 
