@@ -1173,39 +1173,61 @@ int choose_tuning(const birp_volume* vol, const std::vector<birp_view>& views, b
     }
     if (!views.empty() && birp_autotune_lookup(vol->desc.dtype, views[bi].width, views[bi].height, views[bi].samples, &t) == BIRP_OK)
         return BIRP_OK;
-    long long rays = 0;
-    for (const birp_view& v : views) rays += (long long)v.width * v.height;
+    long long rays = 0, samples = 0;
+    for (const birp_view& v : views) {
+        rays += (long long)v.width * v.height;
+        samples += (long long)v.width * v.height * v.samples;
+    }
     // Untuned: the images of signed cubes and CMEM models depend on the lanes per ray, which no number of views
-    // changes. us with 1 / 2 / 4 lanes, signed cube: 16 of 144x84 n = 200 60 / 43 / 44, 16 of 288x168 n = 320
-    // 133 / 119 / 140; CMEM model: 4 of 72x42 n = 200 133 / 71 / 42, 16 of 288x168 n = 320 365 / 350 / 346.
+    // changes. us with 1 / 2 / 4 lanes, signed cube: 16 of 144x84 n = 200 72 / 52 / 57, 16 of 288x168 n = 400
+    // 191 / 165 / 207; 576x336, n = 100, 2 views 40 / 42 / 53, 16 views 163 / 187 / 302, n = 400 114 / 103 / 118
+    // and 538 / 558 / 754. CMEM model: 4 of 72x42 n = 200 133 / 71 / 42, 16 of 288x168 n = 320 365 / 350 / 346.
     const int kind = fast_kernel_dtype(vol->dv);
-    t = tuning_is_free(kind) ? launch_tuning(rays) : kind == BIRP_KDT_CMEM ? birp_tuning{4, 4, 4, 1} : birp_tuning{4, 8, 2, 1};
+    if (tuning_is_free(kind)) t = launch_tuning(rays, samples);
+    else if (kind == BIRP_KDT_CMEM) t = birp_tuning{4, 4, 4, 1};
+    else {
+        const birp_view& v = views[bi];
+        const long long r = (long long)v.width * v.height;
+        t = r >= 150000 && 7LL * v.samples * v.samples <= r ? birp_tuning{8, 8, 1, 1} : birp_tuning{4, 8, 2, 1};
+    }
     return BIRP_OK;
 }
 
-// A launch's fast render over a cube without negative values, by its rays (its images do not depend on the
-// tuning): few rays are a few waves waiting on each sample's loads, and 4 lanes per ray over 4x4 rays cut
-// the chain of each ray's samples by four; where the waves fill the SIMDs every lane's FP64 ray setup counts,
-// and fewer lanes per ray repeat it less. us per launch (FP16, 190^3 cube, orbit views), by lanes per ray
-// (tile):
-//                            rays    1 (8x8)  2 (4x8)  4 (4x4)
-//   144x84,  n = 320, 1       12 k    21.7     16.8     14.1
-//   288x168, n = 320, 2       97 k    22.7     19.3     19.6
-//   288x168, n = 800, 4      194 k    70.4     55.9     52.5
-//   576x336, n = 800, 1      194 k    43.4     39.3     39.6
-//   288x168, n = 320, 16     774 k    79.4     72.9     80.2
-//   576x336, n = 800, 16     3.1 M   505      487      521
-//   64 mixed orbit views     5.4 M   595      593      690   (BF16 616, 652, 759)
-//   256 mixed orbit views   21.7 M  2238     2308     2710
-birp_tuning launch_tuning(long long rays) {
-    if (rays <= 150000) return birp_tuning{4, 4, 4, 4};
-    if (rays <= 4000000) return birp_tuning{4, 8, 2, 4};
+// A launch's fast render over a cube without negative values, by its rays and their samples (its images do not
+// depend on the tuning). Few rays are a few waves waiting on each sample's loads, and 4 lanes per ray over 4x4 rays
+// cut the chain of each ray's samples by four; every lane repeats its ray's FP64 setup, worth about 40 samples,
+// which counts where the waves fill the SIMDs, the more the fewer samples follow it. us per launch over a
+// 200^3 cube with 1 (8x8) / 2 (4x8) / 4 (4x4) lanes:
+//                           rays            FP32                     FP16
+//   144x84,  n = 40          12 k     6.5 /   5.7 /   5.9      6.1 /   5.5 /   5.5
+//   144x84,  n = 400         12 k    33.0 /  19.0 /  11.6     34.4 /  19.4 /  11.3
+//   300x170, n = 100         51 k    11.1 /   8.7 /   8.7     10.4 /   8.4 /   8.2
+//   300x170, n = 400         51 k    32.0 /  19.9 /  18.2     31.7 /  20.2 /  16.1
+//   400x240, n = 200         96 k    18.2 /  14.3 /  14.5     17.6 /  13.5 /  13.4
+//   576x336, n = 40         194 k     8.5 /   9.3 /  12.7      7.5 /   9.1 /  12.3
+//   576x336, n = 200        194 k    21.7 /  22.2 /  24.3     21.0 /  19.6 /  21.2
+//   576x336, n = 800        194 k    71.9 /  71.5 /  70.7     66.4 /  57.4 /  55.3
+//   1000x600, n = 40        600 k    16.4 /  19.9 /  30.2     14.9 /  19.5 /  29.6
+//   1000x600, n = 400       600 k   106.8 / 100.4 / 100.8     84.5 /  76.9 /  81.0
+//   16 of 288x168, n = 100  774 k    47.7 /  51.7 /  68.0     40.0 /  44.1 /  60.5
+//   16 of 288x168, n = 400  774 k   139.4 / 132.3 / 141.0    104.8 / 100.9 / 117.4
+//   16 of 576x336, n = 200  3.1 M   234   / 244   / 291      182   / 199   / 253
+//   16 of 576x336, n = 800  3.1 M   867   / 866   / 881      638   / 624   / 680
+//   64 of 576x336, n = 400   12 M  1719   /1742   /1860     1260   /1332   /1562
+// Up to 10,000 rays of 500 samples and more the 4 lanes' tiles are 8x2 (72x42, n = 2000, FP16 41.8 -> 37.6 us, FP32 the
+// same; n = 160 9.0 -> 9.4, 200x120 1% slower).
+birp_tuning launch_tuning(long long rays, long long samples) {
+    const double n = (double)samples / (double)rays;
+    if (rays <= 10000 && n >= 500) return birp_tuning{8, 2, 4, 4};
+    if (rays <= 50000 || (double)rays <= 300 * n) return birp_tuning{4, 4, 4, 4};
+    if (rays < 150000 || 16 * n * n > (double)rays) return birp_tuning{4, 8, 2, 4};
     return birp_tuning{8, 8, 1, 4};
 }
 
 // A signed cube's view takes 4 lanes per ray up to 20,000 rays and 2 above, where a launch of many views would
-// pay for 4 (us per single view with 1 / 2 / 4 lanes: 144x84 n = 800 69 / 40 / 27, 288x168 n = 320 36 / 24 /
-// 19, 576x336 n = 400 42 / 36 / 43; of many, choose_tuning).
+// pay for 4, but 1 for many rays of few samples (us per single view with 1 / 2 / 4 lanes: 144x84 n = 800 181 / 90 /
+// 48, 300x170 n = 400 90 / 48 / 28, 576x336 n = 400 87 / 55 / 65, 1000x600 n = 40 20 / 23 / 33 and n = 100 48 / 45 /
+// 67; of many, choose_tuning).
 // A CMEM model's chains of transcendentals want more waves per SIMD than a cube's gathers: its views take
 // 4 lanes per ray over 4x4 rays whatever their size (576x336 at n = 800 without the zone bounds: 0.724 ms,
 // against 0.817 ms with 1 lane and 0.733 ms with 2). Its unroll is how a single view's kernel asks the zone
@@ -1213,7 +1235,8 @@ birp_tuning launch_tuning(long long rays) {
 birp_tuning view_tuning(const birp_view& v, const DevVolume& vol) {
     const long long rays = (long long)v.width * v.height;
     if (vol.kind == SK_CMEM) return birp_tuning{4, 4, 4, rays <= 10000 ? 4 : (rays <= 60000 ? 2 : 1)};
-    return rays <= 20000 ? birp_tuning{4, 4, 4, 1} : birp_tuning{4, 8, 2, 1};
+    if (rays <= 20000) return birp_tuning{4, 4, 4, 1};
+    return rays >= 150000 && 64LL * v.samples * v.samples <= rays ? birp_tuning{8, 8, 1, 1} : birp_tuning{4, 8, 2, 1};
 }
 
 void batch_release(birp_batch* b) {
@@ -1716,13 +1739,16 @@ extern "C" int birp_render_views_noalloc(birp_volume* vol, const birp_view* view
     birp_tuning gt[3] = {};
     int nf = 0;
     const bool free_tuning = tuning_is_free(fast_kernel_dtype(vol->dv));  // then all fast views are one launch
-    long long rays = 0;
-    for (int k = 0; k < count; k++)
-        if (views[k].math == BIRP_MATH_FAST) rays += (long long)views[k].width * views[k].height;
+    long long rays = 0, samples = 0;
+    for (int k = 0; k < count; k++) {
+        if (views[k].math != BIRP_MATH_FAST) continue;
+        rays += (long long)views[k].width * views[k].height;
+        samples += (long long)views[k].width * views[k].height * views[k].samples;
+    }
     for (int g = 0; g < 3; g++) {  // lanes per ray 1, 2, 4: poses of group g are contiguous
         for (int k = 0; k < count; k++) {
             if (views[k].math != BIRP_MATH_FAST) continue;
-            const birp_tuning t = free_tuning ? launch_tuning(rays) : view_tuning(views[k], vol->dv);
+            const birp_tuning t = free_tuning ? launch_tuning(rays, samples) : view_tuning(views[k], vol->dv);
             if (t.lanes_per_ray != (1 << g)) continue;
             int rc = fast_pose(vol, &views[k], 0, images_dev[k], t.tile_w, t.tile_h, poses[nf]);
             if (rc) return rc;
@@ -1766,7 +1792,8 @@ extern "C" int birp_render_views_noalloc(birp_volume* vol, const birp_view* view
 static int render_fast_into(birp_volume* vol, const birp_view* view, float* dimg) {
     birp_device* dev = vol->dev;
     if (view->flags & BIRP_RENDER_ACCUMULATE) return fail(BIRP_ERR_UNSUPPORTED, "fast renders do not accumulate");
-    const birp_tuning t = tuning_is_free(fast_kernel_dtype(vol->dv)) ? launch_tuning((long long)view->width * view->height) : view_tuning(*view, vol->dv);
+    const long long rays = (long long)view->width * view->height;
+    const birp_tuning t = tuning_is_free(fast_kernel_dtype(vol->dv)) ? launch_tuning(rays, rays * view->samples) : view_tuning(*view, vol->dv);
     FastPose fp;
     int rc = fast_pose(vol, view, 0, dimg, t.tile_w, t.tile_h, fp);
     if (rc) return rc;

@@ -136,9 +136,9 @@ int default_exact_pipe();
 int tiles_of(const birp_view& v, int tile_w, int tile_h);
 bool take_injected_failure(birp_device* dev);
 int choose_tuning(const birp_volume* vol, const std::vector<birp_view>& views, birp_tuning& t);
-// The tuning of a fast render of `rays` rays over a cube without negative values, alone or as a launch of
-// several views (the images do not depend on it).
-birp_tuning launch_tuning(long long rays);
+// The tuning of a fast render of `rays` (> 0) rays with `samples` samples in all over a cube without negative values,
+// alone or as a launch of several views (the images do not depend on it).
+birp_tuning launch_tuning(long long rays, long long samples);
 // The tuning of a view's fast render over a signed cube or a CMEM model, whose images depend on it: from the view alone.
 birp_tuning view_tuning(const birp_view& v, const birp::DevVolume& vol);
 inline bool tuning_is_free(int kernel_dtype) { return !(kernel_dtype & (BIRP_KDT_SIGNED | BIRP_KDT_CMEM)); }

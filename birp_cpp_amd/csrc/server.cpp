@@ -276,7 +276,7 @@ int slot_alloc_images(Slot& s, size_t pixels) {
 // Kernel groups of a batch: storage kernel x lanes per ray (1, 2, 4). A request over a signed cube or a CMEM
 // model has its tuning from its own view (view_tuning), so that it renders the same whatever shares its
 // launch; the others' images do not depend on the tuning, and all of a storage kernel are one group
-// (lane index 0) tuned for its rays (launch_tuning).
+// (lane index 0) tuned for its rays and samples (launch_tuning).
 constexpr int kGroups = BIRP_KDT_COUNT * 3;
 int lane_index(int lanes) { return lanes == 4 ? 2 : (lanes == 2 ? 1 : 0); }
 int request_group(const Request* r, birp_tuning* t) {
@@ -319,14 +319,15 @@ int launch_slot(birp_server* S, Slot& s) {
     if (rc) return rc;
     int base[kGroups + 1] = {}, fill[kGroups];
     birp_tuning gt[kGroups];
-    long long rays[kGroups] = {};
+    long long rays[kGroups] = {}, samples[kGroups] = {};
     for (Request* r : s.reqs) {
         if (exact_request(r)) continue;
         birp_tuning t{};
         const int g = request_group(r, &t);
         base[g + 1]++;
         rays[g] += (long long)r->req.view.width * r->req.view.height;
-        gt[g] = tuning_is_free(g / 3) ? launch_tuning(rays[g]) : t;
+        samples[g] += (long long)r->req.view.width * r->req.view.height * r->req.view.samples;
+        gt[g] = tuning_is_free(g / 3) ? launch_tuning(rays[g], samples[g]) : t;
     }
     for (int g = 0; g < kGroups; g++) {
         base[g + 1] += base[g];

@@ -85,3 +85,26 @@ def test_a_model_made_behind_other_work_is_served_whole(device):
         for m in models + [other]:
             m.free()
 
+
+
+def test_signed_views_of_every_lanes_class_in_one_launch(device):
+    """A signed cube's views take 4, 2 or 1 lanes per ray by their own rays and samples (20,000 rays; 150,000 and 64 n^2
+    rays): served together, each equals its single render."""
+    rng = np.random.default_rng(4)
+    vals = (1e-5 * np.exp(rng.standard_normal((30, 32, 34)))).astype(np.float32)
+    vals[10:14, 9:13, 11:16] *= -1
+    vol = capi.Volume.upload(device, vals, (2.0, -8.0, -7.0), (0.5, 0.5, 0.45))
+    views = [capi.make_view(w, h, 50.0, 40.0, (5.0, -18.0, 6.0), (10.0, 0.0, 0.0), 40.0, n, capi.SEM_EXTENDED, capi.MATH_FAST)
+             for w, h, n in ((200, 100, 60), (201, 100, 17), (499, 300, 20), (500, 300, 48), (500, 300, 49), (500, 400, 55), (500, 400, 300), (40, 30, 300))]
+    want = [vol.render(v)[0] for v in views]
+    srv = capi.Server(device, memory_budget=1 << 30, max_batch=8, max_inflight=1, batch_window_ms=50.0)
+    try:
+        index = srv.add_volume(vol)
+        ids = [srv.submit(index, v) for v in views]
+        for k, rid in enumerate(ids):
+            status, img, _ = srv.wait(rid, 20000)
+            assert status == capi.OK and want[k].any()
+            assert np.array_equal(img.view(np.uint32), want[k].view(np.uint32)), k
+    finally:
+        srv.destroy()
+        vol.free()
