@@ -170,6 +170,10 @@ int exact_wave_slots(int W, int H, int lanes_per_ray);
 enum SampleMode { SM_QUAD_POS = 0, SM_QUAD_NN, SM_NEAR_NN, SM_QUAD_GEN, SM_LIN_TRI, SM_LIN_NEAREST, SM_CMEM };
 constexpr bool mode_nonneg(int mode) { return mode == SM_QUAD_POS || mode == SM_QUAD_NN || mode == SM_NEAR_NN; }
 int exact_mode_of(const DevVolume& v, const ExactView& ev);
+// Blocks of 4 waves per CU that a many-view exact launch over a cube keeps resident at `lanes` per ray with its samples
+// in flight: the kernels' launch bounds. SM_QUAD_NN with 8 lanes takes 74 registers (6 waves per SIMD), the other
+// modes without negative samples at most 72 (7), the rest fewer.
+constexpr int exact_resident_blocks(int mode, int lanes) { return mode == SM_QUAD_NN && lanes == 8 ? 6 : 7; }
 // Lanes per ray of multi-view exact launches of many tiles: 4 for CMEM, 2 for cubes (the measured
 // best of each). Exact batches of few small images take 4 for cubes too (exact_batch_setup).
 inline int exact_multi_lanes(int mode) { return mode == SM_CMEM ? 4 : 2; }

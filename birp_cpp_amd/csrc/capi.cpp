@@ -1378,14 +1378,14 @@ int exact_batch_setup(birp_batch* b) {
         G.mode = m;
         G.first = (int)b->order.size();
         G.lanes = exact_multi_lanes(m);
-        // A cube group small enough that the GPU holds all its blocks at once (7 blocks of 4 waves
-        // per CU, the occupancy of the 4-samples-in-flight kernel) renders like single views:
+        // A cube group small enough that the GPU holds all its blocks at once (exact_resident_blocks)
+        // renders like single views:
         // 8 lanes per ray when every image has at most 20,000 rays and the 8-lane tiles fit, else 4
         // when every image has at most 60,000 rays, 4 samples in flight, and one snake deal over
         // the CUs (exact_batch_plan). Larger groups keep 2 and 2 (the orbit batch measured 1-2%
         // slower with 4 in flight and 10% slower with 4 lanes).
         if (m != SM_CMEM && dev->ncu > 0) {
-            const long long cap = 7LL * dev->ncu;
+            auto fits = [&](long long blocks, int lanes) { return blocks <= (long long)exact_resident_blocks(m, lanes) * dev->ncu; };
             long long t2 = 0, t4 = 0, t8 = 0;
             bool small = true, tiny = true;
             for (int k = 0; k < n; k++) {
@@ -1397,9 +1397,9 @@ int exact_batch_setup(birp_batch* b) {
                 small = small && rays <= 60000;
                 tiny = tiny && rays <= 20000;
             }
-            if (tiny && t8 <= cap) G.lanes = 8;
-            else if (small && t4 <= cap) G.lanes = 4;
-            G.resident = (G.lanes == 8 ? t8 : G.lanes == 4 ? t4 : t2) <= cap;
+            if (tiny && fits(t8, 8)) G.lanes = 8;
+            else if (small && fits(t4, 4)) G.lanes = 4;
+            G.resident = fits(G.lanes == 8 ? t8 : G.lanes == 4 ? t4 : t2, G.lanes);
             if (G.resident && mode_nonneg(m)) G.pipe = 4;
         }
         prefix.push_back(0);

@@ -888,7 +888,7 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
 // 6 to a SIMD, would lose 2%.
 constexpr int exact_waves(int S, int mode) {
     if (mode == SM_CMEM) return S <= 4 ? 8 : 1;
-    return !mode_nonneg(mode) || S == 16 ? 1 : (mode == SM_QUAD_NN && S == 8 ? 6 : 7);
+    return !mode_nonneg(mode) || S == 16 ? 1 : exact_resident_blocks(mode, S);
 }
 
 // One view: block b renders tile lb(b).

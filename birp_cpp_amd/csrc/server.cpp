@@ -361,10 +361,10 @@ int launch_slot(birp_server* S, Slot& s) {
         elanes[m] = exact_multi_lanes(m);
         epipe[m] = 2;
         if (m == SM_CMEM || S->dev->ncu <= 0) continue;
-        const long long cap = 7LL * S->dev->ncu;
-        if (etiny[m] && et8[m] <= cap) elanes[m] = 8;
-        else if (esmall[m] && et4[m] <= cap) elanes[m] = 4;
-        if (mode_nonneg(m) && (elanes[m] == 8 ? et8[m] : elanes[m] == 4 ? et4[m] : et2[m]) <= cap) epipe[m] = 4;
+        auto fits = [&](long long blocks, int lanes) { return blocks <= (long long)exact_resident_blocks(m, lanes) * S->dev->ncu; };
+        if (etiny[m] && fits(et8[m], 8)) elanes[m] = 8;
+        else if (esmall[m] && fits(et4[m], 4)) elanes[m] = 4;
+        if (mode_nonneg(m) && fits(elanes[m] == 8 ? et8[m] : elanes[m] == 4 ? et4[m] : et2[m], elanes[m])) epipe[m] = 4;
     }
     int nexact = 0;
     for (int m = 0; m < kModes; m++) nexact += ecount[m];
