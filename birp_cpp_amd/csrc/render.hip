@@ -2347,10 +2347,16 @@ int launch_fast_one(const DevVolume& v, int dtype, const FastPose& pose, int tot
     if (twl < 0 || tab_entries < 0 || tab_entries > BIRP_FAST_TAB || total_tiles < 0) return BIRP_ERR_INVALID_ARGUMENT;
     if (total_tiles == 0) return BIRP_OK;
     const int blocks = fast_blocks(total_tiles), grid = (blocks + 7) / 8 * 8;
+    // the variants that launch_tuning and view_tuning ask for: 4 samples in flight, CMEM with 4 lanes per ray
     return with_variant(dtype, lanes_per_ray, unroll, [&](auto kv, auto s, auto u) {
-        hipLaunchKernelGGL((k_render_fast_one<kv.value, s.value, u.value>), dim3(grid), dim3(BIRP_BLOCK), fast_lds_bytes(dtype, tab_entries),
-                           (hipStream_t)stream, v, pose, total_tiles, twl, tab_entries);
-        return hip_status(hipGetLastError());
+        constexpr int KV = kv.value, S = s.value, U = u.value;
+        if constexpr (KV == BIRP_KDT_CMEM ? S == 4 : (KV & BIRP_KDT_SIGNED) || U == 4) {
+            hipLaunchKernelGGL((k_render_fast_one<KV, S, U>), dim3(grid), dim3(BIRP_BLOCK), fast_lds_bytes(dtype, tab_entries),
+                               (hipStream_t)stream, v, pose, total_tiles, twl, tab_entries);
+            return hip_status(hipGetLastError());
+        } else {
+            return (int)BIRP_ERR_INVALID_ARGUMENT;
+        }
     });
 }
 
