@@ -256,9 +256,6 @@ def cpu_reference_container():
 def bench_batched(capi, W, dev, vals, org, spc, fp32_vol):
     vol16 = capi.Volume.upload(dev, vals, org, spc, dtype=capi.DTYPE_F16)
     views = W.orbit_views_mixed(256)
-    tune = os.path.join(ROOT, "birp_cpp_amd", "tuning.jsonl")
-    if os.path.exists(tune):
-        capi.lib().birp_autotune_load(tune.encode())
     b = capi.Batch(vol16, views)
     for _ in range(2):
         b.launch()

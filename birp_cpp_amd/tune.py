@@ -1,27 +1,24 @@
 """Tune the fast-path kernels (tile shape, lanes per ray, unroll) for the standard workloads and
 write a table that batches read after birp_autotune_load:
 
-    python -m birp_cpp_amd.tune [--out birp_cpp_amd/tuning.jsonl]
+    python -m birp_cpp_amd.tune [--out tuning.jsonl]
 
 The views cover every (image-size class, samples class) the workloads use: the 256 orbit poses
 of the batched workload (three image sizes, steps 0.1 and 0.25 RE), the 1600-sample views
 of the precision workload, and 0.5 RE steps as the serving workload draws them. Each
 class is tuned for FP32, BF16 and F16 storage on the 256^3 shell cube, by birp_autotune (every
 candidate timed with HIP events on a batch of that class's views). No table ships with the package: without
-one a batch's tuning follows its number of rays, which a table of per-view classes does not know, and that
+one a batch's tuning follows its rays and samples in all, which a table of per-view classes does not know, and that
 measured no slower in any class (8 orbit views of F16 97 us against 104, two of 512^3 at 1,600 samples
 150 against 165, 256 orbit views the same).
 """
 from __future__ import annotations
 
 import argparse
-import os
 import sys
 
 from birp_cpp_amd import capi
 from birp_cpp_amd import workloads as W
-
-HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 def tuning_views():
@@ -32,10 +29,15 @@ def tuning_views():
     return views
 
 
-def main(argv=None) -> int:
+def parser() -> argparse.ArgumentParser:
     ap = argparse.ArgumentParser(description=__doc__.split("\n\n")[0])
-    ap.add_argument("--out", default=os.path.join(HERE, "tuning.jsonl"))
-    args = ap.parse_args(argv)
+    # in the working folder, not in the package: nothing reads a table that was not asked for
+    ap.add_argument("--out", default="tuning.jsonl")
+    return ap
+
+
+def main(argv=None) -> int:
+    args = parser().parse_args(argv)
     dev = capi.Device(0)
     vals, org, spc, _ = W.cube_256()
     views = tuning_views()
