@@ -882,12 +882,13 @@ __device__ __forceinline__ void exact_block(const DevVolume& v, const ExactView&
 }
 
 // Waves per SIMD the exact kernels' registers leave room for: 7 where no spill follows (72 VGPRs); the rare
-// branch of SM_QUAD_NN and the shuffles of 8 and 16 lanes per ray take more. CMEM with up to 4 lanes per ray
-// spills 5 registers of its surfaces for 8 waves, which wait less on the chains of its zones: 576x336 n = 800
-// 0.476 -> 0.458 ms, 8 orbit views 0.312 -> 0.297 (6 waves; 7 are between); small images, whose waves fit
-// 6 to a SIMD, would lose 2%.
-constexpr int exact_waves(int S, int mode) {
-    if (mode == SM_CMEM) return S <= 4 ? 8 : 1;
+// branch of SM_QUAD_NN and the shuffles of 8 and 16 lanes per ray take more. CMEM with up to 4 lanes per ray waits on
+// the chains of its zones: 7 waves in single views, 8 (spilling 1 register of its surfaces) in launches of many.
+// us with 6 / 7 / 8 waves, means of 3 poses: 320x200 n = 50 24.1 / 24.3 / 24.9, 400x240 n = 400 145.4 / 145.2 / 148.6,
+// 576x336 n = 100 76.8 / 76.4 / 76.8, n = 800 467 / 449 / 454, 1000x600 n = 200 340 / 328 / 328; 16 views of 288x168
+// n = 100 254 / 244 / 242, 4 of 576x336 n = 100 244 / 234 / 230, 8 of 288x168 n = 320 420 / 407 / 409.
+constexpr int exact_waves(int S, int mode, bool many) {
+    if (mode == SM_CMEM) return S <= 4 ? (many ? 8 : 7) : 1;
     return !mode_nonneg(mode) || S == 16 ? 1 : exact_resident_blocks(mode, S);
 }
 
@@ -900,7 +901,7 @@ constexpr int exact_waves(int S, int mode) {
 // even and backward when odd, so that every CU draws one tile from each round and the heavy
 // rounds are spread evenly (the longest-processing-time-first rule). The grid is then nblocks.
 template <int S, int MODE, int P = 1>
-__global__ __launch_bounds__(BIRP_BLOCK, exact_waves(S, MODE)) void k_render_exact(DevVolume v, ExactView ev, int wg_x, int nblocks,
+__global__ __launch_bounds__(BIRP_BLOCK, exact_waves(S, MODE, false)) void k_render_exact(DevVolume v, ExactView ev, int wg_x, int nblocks,
                                                              const int* __restrict__ order, int ncu) {
     if ((int)blockIdx.x >= nblocks) return;
     int lb = blockIdx.x;
@@ -1074,7 +1075,7 @@ __device__ __forceinline__ int find_view(const int* __restrict__ prefix, int n, 
 // more tiles in flight than one view has, the SIMDs stay fed while the longest rays of a view finish.
 // `order` (may be null): block b renders item order[b] instead of item b (a batch's tile plan).
 template <int S, int MODE, int P = 1>
-__global__ __launch_bounds__(BIRP_BLOCK, exact_waves(S, MODE)) void k_render_exact_multi(const DevVolume* __restrict__ vols,
+__global__ __launch_bounds__(BIRP_BLOCK, exact_waves(S, MODE, true)) void k_render_exact_multi(const DevVolume* __restrict__ vols,
                                                                    const ExactView* __restrict__ views,
                                                                    const int* __restrict__ prefix, int nview, int total,
                                                                    const int* __restrict__ order) {
