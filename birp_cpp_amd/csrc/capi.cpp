@@ -748,27 +748,10 @@ extern "C" int birp_volume_sample(birp_volume* v, const float* xyz, long long n,
     if (v->dv.kind == SK_CUBE && !v->dv.linear) return fail(BIRP_ERR_UNSUPPORTED, "point sampling needs an FP32 volume");
     birp_device* dev = v->dev;
     (void)hipSetDevice(dev->ordinal);
-    const size_t bytes = (size_t)n * 16;
-    int rc;
-    // Up to 2^18 points (4 MiB of the device's pinned staging) the kernel reads the points and writes their samples
-    // through the mapping. Copies of pageable arrays cost two engine trips, and what the runtime makes of them depends
-    // on the process: until its first large one it takes 6 ms once and 95 us per call of 10,000 points, 38 after; a
-    // cube uploaded through the ring is not such a copy. us per call of 1,000 / 10,000 / 200,000 points 37 / 95 /
-    // 150 -> 19 / 22 / 127, a process's first 84 / 6,400 / 7,500 -> 127 / 180 / 1,550.
-    constexpr long long kStagedPoints = 1 << 18;
-    if (n <= kStagedPoints && pinned_staging(dev, 256 + bytes) == BIRP_OK && dev->pinned_dev) {
-        float* host = (float*)((char*)dev->pinned + 256);
-        float* mapped = (float*)((char*)dev->pinned_dev + 256);
-        memcpy(host, xyz, (size_t)n * 12);
-        if ((rc = launch_sample_points(v->dv, mapped, n, mapped + 3 * n, dev->stream)) != BIRP_OK) return fail(rc, "sample launch failed");
-        const hipError_t e = hipStreamSynchronize(dev->stream);
-        if (e != hipSuccess) return hip_fail(e, "sample");
-        memcpy(out, host + 3 * n, (size_t)n * 4);
-        return BIRP_OK;
-    }
-    (void)hipGetLastError();
     void* buf = nullptr;
-    if ((rc = device_scratch(dev, bytes, &buf))) return rc;
+    size_t bytes = (size_t)n * 16;
+    int rc = device_scratch(dev, bytes, &buf);
+    if (rc) return rc;
     float* dxyz = (float*)buf;
     float* dout = dxyz + 3 * n;
     hipError_t e = hipMemcpyAsync(dxyz, xyz, (size_t)n * 12, hipMemcpyHostToDevice, dev->stream);
