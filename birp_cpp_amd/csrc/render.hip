@@ -486,7 +486,10 @@ __device__ __forceinline__ Range range_pow(Range x, double e) {
 // and cp are within 1e-6), the arc cosines' arguments by 2e-6, the radii by 1e-4 RE + 3e-5 of their terms
 // (FP32 powers and exponentials are within 1e-5). Where the model leaves the reals or is too steep for that
 // the cell bounds nothing: at the cusps, whose arc cosine's argument rounds past 1 in the reference
-// (NaN), and in the last cells of the tail, where 2 / (1 + ct) diverges and a power's base may be negative.
+// (NaN), in the last cells of the tail, where 2 / (1 + ct) diverges and a power's base may be negative, where an
+// exponent multiplies the rounding of its base beyond the slack, and where a product that is finite in double leaves
+// FP32's range: with a bow shock exponent of 8.5 (10,000 particles per cm^3), ry rz does in the tail, and the
+// reference's shock is NaN or 0 there.
 __global__ __launch_bounds__(BIRP_BLOCK) void k_cmem_zones(CmemParams m, float4* zones) {
     const int cell = blockIdx.x * BIRP_BLOCK + threadIdx.x;
     if (cell >= BIRP_ZONE_CT * BIRP_ZONE_CP) return;
@@ -513,14 +516,19 @@ __global__ __launch_bounds__(BIRP_BLOCK) void k_cmem_zones(CmemParams m, float4*
     const Range base = half + (2.0 * m.a5) * (st * ct * grow);
     known = known && base.lo > 1e-4;
     const Range power = (double)m.p1 * (Range{m.beta_c[0], m.beta_c[0]} + (double)m.beta_c[1] * cp + (double)m.beta_c[3] * (sp * sp));
+    auto within = [&](Range a, double least, double most) { known = known && fmin(fabs(a.lo), fabs(a.hi)) >= least && fmax(fabs(a.lo), fabs(a.hi)) <= most; };
+    within(power, 0.0, 256.0);
     const Range f = range_exp(power * Range{log(fmax(base.lo, 1e-300)), log(fmax(base.hi, 1e-300))});
     const Range dip_n = range_exp(((double)m.p3 * m.dn) * range_pow(north, m.a21)), dip_s = range_exp(((double)m.p3 * m.ds) * range_pow(south, m.a21));
+    for (Range a : {f, dip_n, dip_s}) within(a, 0.0, 0x1p100);
     const Range far = ((double)m.p0 * m.r0_lin) * f, q = ((double)m.p2 * m.charlie) * (dip_n + dip_s);
     const Range mp = far + q;
     const double mp_wide = 1e-4 + 3e-5 * (fmax(fabs(far.lo), fabs(far.hi)) + fmax(fabs(q.lo), fabs(q.hi)));
     const Range flare{2 / (1 + ct.hi), 2 / (1 + ct.lo)};
     const Range ry = (double)m.bs * range_pow(flare, m.ay_bs), rz = (double)m.bs * range_pow(flare, m.az_bs);
     known = known && m.bs > 0;
+    within({m.ay_bs, m.az_bs}, 0.0, 64.0);
+    for (Range a : {ry, rz}) within(a, 0x1p-60, 0x1p60);  // their products and squares
     Range bs = ry;  // with one exponent: ry / sqrt(cos^2 + sin^2)
     if (m.az_bs != m.ay_bs) {
         const Range u = rz * cp, w = ry * sp, n = ry * rz;
