@@ -55,8 +55,8 @@ extern "C" {
  * EXACT: FP32 with the reference's operation order (no FMA contraction, correctly rounded
  *        division and square root, std::lerp's branches, the double scale chain); bit-identical
  *        to the reference CPU render for finite cubes.
- * FAST:  FP32 with FMA, FP64 camera basis / ray origin / cube entry and FP32 Kahan (compensated)
- *        accumulation; the only form for BF16/F16 storage. For CMEM models: the model in FP32
+ * FAST:  FP32 with FMA, FP64 camera basis / ray origin / cube entry and FP64 sums (over signed
+ *        cubes and CMEM models FP32 Kahan sums per lane); the only form for BF16/F16 storage. For CMEM models: the model in FP32
  *        with the hardware exp2/log2 and polynomial arc cosines (within the reference FP32
  *        model's own error of the FP64 model). */
 #define BIRP_MATH_EXACT 0
@@ -148,7 +148,8 @@ int birp_volume_upload(birp_device* dev, const birp_volume_desc* desc, const flo
  * passes (Cmem.cpp:18-34, the defaults of Cmem.h:21-39). */
 void birp_cmem_default_params(birp_cmem_params* params);
 int birp_cmem_init(const birp_cmem_params* params, birp_cmem_state* state);
-/* Replaces a CMEM object as a Space (Cmem.h:19-97). */
+/* Replaces a CMEM object as a Space (Cmem.h:19-97). The model holds 512 KiB on the device, filled by
+ * the first render that reads them. */
 int birp_cmem_create(birp_device* dev, const birp_cmem_state* state, birp_volume** out);
 int birp_volume_free(birp_volume* vol);
 /* Device bytes held by the volume (all layouts it keeps). */
@@ -227,7 +228,7 @@ typedef struct birp_tuning {
 int birp_batch_create(birp_volume* vol, const birp_view* views, int count, birp_batch** out);
 int birp_batch_free(birp_batch* b);
 /* Selects kernel tuning for the batch: an explicit choice, or NULL for a loaded tuning table's or, without
- * one for the batch's class, the one that suits its number of rays. */
+ * one for the batch's class, the one that suits its rays and samples. */
 int birp_batch_set_tuning(birp_batch* b, const birp_tuning* tuning);
 /* Launch without waiting (birp_batch_wait waits for completion): the batch's kernels go straight
  * onto the device stream, which measured faster per launch than replaying the captured graph. */
